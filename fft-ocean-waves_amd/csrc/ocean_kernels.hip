@@ -4,7 +4,7 @@
 //   tilde_h0_k         (main.cpp:553-583, tilde_h0_k_cs.glsl)   -> k_tilde_h0_k, k_tilde_h0_k_noise
 //   tilde_h0_t         (main.cpp:587-608, tilde_h0_t_cs.glsl)   -> k_tilde_h0_t            (pass API)
 //   butterfly_fft      (main.cpp:612-683, butterfly_cs.glsl,
-//                       inversion_cs.glsl)                      -> k_c2c_rows + k_c2c_cols_inv (pass API)
+//                       inversion_cs.glsl)                      -> k_ifft2_rows + k_ifft2_cols_inv (pass API)
 //   generate_normal_map(main.cpp:687-707, normal_map_cs.glsl)   -> k_normals
 //   update() frame     (main.cpp:240-244)                       -> k_cols + k_rows + k_normals
 //
@@ -607,42 +607,102 @@ __global__ __launch_bounds__(256) void k_normals(const float* __restrict__ heigh
 
 // ------------------------------------------------------------------ A5+A6 pass API (general complex input)
 
-// Row transforms of a general complex N x N field (the horizontal butterflies).
-template <int N, int E>
-__global__ __launch_bounds__(N / E) void k_c2c_rows(const float2* __restrict__ src, float2* __restrict__ dst,
-                                                    const float2* __restrict__ tw)
+// The inversion pass keeps Re of the inverse DFT of F, which is the inverse DFT
+// of F's Hermitian part A(y, x) = (F(y, x) + conj F(-y, -x))/2.  So:
+//   rows     A's rows 0..N/2 only (row N-y of the result is the conjugate of row
+//            y's); rows 0 and N/2 have real results and share one transform;
+//   columns  the results are real: two columns share one transform.
+// Half the transforms and half the intermediate (4 instead of 8 bytes a texel)
+// of transforming F itself: 20 instead of 28 bytes a texel cross the kernels.
+// Both calls' time against whole complex transforms (us): N=256 6.2 -> 6.2 (two
+// launches), 512 9.1 -> 6.4, 1024 16.0 -> 10.9, 2048 48.9 -> 22.9, 4096 302 ->
+// 74; at N=2048 84 MB move at 3.7 TB/s, one block of 16 waves per CU and kernel.
+//
+// Rows: a group of T = N/E threads per row y < N/2, which reads rows y and N-y of
+// src.  mid row y: the row's transform; row 0: that of row 0 in the real parts,
+// of row N/2 in the imaginary parts.
+template <int N, int E, int NB>
+__global__ __launch_bounds__(NB) void k_ifft2_rows(const float2* __restrict__ src, float2* __restrict__ mid,
+                                                   const float2* __restrict__ tw)
 {
-    constexpr int T = N / E;
-    __shared__ float2 lds[lds_len(N)];
-    const int j = threadIdx.x;
-    const size_t row = (size_t)blockIdx.x * N;
+    constexpr int T = N / E, GPB = NB / T;
+    using Sync = typename std::conditional<(T <= 64), WaveSync, BlockSync>::type;
+    static_assert(NB % T == 0 && (T <= 64 || GPB == 1), "groups inside a wave, or one per block");
+    __shared__ float2 lds[GPB * lds_len(N)];
+    const int g = threadIdx.x / T, j = threadIdx.x % T;
+    const int y = blockIdx.x * GPB + g;
+    // the Hermitian part of src's row a (mirror row b)
+    auto fold = [&](int a, int b, float2 (&v)[E]) {
+        float2 m[E];
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            const int x = j + r * T;
+            v[r] = src[(size_t)a * N + x];
+            m[r] = src[(size_t)b * N + ((N - x) & (N - 1))];
+        }
+#pragma unroll
+        for (int r = 0; r < E; ++r) v[r] = make_float2(0.5f * (v[r].x + m[r].x), 0.5f * (v[r].y - m[r].y));
+    };
     float2 v[E];
+    fold(y, (N - y) & (N - 1), v);
+    if (y == 0) {
+        float2 w[E];
+        fold(N / 2, N / 2, w);
 #pragma unroll
-    for (int r = 0; r < E; ++r) v[r] = src[row + j + r * T];
-    fft_inverse<N, E>(v, j, lds, tw, BlockSync{});
+        for (int r = 0; r < E; ++r) v[r] = make_float2(v[r].x - w[r].y, v[r].y + w[r].x);
+    }
+    fft_inverse<N, E>(v, j, lds + g * lds_len(N), tw, Sync{});
 #pragma unroll
-    for (int r = 0; r < E; ++r) dst[row + j + r * T] = v[r];
+    for (int r = 0; r < E; ++r) mid[(size_t)y * N + j + r * T] = v[r];
 }
 
-// Column transforms + inversion: out = (-1)^(x+y) Re(.) / N^2.
-template <int N, int E, int C>
-__global__ __launch_bounds__(C*(N / E)) void k_c2c_cols_inv(const float2* __restrict__ src, float* __restrict__ out,
-                                                            const float2* __restrict__ tw)
+// Columns + inversion, out = (-1)^(x+y) (.) / N^2: C column pairs (2p, 2p + 1) per
+// block, a group of T = N/E threads each; Z = R(., 2p) + i R(., 2p+1), whose rows
+// above N/2 follow from mid's by conjugation.  Both ways go through LDS, where
+// C lanes read 16C contiguous bytes of a mid row and write 8C of an output row.
+// V2: out is 8-byte aligned.
+template <int N, int E, int C, bool V2>
+__global__ __launch_bounds__(C*(N / E)) void k_ifft2_cols_inv(const float2* __restrict__ mid, float* __restrict__ out,
+                                                              const float2* __restrict__ tw)
 {
-    constexpr int T = N / E;
-    __shared__ float2 lds[C * lds_len(N)];
-    const int c = threadIdx.x % C;
-    const int j = threadIdx.x / C;
-    const int x = blockIdx.x * C + c;
-    float2 v[E];
-#pragma unroll
-    for (int r = 0; r < E; ++r) v[r] = src[(size_t)(j + r * T) * N + x];
-    fft_inverse<N, E>(v, j, lds + c * lds_len(N), tw, BlockSync{});
+    constexpr int T = N / E, NB = C * T, LEN = strip_len(N);
+    using Sync = typename std::conditional<(T <= 64), WaveSync, BlockSync>::type;
     constexpr float scale = 1.0f / ((float)N * (float)N);
+    __shared__ float2 lds[C * LEN];
+    const int p0 = xcd_logical(blockIdx.x, gridDim.x) * C;
 #pragma unroll
-    for (int r = 0; r < E; ++r) {
-        const int y = j + r * T;
-        out[(size_t)y * N + x] = (((x + y) & 1) ? -scale : scale) * v[r].x;
+    for (int it = 0; it < E / 2; ++it) {
+        const int    k = threadIdx.x + it * NB, c = k % C, y = k / C;
+        const float4 q = reinterpret_cast<const float4*>(mid + (size_t)y * N)[p0 + c];
+        float2*      buf = lds + c * LEN;
+        buf[lds_pad(y)]                       = y == 0 ? make_float2(q.x, q.z) : make_float2(q.x - q.w, q.y + q.z);
+        buf[lds_pad(y == 0 ? N / 2 : N - y)] = y == 0 ? make_float2(q.y, q.w) : make_float2(q.x + q.w, q.z - q.y);
+    }
+    __syncthreads();
+    {
+        const int j = threadIdx.x % T;
+        float2*   buf = lds + (threadIdx.x / T) * LEN;
+        float2    v[E];
+#pragma unroll
+        for (int r = 0; r < E; ++r) v[r] = buf[lds_pad(j + r * T)];
+        fft_inverse<N, E>(v, j, buf, tw, Sync{});
+        Sync{}();
+#pragma unroll
+        for (int r = 0; r < E; ++r) buf[lds_pad(j + r * T)] = v[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < E; ++it) {
+        const int    k = threadIdx.x + it * NB, c = k % C, y = k / C;
+        const float2 q = lds[c * LEN + lds_pad(y)];
+        const float  s = (y & 1) ? -scale : scale;  // of the even column
+        float*       o = out + (size_t)y * N + 2 * (p0 + c);
+        if constexpr (V2) {
+            *reinterpret_cast<float2*>(o) = make_float2(s * q.x, -s * q.y);
+        } else {
+            o[0] = s * q.x;
+            o[1] = -s * q.y;
+        }
     }
 }
 
@@ -878,11 +938,19 @@ static bool variant_ok_n(int cols_v, int rows_v)
 }
 
 template <int N>
-static hipError_t launch_ifft2_n(const float2* src, float2* tmp, float* out, const float2* const* tw, hipStream_t s)
+static hipError_t launch_ifft2_n(const float2* src, float2* mid, float* out, const float2* const* tw, hipStream_t s)
 {
-    constexpr int E = 16, T = N / E, C = (512 / T) < 16 ? (512 / T) : 16;
-    hipLaunchKernelGGL((k_c2c_rows<N, E>), dim3(N), dim3(T), 0, s, src, tmp, tw[radix_slot(E)]);
-    hipLaunchKernelGGL((k_c2c_cols_inv<N, E, C>), dim3(N / C), dim3(C * T), 0, s, tmp, out, tw[radix_slot(E)]);
+    // Radix 8: at radix 16 a thread's 30 loads and longer chain cost the small
+    // sizes (N=256 6.2 -> 6.8 us) and gain nothing at the large ones.  4 column
+    // pairs per block (64-byte runs read, 32 written), 2 at N = 4096, whose four
+    // would be 2048 threads; 2 or 8 at N = 512..2048 are within 4% or slower.
+    constexpr int T = N / 8, NB = T < 64 ? 64 : T, C = N <= 2048 ? 4 : 2;
+    hipLaunchKernelGGL((k_ifft2_rows<N, 8, NB>), dim3(N / 2 / (NB / T)), dim3(NB), 0, s, src, mid, tw[radix_slot(8)]);
+    const dim3 grid(N / 2 / C), block(C * T);
+    if (reinterpret_cast<uintptr_t>(out) & 7)
+        hipLaunchKernelGGL((k_ifft2_cols_inv<N, 8, C, false>), grid, block, 0, s, mid, out, tw[radix_slot(8)]);
+    else
+        hipLaunchKernelGGL((k_ifft2_cols_inv<N, 8, C, true>), grid, block, 0, s, mid, out, tw[radix_slot(8)]);
     return hipGetLastError();
 }
 
