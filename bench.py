@@ -69,19 +69,15 @@ LAUNCH_FRAMES = launch_frames_for(1024)
 # when the schedule in use matches, otherwise null.
 MEASURED_TRAFFIC = {
     ("k_rows_nrm", 9, 4, 16): 13.5 + 32.1,
-    ("k_cols_lds", 9, 4, 16): 1.9 + 12.6,
     ("k_rows_nrm", 9, 3, 8): 15.8 + 32.0,
-    ("k_cols_lds", 9, 3, 8): 2.9 + 12.9,
     ("k_rows_nrm", 9, 5, 32): 12.9 + 32.0,
-    ("k_cols_lds", 9, 5, 32): 1.4 + 12.6,
 }
 
 
 def kernel_names(sched):
     """Kernel names of a (column, row) schedule as ocn_get_schedule reports it."""
     cv, rv = sched["cols_variant"], sched["rows_variant"]
-    cols = ("k_cols" if cv < 7 else "k_cols_lds2" if 10 <= cv < 13 else "k_cols_lds_f2" if cv >= 19
-            else "k_cols_lds2b" if cv >= 17 else "k_cols_ldsb" if cv >= 15 else "k_cols_lds")
+    cols = "k_cols_lds" if cv in (13, 14, 21) else "k_cols"
     rows = "k_rows" if sched["rows_band"] == 0 else "k_rows_nrm_par" if rv >= 6 else "k_rows_nrm"
     return cols, rows
 

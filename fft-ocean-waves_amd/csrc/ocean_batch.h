@@ -10,7 +10,7 @@
 namespace ocn {
 
 // Block shapes shared by every N in a batch.
-constexpr int kBatchColsThreads = 768;   // 3 * C * (N/16) with C = kBatchColsWidth / N
+constexpr int kBatchColsThreads = 512;   // C * (N/8) with C = kBatchColsWidth / N
 constexpr int kBatchColsWidth   = 4096;  // C * N: columns per column block times N (N = 64: C = N/2)
 constexpr int kBatchRowsThreads = 256;   // (256 / T) groups of T = N/8 threads
 constexpr int kBatchMinN        = 64;
@@ -29,7 +29,8 @@ __host__ __device__ constexpr int batch_rows_band(int N) { return N <= 64 ? 2 : 
 
 // Device-side descriptor of one batch member (one ocean cascade, one frame).
 struct BatchMember {
-    const float4* h0;
+    float4*       h0;
+    float4*       uv;      // folded spectrum (uv_entries(N))
     float2*       z1;
     float2*       z2;
     const float2* tw8;
@@ -56,16 +57,16 @@ __host__ __device__ constexpr int batch_cols_per_block(int N)
     return kBatchColsWidth / N < N / 2 ? kBatchColsWidth / N : N / 2;
 }
 // Column strip widths a member of size N may use: the default C = 4096/N (N/2
-// at N = 64), whose 3C transform groups fill the 768-thread block, or half of
+// at N = 64), whose C transform groups fill the 512-thread block, or half of
 // it up to N = 1024 (the transforms then take half the block, every thread
-// still folds and stores).  N = 2048 / 4096 transforms synchronise the whole
+// still stores).  N = 2048 / 4096 transforms synchronise the whole
 // block, so they keep the default.
 inline bool batch_cols_valid(int N, int C)
 {
     const int C0 = batch_cols_per_block(N);
     return C == C0 || (N <= 1024 && C0 >= 2 && C == C0 / 2);
 }
-// strips of cols_lds_strip: the self-mirror columns 0 and N/2 share one slot
+// strips of cols_strip: the self-mirror columns 0 and N/2 share one slot
 inline int batch_cols_items_per_member(int N, int C) { return (N / 2) / C; }
 // groups per row block: one band per block in the wide launch
 inline int batch_rows_groups_per_block(int N)

@@ -4,7 +4,7 @@
 //
 // A batch member is one ocean cascade (its own N, parameters, h0, intermediate
 // and outputs).  A frame is two launches over device tables of work items:
-//   k_batch_cols: item (member, strip)   -> cols_lds_strip<N, C>, 768 threads,
+//   k_batch_cols: item (member, strip)   -> cols_strip<N, 8, C>,   512 threads,
 //                 C = 4096/N columns (N/2 at N = 64) or, per member, half of it
 //   k_batch_rows: item (member, band set) -> rows_nrm_band<N, 8>,        256 threads
 //                 (bands of the member's R rows)
@@ -32,7 +32,7 @@ constexpr int cols_lds_need()
 {
     int m = 0;
     for (int N = kBatchMinN; N <= kBatchMaxN; N *= 2) {
-        const int need = 3 * batch_cols_per_block(N) * strip_len(N);
+        const int need = batch_cols_per_block(N) * strip_len(N);
         m = m > need ? m : need;
     }
     return m;
@@ -46,7 +46,7 @@ constexpr int rows_lds_need()
     }
     return m;
 }
-constexpr int kColsLds = cols_lds_need();  // 3 * C * strip_len(N)
+constexpr int kColsLds = cols_lds_need();  // C * strip_len(N)
 constexpr int kRowsLds = rows_lds_need();  // (256 / T) * lds_len(N), T = N/8 (N = 4096: the wide launch)
 
 template <int N>
@@ -54,14 +54,13 @@ __device__ __forceinline__ void batch_cols_item(const BatchMember& m, int strip,
 {
     // m.cols is C or (N <= 1024) C/2 (batch_cols_valid, checked on the host)
     constexpr int C = batch_cols_per_block(N);
-    using Sync = typename std::conditional<(N / 16 <= 64), WaveSync, BlockSync>::type;
     if constexpr (N <= 1024 && C >= 2) {
         if (m.cols != C) {
-            cols_lds_strip<N, C / 2, Sync, kBatchColsThreads>(m.h0, m.z1, m.z2, m.tw16, m.sc, t_rev, strip, lds);
+            cols_strip<N, 8, C / 2, kBatchColsThreads>(m.uv, m.z1, m.z2, m.tw8, m.sc, t_rev, strip, lds);
             return;
         }
     }
-    cols_lds_strip<N, C, Sync, kBatchColsThreads>(m.h0, m.z1, m.z2, m.tw16, m.sc, t_rev, strip, lds);
+    cols_strip<N, 8, C, kBatchColsThreads>(m.uv, m.z1, m.z2, m.tw8, m.sc, t_rev, strip, lds);
 }
 
 template <int N, bool RENDER>
@@ -109,7 +108,7 @@ __device__ __forceinline__ void batch_rows(const BatchMember* __restrict__ membe
 
 }  // namespace
 
-__global__ __launch_bounds__(kBatchColsThreads) void k_batch_cols(const BatchMember* __restrict__ members,
+__global__ __launch_bounds__(kBatchColsThreads, 4) void k_batch_cols(const BatchMember* __restrict__ members,
                                                                   const int2* __restrict__ items, double t_rev)
 {
     __shared__ float2 lds[kColsLds];

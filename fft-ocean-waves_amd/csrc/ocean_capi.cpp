@@ -141,58 +141,53 @@ int frames_class(int nframes)
 }
 
 // Built-in schedules: the fastest (column variant, row variant) measured on
-// MI355X per N for one frame per launch and for batches of frames; the
-// autotuner may replace them.  Column variants: 0 (16,1) 1 (16,2) 2 (16,4)
-// 3 (16,8) 4 (8,2) 5 (8,4) 6 (8,8) as (radix, columns per block) of k_cols,
-// 7..9 k_cols_lds with 1, 2, 4 columns per block, 10..12 k_cols_lds2 with 2, 4,
-// 8 columns per block, 13..14 k_cols_lds with 1, 2 columns and twice the
-// threads, 15..16 k_cols_ldsb (N >= 2048) with 1, 2 columns.  Row variants:
-// 0 radix 16,
-// 1 radix 8 (each followed by the normal-map kernel), 2..5 the fused
-// row + normals walk with bands of 4, 8, 16, 32 rows, 6..7 the fused
-// parallel bands of 4 and 2 rows, 8 the parallel bands of 2 rows with twice
-// the threads.  Single frames at N = 256..1024 take the parallel bands after
-// the column strips with twice the threads (graph-timed sweep of every pair
-// in one box: N=1024 31.7 -> 27.4 us, N=512 19.9 -> 12.7 us, N=256 11.9 ->
-// 8.8 us against the earlier single-frame defaults).
+// MI355X per N and frames per launch; the autotuner may replace them.  Column
+// variants (kColsVariants): 13, 14 and 21 k_cols_lds with 1, 2 and 4 columns
+// per block, the others k_cols with C columns: 7, 8, 9, 12 with 1, 2, 4, 8
+// (N <= 1024), 15..17 with 2 and 18 with 4 (N >= 2048).  Row variants: 0 radix
+// 16, 1 radix 8 (each followed by the normal-map kernel), 2..5 the fused
+// row + normals walk with bands of 4, 8, 16, 32 rows, 6..7 the fused parallel
+// bands of 4 and 2 rows, 8 the parallel bands of 2 rows with twice the threads.
+//
+// Columns: k_cols_lds runs a column's three transforms side by side and spreads
+// the folds over the block, the shorter chain while a launch has less than
+// about four blocks per CU; beyond that k_cols, which does less work per column
+// in a third of the LDS, is faster.  Both sides of the line (us per frame,
+// whole frames, k_cols_lds / k_cols): N=256, 32 frames 1.02 / 1.05; N=512, 4
+// frames 5.36 / 5.60, 8 frames 5.22 / 4.53; N=1024, 1 frame 25.4 / 25.7, 2
+// frames 18.9 / 19.5, 4 frames 16.4 / 15.1, 16 frames 11.6 / 11.3.
 std::pair<int, int> default_schedule(int N, int nframes)
 {
     const bool batch = nframes > 1;
-    // Multi-frame launches: the row pass's band height follows the frames per
-    // launch (sweep of every pair at 2..32 frames per launch over a 600-frame
-    // sequence).  The walks of one launch fill the GPU best at about four per
-    // CU: a few frames need short (parallel) bands, 16-32 frames the long
-    // walks.  Launches whose intermediates fit the 256 MB Infinity Cache
-    // beside h0 (up to 20 N=1024 frames, 4 N=2048 frames) are the fastest per
-    // frame, since the row pass then reads them from there.
-    // Column strips over pairs of frames (variant 19, k_cols_lds_f2 with 4
-    // columns: one h0 load and dispersion per texel pair for two frames) at
-    // N <= 512 where they measured faster per frame over the sequence: N=512
-    // from 8 frames per launch (8: 4.59 -> 4.41 us, 32: 3.31-3.46 -> 3.25),
-    // N=256 from 16 (32: 1.09 -> 1.07), N=128 at 32 (0.73 -> 0.71), N=64 from 8.
+    // The row pass's band height follows the frames per launch (sweep of every
+    // pair at 2..32 frames per launch over a 600-frame sequence).  The walks of
+    // one launch fill the GPU best at about four per CU: a few frames need
+    // short (parallel) bands, 16-32 frames the long walks.  Launches whose
+    // intermediates fit the 256 MB Infinity Cache beside the spectrum (up to 20
+    // N=1024 frames, 4 N=2048 frames) are the fastest per frame, since the row
+    // pass then reads them from there.
     int cv, rv;
     switch (N) {
-    case 64: cv = !batch ? 14 : nframes >= 8 ? 19 : 9; rv = batch ? 1 : 8; break;
-    case 128: cv = !batch ? 14 : nframes >= 32 ? 19 : 9; rv = batch ? 2 : 8; break;
-    case 256: cv = !batch ? 13 : nframes >= 16 ? 19 : 9; rv = 8; break;
-    case 512: cv = !batch ? 14 : nframes <= 4 ? 9 : 19; rv = batch ? 7 : 8; break;
+    case 64: cv = 14; rv = batch ? 1 : 8; break;
+    case 128: cv = 14; rv = batch ? 2 : 8; break;
+    case 256: cv = nframes >= 5 && nframes <= 16 ? 21 : 14; rv = 8; break;
+    case 512: cv = nframes <= 2 ? 14 : nframes <= 6 ? 21 : 12; rv = batch ? 7 : 8; break;
     case 1024:
-        cv = batch ? 9 : 14;
+        cv = !batch ? 13 : nframes <= 2 ? 14 : 9;
         rv = !batch ? 7 : nframes <= 6 ? 7 : nframes <= 9 ? 3 : nframes <= 16 ? 4 : 5;
         break;
-    // N=2048: LDS-staged block-synchronised columns for single frames and
-    // launches of a few frames (single 96.6 -> 79.4 us, 2 frames 90.4 -> 83.7
-    // us per frame), k_cols radix 16 with 4 columns for 32
+    // N=2048: 2 columns per block up to a few frames (single frames 79.4 -> 65.1
+    // us, 4 frames 57.6 -> 51.6 us per frame against the earlier LDS-staged
+    // strips), 4 columns (whole 64-byte runs) from 5 frames: 8 frames 63.4 ->
+    // 61.1, 32 frames 67.9 -> 56.7
     case 2048:
-        cv = nframes < 32 ? 16 : 2;
+        cv = nframes <= 4 ? 16 : 18;
         rv = !batch ? 2 : nframes <= 2 ? 3 : nframes <= 4 ? 4 : 5;
         break;
-    // 4096: k_cols_ldsb (one 4096-point transform over four waves, block
-    // barriers at the stage exchanges): 8-frame launches 394 -> 353 us per
-    // frame, single frames 448 -> 406 us, against k_cols radix 16; from 4
-    // frames per launch its two-pass form with two columns per strip
-    // (k_cols_lds2b): 8-frame launches 356 -> 330 us per frame
-    default: cv = nframes >= 4 ? 17 : 15; rv = batch ? 5 : 4; break;
+    // N=4096: 2 columns per block, 1024 threads (single frames 405 -> 270 us,
+    // 4 frames 337 -> 301 us per frame against the earlier strips; 1 column
+    // 325 / 348)
+    default: cv = nframes == 2 || nframes == 3 ? 15 : 17; rv = batch ? 5 : 4; break;
     }
     if (!ocn::schedule_valid(N, cv, rv)) {
         cv = 0;
@@ -213,7 +208,7 @@ struct ocn_handle {
     int        rows_variant = 0;
     bool       tuned = false;       // schedule set by ocn_autotune / ocn_set_schedule
     float4*    h0 = nullptr;        // N*N
-    float4*    h0t = nullptr;       // N*N, h0 transposed (N >= 2048: read by the column strips)
+    float4*    uv = nullptr;        // uv_entries(N): the folded spectrum, read by the column pass
     float2*    z1 = nullptr;        // zcap*N*N: intermediate; frame 0 doubles as butterfly scratch
     float2*    z2 = nullptr;        // zcap*N*N/2
     float2*    tw[3] = {nullptr, nullptr, nullptr};  // Stockham twiddles, radix 4 / 8 / 16
@@ -230,8 +225,8 @@ namespace {
 
 void free_all(ocn_handle* h)
 {
-    void* ptrs[] = {h->h0, h->h0t, h->z1, h->z2, h->tw[0], h->tw[1], h->tw[2], h->spec[0], h->spec[1], h->spec[2],
-                    h->noise, h->height, h->dx, h->dz, h->jac, h->normals};
+    // uv and the output textures lie behind h0, the other radices' twiddles behind tw[0]
+    void* ptrs[] = {h->h0, h->z1, h->z2, h->tw[0], h->spec[0], h->spec[1], h->spec[2], h->noise};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
 }
@@ -259,21 +254,25 @@ int dalloc(T** p, size_t count, const char* what)
     return OCN_OK;
 }
 
+// The three radices' tables in one allocation and one copy (tw[0] owns it).
 int upload_twiddles(ocn_handle* h)
 {
-    const int radices[3] = {4, 8, 16};
+    const int          radices[3] = {4, 8, 16};
+    std::vector<float> all;
+    size_t             at[3];
     for (int i = 0; i < 3; ++i) {
-        std::vector<float> t = stockham_twiddles(h->p.N, radices[i]);
-        if (h->tw[i]) (void)hipFree(h->tw[i]);
-        h->tw[i] = nullptr;
-        int rc = dalloc(&h->tw[i], t.size() / 2 + 1, "twiddles");
-        if (rc) return rc;
-        if (!t.empty()) {
-            hipError_t e = hipMemcpy(h->tw[i], t.data(), t.size() * sizeof(float), hipMemcpyHostToDevice);
-            if (e != hipSuccess) return hip_fail(e, "hipMemcpy(twiddles)");
-        }
+        at[i] = all.size() / 2;
+        const std::vector<float> t = stockham_twiddles(h->p.N, radices[i]);
+        all.insert(all.end(), t.begin(), t.end());
+        all.resize((all.size() + 31) & ~size_t(31));  // 128-byte starts
     }
-    return OCN_OK;
+    if (h->tw[0]) (void)hipFree(h->tw[0]);
+    h->tw[0] = h->tw[1] = h->tw[2] = nullptr;
+    int rc = dalloc(&h->tw[0], all.size() / 2, "twiddles");
+    if (rc) return rc;
+    for (int i = 1; i < 3; ++i) h->tw[i] = h->tw[0] + at[i];
+    hipError_t e = hipMemcpy(h->tw[0], all.data(), all.size() * sizeof(float), hipMemcpyHostToDevice);
+    return e == hipSuccess ? OCN_OK : hip_fail(e, "hipMemcpy(twiddles)");
 }
 
 // Sizes the intermediate buffers for launches of up to `frames` frames.  Only
@@ -333,8 +332,7 @@ void frame_args(const ocn_handle* h, float2* z1, float2* z2, const double* t, in
                 size_t out_stride, ocn::FrameArgs* a)
 {
     const size_t nn = (size_t)h->p.N * h->p.N;
-    a->h0 = h->h0;
-    a->h0t = h->h0t;
+    a->uv = h->uv;
     a->z1 = z1;
     a->z2 = z2;
     for (int i = 0; i < 3; ++i) a->tw[i] = h->tw[i];
@@ -712,15 +710,18 @@ int ocn_create(const ocn_params* p, ocn_handle** out)
     h->cols_variant = sch.first;
     h->rows_variant = sch.second;
     const size_t nn = (size_t)p->N * p->N;
-    if ((rc = dalloc(&h->h0, nn, "h0")) || (p->N >= 2048 && (rc = dalloc(&h->h0t, nn, "h0 transposed"))) ||
-        (rc = reserve_z(h, 1)) || (rc = dalloc(&h->height, nn, "height")) ||
-        (rc = dalloc(&h->dx, nn, "dx")) || (rc = dalloc(&h->dz, nn, "dz")) ||
-        (rc = dalloc(&h->jac, nn, "jacobian")) || (rc = dalloc(&h->normals, nn, "normals")) ||
+    if ((rc = dalloc(&h->h0, 3 * nn + ocn::uv_entries(p->N), "h0")) || (rc = reserve_z(h, 1)) ||
         (rc = upload_twiddles(h))) {
         free_all(h);
         delete h;
         return rc;
     }
+    h->uv     = h->h0 + nn;
+    h->normals = h->uv + ocn::uv_entries(p->N);
+    h->height = reinterpret_cast<float*>(h->normals + nn);
+    h->dx     = h->height + nn;
+    h->dz     = h->dx + nn;
+    h->jac    = h->dz + nn;
     // set-up of the static scratch of ocn_update_frames_noalloc on this device
     // (its address is looked up once per device, never in the frame call)
     if ((e = ocn::static_scratch_resolve(h->device)) != hipSuccess) {
@@ -767,7 +768,7 @@ int ocn_tilde_h0_k(ocn_handle* h, void* stream)
     TraceRange trace("ocn_tilde_h0_k");
     int rc = check_handle(h);
     if (rc || (rc = set_device(h))) return rc;
-    hipError_t e = ocn::launch_h0(h->p.N, h->h0, h->h0t, nullptr, spec_const(h->p), (hipStream_t)stream);
+    hipError_t e = ocn::launch_h0(h->p.N, h->h0, h->uv, nullptr, spec_const(h->p), (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "tilde_h0_k launch");
     h->h0_ready = true;
     return OCN_OK;
@@ -784,7 +785,7 @@ int ocn_tilde_h0_k_from_noise(ocn_handle* h, const uint8_t* noise_host, void* st
     if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(noise)");
     e = hipStreamSynchronize((hipStream_t)stream);  // noise_host may be freed by the caller on return
     if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
-    e = ocn::launch_h0(h->p.N, h->h0, h->h0t, h->noise, spec_const(h->p), (hipStream_t)stream);
+    e = ocn::launch_h0(h->p.N, h->h0, h->uv, h->noise, spec_const(h->p), (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "tilde_h0_k launch");
     h->h0_ready = true;
     return OCN_OK;
@@ -939,7 +940,7 @@ int ocn_get_schedule(const ocn_handle* h, int nframes, int* cols_variant, int* r
     int cv, rv;
     pick_schedule(const_cast<ocn_handle*>(h), nframes, &cv, &rv);
     int E, C;
-    ocn::cols_variant_shape(cv, &E, &C);
+    ocn::cols_variant_shape(h->p.N, cv, &E, &C);
     if (cols_variant) *cols_variant = cv;
     if (rows_variant) *rows_variant = rv;
     if (cols_radix) *cols_radix = E;
@@ -1177,12 +1178,13 @@ int ocn_batch_create(const ocn_params* params, int count, ocn_batch** out)
     int        rc = OCN_OK;
     hipError_t e  = hipGetDevice(&b->device);
     if (e != hipSuccess) rc = hip_fail(e, "hipGetDevice");
-    // Per member, 256-byte aligned: h0 16, z1 8, z2 4, height/dx/dz/jacobian 4 each, normals 16 bytes per texel.
+    // Per member, 256-byte aligned: h0 16, its folded form 8, z1 8, z2 4, height/dx/dz/jacobian 4 each, normals 16
+    // bytes per texel.
     auto   al    = [](size_t x) { return (x + 255) & ~size_t(255); };
     size_t total = 0;
     for (const ocn_params& p : b->params) {
         const size_t nn = (size_t)p.N * p.N;
-        total += al(nn * 16) + al(nn * 8) + al(nn * 4) + 4 * al(nn * 4) + al(nn * 16);
+        total += al(nn * 16) + al(ocn::uv_entries(p.N) * 16) + al(nn * 8) + al(nn * 4) + 4 * al(nn * 4) + al(nn * 16);
     }
     if (!rc) rc = dalloc(&b->pool, total, "batch pool");
     for (const ocn_params& p : b->params) {
@@ -1198,7 +1200,8 @@ int ocn_batch_create(const ocn_params* params, int count, ocn_batch** out)
             const ocn_params& p  = b->params[i];
             const size_t      nn = (size_t)p.N * p.N;
             ocn::BatchMember  m{};
-            m.h0      = reinterpret_cast<const float4*>(q), q += al(nn * 16);
+            m.h0      = reinterpret_cast<float4*>(q), q += al(nn * 16);
+            m.uv      = reinterpret_cast<float4*>(q), q += al(ocn::uv_entries(p.N) * 16);
             m.z1      = reinterpret_cast<float2*>(q), q += al(nn * 8);
             m.z2      = reinterpret_cast<float2*>(q), q += al(nn * 4);
             m.height  = reinterpret_cast<float*>(q), q += al(nn * 4);
@@ -1265,7 +1268,7 @@ int ocn_batch_tilde_h0_k(ocn_batch* b, void* stream)
     hipError_t e = hipSetDevice(b->device);
     if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
     for (size_t i = 0; i < b->members.size(); ++i) {
-        e = ocn::launch_h0(b->params[i].N, const_cast<float4*>(b->members[i].h0), nullptr, nullptr, b->members[i].sc,
+        e = ocn::launch_h0(b->params[i].N, b->members[i].h0, b->members[i].uv, nullptr, b->members[i].sc,
                            (hipStream_t)stream);
         if (e != hipSuccess) return hip_fail(e, "batch tilde_h0_k launch");
     }
@@ -1538,7 +1541,7 @@ int ocn_batch_get_h0(const ocn_batch* b, int member, void** h0)
     if (!h0) return fail(OCN_EINVAL, "h0 is NULL");
     if (member < 0 || member >= (int)b->members.size())
         return fail(OCN_EINVAL, "member %d out of range [0, %zu)", member, b->members.size());
-    *h0 = const_cast<float4*>(b->members[member].h0);
+    *h0 = b->members[member].h0;
     return OCN_OK;
 }
 

@@ -30,15 +30,15 @@ __device__ __forceinline__ void st_out(float4* p, float4 v)
 
 // ------------------------------------------------------------------ noise
 
-// Philox4x32-10 (Salmon et al., SC'11).
+// Philox4x32-10 (Salmon et al., SC'11).  Whole 64-bit products: one
+// quarter-rate multiply each instead of two for the halves.
 __device__ __forceinline__ uint4 philox4x32_10(uint4 c, uint2 k)
 {
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
         if (r) { k.x += 0x9E3779B9u; k.y += 0xBB67AE85u; }
-        const uint32_t hi0 = __umulhi(0xD2511F53u, c.x), lo0 = 0xD2511F53u * c.x;
-        const uint32_t hi1 = __umulhi(0xCD9E8D57u, c.z), lo1 = 0xCD9E8D57u * c.z;
-        c = make_uint4(hi1 ^ c.y ^ k.x, lo1, hi0 ^ c.w ^ k.y, lo0);
+        const uint64_t p0 = (uint64_t)0xD2511F53u * c.x, p1 = (uint64_t)0xCD9E8D57u * c.z;
+        c = make_uint4((uint32_t)(p1 >> 32) ^ c.y ^ k.x, (uint32_t)p1, (uint32_t)(p0 >> 32) ^ c.w ^ k.y, (uint32_t)p0);
     }
     return c;
 }
@@ -153,55 +153,51 @@ __device__ __forceinline__ float2 evolve_amp(const SpecConst& sc, float4 h, floa
     return make_float2(fmaf(h.x, c, -h.y * s) + fmaf(h.z, c, bi * s), fmaf(h.x, s, h.y * c) + fmaf(bi, c, -h.z * s));
 }
 
-// -i m * H  (tilde_h0_t_cs.glsl:113-126)
-__device__ __forceinline__ float2 choppy(float m, float2 h) { return make_float2(m * h.y, -m * h.x); }
-
-// Hermitian parts (F(t) + conj F(t'))/2 of the three spectra at texel t and its
-// mirror t' = -t mod N.  Both share |k| (n' = -n except on the Nyquist row or
-// column, where n' = n = -N/2), hence one phase and one sincos for the pair.
-// p = h0 at t, q = h0 at t'; (nx, ny) and (qx, qy) are their centred indices.
-// pair_fold_at takes the phase fr (turns) and the choppy factor kinv of the
-// pair, so that frames of one texel pair share the dispersion evaluation.
-// pair_fold_sc takes its sin and cos, for pairs that also share the phase.
-__device__ __forceinline__ void pair_fold_sc(const SpecConst& sc, float4 p, float4 q, int nx, int ny, int qx, int qy,
-                                             float kinv, float s, float c, float2& ay, float2& ax, float2& az)
+// -i m * H  (tilde_h0_t_cs.glsl:113-126).  Its products stay out of the sums
+// they go into (no fused multiply-add), so that every kernel instance that
+// folds a texel gives the transform the same input, bit for bit.
+__device__ __forceinline__ float2 choppy(float m, float2 h)
 {
-    const float2 H = evolve_amp(sc, p, s, c);
-    const float2 G = evolve_amp(sc, q, s, c);
-    const float mx = (float)nx * kinv, mz = (float)ny * kinv;
-    const float gx = (float)qx * kinv, gz = (float)qy * kinv;
-    ay = make_float2(0.5f * (H.x + G.x), 0.5f * (H.y - G.y));
-    ax = make_float2(0.5f * (mx * H.y + gx * G.y), 0.5f * (gx * G.x - mx * H.x));
-    az = make_float2(0.5f * (mz * H.y + gz * G.y), 0.5f * (gz * G.x - mz * H.x));
+#pragma clang fp contract(off)
+    return make_float2(m * h.y, -m * h.x);
 }
 
-__device__ __forceinline__ void pair_fold_at(const SpecConst& sc, float4 p, float4 q, int nx, int ny, int qx, int qy,
-                                             float kinv, float fr, float2& ay, float2& ax, float2& az)
+// ------------------------------------------------------------------ folded spectrum
+
+// The column pass needs, per texel u of the half plane tx <= N/2, only the
+// Hermitian parts A = (H(u) + conj H(-u))/2 of the height spectrum and, on the
+// edges, B = (H(u) - conj H(-u))/2.  With a, b = h0k, h0mk at u and a', b' at
+// the mirror -u, H(u) = a e + C(b) conj(e) (e = e^{i w t}, |k| and so w shared by
+// u and -u), hence A = P e + Q conj(e) = U cos + V sin with
+//   P = (a + conj C(b'))/2, Q = (C(b) + conj a')/2, U = P + Q, V = i (P - Q):
+// four real coefficients per half-plane texel, made with h0 (k_tilde_h0_k),
+// that are half of what h0 itself holds for the pair, and one multiply-add per
+// component and frame.  The choppy spectra follow: -i k/|k| changes sign with
+// k, so their Hermitian parts are -i (n kinv) A, except where the centred index
+// n of the mirror is not -n: column tx = 0 for Dx and row ty = 0 for Dz (index
+// -N/2), where they are -i (n kinv) B, with B = U' cos + V' sin from
+// P' = (a - conj C(b'))/2 and Q' = (C(b) - conj a')/2.
+//
+// Layout, float4 (U.re, U.im, V.re, V.im): column tx of the half plane at
+// tx*N + ty (a column is one contiguous run: a wave that transforms a column
+// reads 1 KB per load), then the N entries of B in column 0 (by ty), then the
+// N/2 + 1 of B in row 0 (by tx).
+__host__ __device__ constexpr size_t uv_bcol(int N) { return (size_t)N * (N / 2 + 1); }
+__host__ __device__ constexpr size_t uv_brow(int N) { return uv_bcol(N) + N; }
+
+// (U, V) of A (sign = 1) or B (sign = -1) from h0 at u (p) and at -u (q).
+__device__ __forceinline__ float4 fold_coeffs(float4 p, float4 q, int conj_mode, float sign)
 {
-    float s, c;
-    sincos_turns(fr, s, c);
-    const float2 H = evolve_amp(sc, p, s, c);
-    const float2 G = evolve_amp(sc, q, s, c);
-    const float mx = (float)nx * kinv, mz = (float)ny * kinv;
-    const float gx = (float)qx * kinv, gz = (float)qy * kinv;
-    ay = make_float2(0.5f * (H.x + G.x), 0.5f * (H.y - G.y));
-    ax = make_float2(0.5f * (mx * H.y + gx * G.y), 0.5f * (gx * G.x - mx * H.x));
-    az = make_float2(0.5f * (mz * H.y + gz * G.y), 0.5f * (gz * G.x - mz * H.x));
+    const float bi = conj_mode ? -p.w : p.w, qi = conj_mode ? -q.w : q.w;  // Im C(b), Im C(b')
+    const float Px = 0.5f * (p.x + sign * q.z), Py = 0.5f * (p.y - sign * qi);
+    const float Qx = 0.5f * (p.z + sign * q.x), Qy = 0.5f * (bi - sign * q.y);
+    return make_float4(Px + Qx, Py + Qy, Qy - Py, Px - Qx);
 }
 
-__device__ __forceinline__ void pair_fold(const SpecConst& sc, float4 p, float4 q, int nx, int ny, int qx, int qy,
-                                          double t_rev, float2& ay, float2& ax, float2& az)
+// U cos + V sin.
+__device__ __forceinline__ float2 fold_at(float4 uv, float s, float c)
 {
-    float kinv, s, c;
-    sincos_turns(phase_turns(sc, nx * nx + ny * ny, t_rev, kinv), s, c);
-    const float2 H = evolve_amp(sc, p, s, c);
-    const float2 G = evolve_amp(sc, q, s, c);
-    const float mx = (float)nx * kinv, mz = (float)ny * kinv;
-    const float gx = (float)qx * kinv, gz = (float)qy * kinv;
-    ay = make_float2(0.5f * (H.x + G.x), 0.5f * (H.y - G.y));
-    // -i m H = (m H.y, -m H.x);  conj(-i g G) = (g G.y, g G.x)
-    ax = make_float2(0.5f * (mx * H.y + gx * G.y), 0.5f * (gx * G.x - mx * H.x));
-    az = make_float2(0.5f * (mz * H.y + gz * G.y), 0.5f * (gz * G.x - mz * H.x));
+    return make_float2(fmaf(uv.x, c, uv.z * s), fmaf(uv.y, c, uv.w * s));
 }
 
 // ------------------------------------------------------------------ intermediate column order
@@ -284,7 +280,7 @@ __host__ __device__ constexpr int strip_group()
 
 // ------------------------------------------------------------------ column pass: one strip
 
-// Strips of cols_lds_strip per frame: the N/2 + 1 half-plane columns
+// Column strips per frame: the N/2 + 1 half-plane columns
 // 0 .. N/2 in strips of C, with the two self-mirror columns 0 and N/2 sharing
 // one transform (below), i.e. N/2 column slots.
 template <int N, int C>
@@ -307,424 +303,272 @@ __host__ __device__ constexpr int strip_len(int N)
     return N == 1024 ? 1091 : N == 512 ? 547 : N == 256 ? 275 : N == 128 ? 152 : N == 64 ? 76 : lds_len(N);
 }
 
-// Phases of cols_lds_strip (below), shared with the two-frame strip.
-// Strip 0, after the folds: column slot 0 += i * (the Nyquist column's fold),
-// its N rows spread over the whole block (strip is the same for every thread
-// of the block).  Begins with a block barrier.
-template <int N, int C, int NB, bool HT, int CL = C>
-__device__ __forceinline__ void strip_nyquist(const float4* __restrict__ h0, const SpecConst& sc, double t_rev,
-                                              float2* lds)
+// Z1 of rows 2m and 2m+1 at column tx, and at its mirror N - tx: G_h + i G_dx
+// with G(-tx) = conj G(tx).  (y, x) = (G_h, G_dx).
+__device__ __forceinline__ float4 zpack(float2 y0, float2 x0, float2 y1, float2 x1)
 {
-    auto at = [&](int x, int y) -> float4 { return HT ? h0[(size_t)x * N + y] : h0[(size_t)y * N + x]; };
-    constexpr int LEN = strip_len(N);
-    __syncthreads();
-    for (int ty = threadIdx.x; ty < N; ty += NB) {
-        const int my = (N - ty) & (N - 1);
-        float2 by, bx, bz;
-        pair_fold(sc, at(N / 2, ty), at(N / 2, my), 0, ty - N / 2, 0, my - N / 2, t_rev, by, bx, bz);
-        float2& ay = lds[0 * CL * LEN + lds_pad(ty)];
-        float2& ax = lds[1 * CL * LEN + lds_pad(ty)];
-        float2& az = lds[2 * CL * LEN + lds_pad(ty)];
-        ay = make_float2(ay.x - by.y, ay.y + by.x);
-        ax = make_float2(ax.x - bx.y, ax.y + bx.x);
-        az = make_float2(az.x - bz.y, az.y + bz.x);
-    }
+    return make_float4(y0.x - x0.y, y0.y + x0.x, y1.x - x1.y, y1.y + x1.x);
+}
+__device__ __forceinline__ float4 zpack_mirror(float2 y0, float2 x0, float2 y1, float2 x1)
+{
+    return make_float4(y0.x + x0.y, x0.x - y0.y, y1.x + x1.y, x1.x - y1.y);
 }
 
-// The 3C column transforms in place, one per T-thread group of the first NT
-// threads (Sync: WaveSync when a group lies in one wave, else BlockSync).
-template <int N, int C, class Sync, int NB>
-__device__ __forceinline__ void strip_transform(const float2* __restrict__ tw, float2* lds)
+// Z2 tile m (Z2 rows 2m, 2m+1; Z2 row q pairs G_dz rows 2q and 2q+1) of column
+// tx and its mirror, from the column's G_dz in its LDS buffer.  The mirror's
+// position is N/2 + tx (zpos); in slot 0 the real parts are column 0's and the
+// imaginary parts column N/2's.
+template <int N>
+__device__ __forceinline__ void z2_store(float2* __restrict__ z2, int m, int tx, const float2* buf)
 {
-    constexpr int E = 16, T = N / E, NT = 3 * C * T, LEN = strip_len(N);
-    const bool active = NB == NT || (int)threadIdx.x < NT;  // takes part in the transforms
-    if (active) {
+    const float2 a = buf[lds_pad(4 * m)], b = buf[lds_pad(4 * m + 1)];
+    const float2 d = buf[lds_pad(4 * m + 2)], e = buf[lds_pad(4 * m + 3)];
+    float4*      t2 = ztile<N>(z2, m) + tx;
+    t2[0]     = tx == 0 ? make_float4(a.x, b.x, d.x, e.x) : zpack(a, b, d, e);
+    t2[N / 2] = tx == 0 ? make_float4(a.y, b.y, d.y, e.y) : zpack_mirror(a, b, d, e);
+}
+
+// LDS-staged column transforms of one strip, for single frames: the C
+// half-plane columns tx = strip*C + c, block of NB >= 3*C*T threads (T = N/16,
+// a transform inside one wave); lds holds 3*C*strip_len(N), z1/z2 point at the
+// frame's intermediate.
+// Phase A: all NB threads fold the spectrum into per-(field, column) LDS
+// buffers, consecutive threads down a column, two rows ty and N - ty per
+// task: they share |k| and so one dispersion phase.  Phase B: each of the 3C
+// transforms runs inside one T-thread group and leaves its result in natural
+// order in its buffer.  Phase C: every thread stores Z1 = G_h + i G_dx (at tx
+// and its mirror N - tx) and Z2 = G_dz(2p) + i G_dz(2p+1), in two-row tiles
+// (zidx).
+// The three fields' transforms run side by side and the folds are spread over
+// the whole block: with about one block per CU (a single frame) that is the
+// shorter chain; with many blocks cols_strip does less work per column.
+// The self-mirror columns 0 and N/2 have Hermitian folded spectra,
+// A(-ty) = conj A(ty), so their column transforms are real: column slot 0 of
+// strip 0 transforms A_0 + i A_{N/2} and its result holds column 0 in the real
+// parts and column N/2 in the imaginary parts.  That leaves N/2 column slots, a
+// whole number of strips (at N = 1024 and C = 2, exactly one block per CU for a
+// single frame instead of 257 blocks on 256 CUs).
+template <int N, int C, int NB>
+__device__ __forceinline__ void cols_lds_strip(const float4* __restrict__ uv, float2* __restrict__ z1,
+                                               float2* __restrict__ z2, const float2* __restrict__ tw,
+                                               const SpecConst& sc, double t_rev, int strip, float2* lds)
+{
+    constexpr int E = 16, T = N / E, NT = 3 * C * T, LEN = strip_len(N), H = N / 2 + 1;
+    constexpr int ITERS = (C * H + NB - 1) / NB;  // row-pair tasks per thread
+    static_assert(NB >= NT && T <= 64 && 64 % T == 0, "transforms inside one wave");
+    static_assert((N / 2) % C == 0, "strips of C columns tile the half plane");
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        const int k = threadIdx.x + it * NB;
+        if (k < C * H) {
+            const int    c = k / H, ra = k % H, rb = (N - ra) & (N - 1);
+            const int    tx = strip * C + c, nx = tx - N / 2, ny = ra - N / 2;
+            const float4 qa = uv[(size_t)tx * N + ra], qb = uv[(size_t)tx * N + rb];
+            float        kinv, s, cs;
+            sincos_turns(turns(omega_fp64(sc, nx * nx + ny * ny, kinv), t_rev), s, cs);
+            const float2 A = fold_at(qa, s, cs), B = fold_at(qb, s, cs);
+            // Dx takes B's coefficients in column 0, Dz in row 0 (folded spectrum, above)
+            const float2 Ax = tx == 0 ? fold_at(uv[uv_bcol(N) + ra], s, cs) : A;
+            const float2 Bx = tx == 0 ? fold_at(uv[uv_bcol(N) + rb], s, cs) : B;
+            const float2 Az = ra == 0 ? fold_at(uv[uv_brow(N) + tx], s, cs) : A;
+            const float  mx = (float)nx * kinv, mz = (float)ny * kinv;
+            lds[(0 * C + c) * LEN + lds_pad(ra)] = A;
+            lds[(1 * C + c) * LEN + lds_pad(ra)] = choppy(mx, Ax);
+            lds[(2 * C + c) * LEN + lds_pad(ra)] = choppy(mz, Az);
+            if (rb != ra) {  // rows 0 and N/2 are their own partners
+                lds[(0 * C + c) * LEN + lds_pad(rb)] = B;
+                lds[(1 * C + c) * LEN + lds_pad(rb)] = choppy(mx, Bx);
+                lds[(2 * C + c) * LEN + lds_pad(rb)] = choppy(-mz, B);
+            }
+        }
+    }
+    if (strip == 0) {
+        // column slot 0 += i * (the Nyquist column's folds), its rows spread
+        // over the whole block; its Dx spectrum is 0 (nx = 0)
+        __syncthreads();
+        for (int ty = threadIdx.x; ty < N; ty += NB) {
+            const int ny = ty - N / 2;
+            float     kinv, s, cs;
+            sincos_turns(phase_turns(sc, ny * ny, t_rev, kinv), s, cs);
+            const float2 h = fold_at(uv[(size_t)(N / 2) * N + ty], s, cs);
+            const float2 z = choppy((float)ny * kinv, ty == 0 ? fold_at(uv[uv_brow(N) + N / 2], s, cs) : h);
+            float2&      ah = lds[0 * C * LEN + lds_pad(ty)];
+            float2&      az = lds[2 * C * LEN + lds_pad(ty)];
+            ah = make_float2(ah.x - h.y, ah.y + h.x);
+            az = make_float2(az.x - z.y, az.y + z.x);
+        }
+    }
+    __syncthreads();
+    if (NB == NT || (int)threadIdx.x < NT) {
         const int g = threadIdx.x / T, j = threadIdx.x % T;
-        float2* buf = lds + g * LEN;
-        float2  v[E];
+        float2*   buf = lds + g * LEN;
+        float2    v[E];
 #pragma unroll
         for (int r = 0; r < E; ++r) v[r] = buf[lds_pad(j + r * T)];
-        fft_inverse<N, E>(v, j, buf, tw, Sync{});
-        Sync{}();
+        fft_inverse<N, E>(v, j, buf, tw, WaveSync{});
+        WaveSync{}();
 #pragma unroll
         for (int r = 0; r < E; ++r) buf[lds_pad(j + r * T)] = v[r];
     }
-}
-
-// Z1 = G_h + i G_dx and Z2 = G_dz(2p) + i G_dz(2p+1) of the strip's columns
-// and their mirrors from the transformed LDS buffers, in two-row tiles:
-// thread k stores Z1 tile m = k / C (rows 2m, 2m+1) and, for m < N/4, Z2
-// tile m (Z2 rows 2m, 2m+1, i.e. G_dz rows 4m..4m+3) of column c = k % C.
-template <int N, int C, int NB, int CL = C>
-__device__ __forceinline__ void strip_store(float2* __restrict__ z1, float2* __restrict__ z2, int strip,
-                                            const float2* lds)
-{
-    constexpr int LEN = strip_len(N);
+    __syncthreads();
+    // thread k stores Z1 tile m = k / C (rows 2m, 2m+1) and, for m < N/4, Z2
+    // tile m (Z2 rows 2m, 2m+1, i.e. G_dz rows 4m..4m+3) of column c = k % C
     constexpr int ITZ = (C * N / 2 + NB - 1) / NB;
 #pragma unroll
     for (int it = 0; it < ITZ; ++it) {
         const int k = threadIdx.x + it * NB;
         if (k < C * N / 2) {
-            const int    c   = k % C, m = k / C;
-            const int    tx  = strip * C + c;
-            const float2 y0  = lds[(0 * CL + c) * LEN + lds_pad(2 * m)];
-            const float2 x0  = lds[(1 * CL + c) * LEN + lds_pad(2 * m)];
-            const float2 y1  = lds[(0 * CL + c) * LEN + lds_pad(2 * m + 1)];
-            const float2 x1  = lds[(1 * CL + c) * LEN + lds_pad(2 * m + 1)];
-            float4*      t1  = ztile<N>(z1, m);
-            const bool   z2t = m < N / 4;  // Z2 row q pairs G_dz rows 2q and 2q+1
-            float2       a{}, b{}, d{}, e{};
-            if (z2t) {
-                a = lds[(2 * CL + c) * LEN + lds_pad(4 * m)];
-                b = lds[(2 * CL + c) * LEN + lds_pad(4 * m + 1)];
-                d = lds[(2 * CL + c) * LEN + lds_pad(4 * m + 2)];
-                e = lds[(2 * CL + c) * LEN + lds_pad(4 * m + 3)];
-            }
-            float4* t2 = ztile<N>(z2, m);
-            if (tx == 0) {
-                // packed self-mirror columns: real parts are column 0's (real)
-                // transforms, imaginary parts column N/2's
-                t1[0]     = make_float4(y0.x, x0.x, y1.x, x1.x);
-                t1[N / 2] = make_float4(y0.y, x0.y, y1.y, x1.y);
-                if (z2t) {
-                    t2[0]     = make_float4(a.x, b.x, d.x, e.x);
-                    t2[N / 2] = make_float4(a.y, b.y, d.y, e.y);
-                }
-            } else {
-                const int mxc = N - tx;
-                t1[tx]        = make_float4(y0.x - x0.y, y0.y + x0.x, y1.x - x1.y, y1.y + x1.x);
-                t1[zpos<N>(mxc)] = make_float4(y0.x + x0.y, x0.x - y0.y, y1.x + x1.y, x1.x - y1.y);
-                if (z2t) {
-                    t2[tx]        = make_float4(a.x - b.y, a.y + b.x, d.x - e.y, d.y + e.x);
-                    t2[zpos<N>(mxc)] = make_float4(a.x + b.y, b.x - a.y, d.x + e.y, e.x - d.y);
-                }
-            }
+            const int    c = k % C, m = k / C, tx = strip * C + c;
+            const float2 y0 = lds[(0 * C + c) * LEN + lds_pad(2 * m)];
+            const float2 x0 = lds[(1 * C + c) * LEN + lds_pad(2 * m)];
+            const float2 y1 = lds[(0 * C + c) * LEN + lds_pad(2 * m + 1)];
+            const float2 x1 = lds[(1 * C + c) * LEN + lds_pad(2 * m + 1)];
+            float4*      t1 = ztile<N>(z1, m) + tx;
+            t1[0]     = tx == 0 ? make_float4(y0.x, x0.x, y1.x, x1.x) : zpack(y0, x0, y1, x1);
+            t1[N / 2] = tx == 0 ? make_float4(y0.y, x0.y, y1.y, x1.y) : zpack_mirror(y0, x0, y1, x1);
+            if (m < N / 4) z2_store<N>(z2, m, tx, lds + (2 * C + c) * LEN);
         }
     }
 }
 
-// LDS-staged column transforms of one strip: the C half-plane columns
-// tx = strip*C + c, block of 3*C*T threads (T = N/16), frame time t_rev;
-// z1/z2 point at the frame's intermediate, lds holds 3*C*strip_len(N).
-// Phase A: every thread evaluates Hermitian parts (consecutive threads take
-// consecutive columns, then rows ty with their partner rows N - ty, whose
-// texel pairs share |k| and one phase) into per-(field, column) LDS buffers.
-// Phase B: each of the 3C transforms runs inside one T-thread group (Sync:
-// WaveSync when a group lies in one wave, else BlockSync) and leaves its
-// result in natural order in the same buffer.  Phase C: every thread stores
-// Z1 = G_h + i G_dx (columns tx and N-tx) and Z2 = G_dz(2p) + i G_dz(2p+1),
-// both in two-row tiles (zidx).
-// The self-mirror columns 0 and N/2 (their own mirrors) have Hermitian folded
-// spectra, A(-ty) = conj A(ty), so their column transforms are real: column
-// slot 0 of strip 0 transforms A_0 + i A_{N/2} and its result holds column 0 in
-// the real parts and column N/2 in the imaginary parts.  That leaves N/2
-// column slots, a whole number of strips (at N = 1024 and C = 2, exactly one
-// block per CU for a single frame instead of 257 blocks on 256 CUs).
-//
-// HT: h0 is given transposed (h0[x * N + y] holds texel (x, y)), so the strip
-// reads its columns as contiguous runs instead of one 16-byte value per row.
-template <int N, int C, class Sync, int NB = 3 * C * (N / 16), bool HT = false>
-__device__ __forceinline__ void cols_lds_strip(const float4* __restrict__ h0, float2* __restrict__ z1,
-                                               float2* __restrict__ z2, const float2* __restrict__ tw,
-                                               const SpecConst& sc, double t_rev, int strip, float2* lds)
+// Column transforms of one strip in registers: the C half-plane columns
+// tx = strip*C + c, one group of T = N/E threads per column (NB >= C*T threads
+// in the block, the rest only store); lds holds C*strip_len(N).
+// A group folds its column straight into registers (thread j rows j + r*T, each
+// load one contiguous run of the column), since the three folded spectra are
+// real multiples of one another (-i n kinv A): it runs the three transforms one
+// after another in its one LDS buffer and keeps the results in registers until
+// they are staged, so the strip needs a third of the LDS of cols_lds_strip
+// (35 KB at N = 1024 and C = 4: four blocks of four waves per CU instead of one
+// of twelve) and one block's loads, arithmetic and stores overlap another's.
+// Dz goes first: its result leaves the registers before the height's and Dx's,
+// which meet in Z1, are made.  Stores go through the buffers so that C lanes
+// write C adjacent columns of a tile (16 bytes each).
+// Column slot 0 packs columns 0 and N/2 as in cols_lds_strip.  Its folds, two
+// columns' for each transform, are spread over the whole block (slot0_fold):
+// left to the slot's own group, strip 0 took several times a strip's time, and
+// launches of few blocks waited for it.
+template <int N, int NB>
+__device__ __forceinline__ void slot0_fold(const float4* __restrict__ uv, const SpecConst& sc, double t_rev,
+                                           int field, float2* buf)
 {
-    auto at = [&](int x, int y) -> float4 { return HT ? h0[(size_t)x * N + y] : h0[(size_t)y * N + x]; };
-    // NB = threads of the block: all of them fold (phase A) and store (phase
-    // C); the 3C transforms take the first NT.  A block wider than NT (a
-    // single frame, whose few blocks leave the SIMDs short of waves, or the
-    // batch's block shared by every N) splits the folds and stores finer.
-    constexpr int E = 16, T = N / E, NT = 3 * C * T, LEN = strip_len(N);
-    constexpr int ITERS = (C * (N / 2 + 1) + NB - 1) / NB;  // row-pair tasks per thread
-    static_assert(NB >= NT, "block too small for the strip");
-    static_assert(NB == NT || !std::is_same<Sync, BlockSync>::value, "block barriers need every thread active");
+#pragma unroll 1
+    for (int ty = threadIdx.x; ty < N; ty += NB) {
+        const int    ny   = ty - N / 2;
+        const bool   edge = field == 2 && ty == 0;
+        const float4 qa = uv[field == 1 ? uv_bcol(N) + ty : edge ? uv_brow(N) : (size_t)ty];
+        const float4 qb = uv[edge ? uv_brow(N) + N / 2 : (size_t)(N / 2) * N + ty];
+        float        k0, kN, s, c;
+        sincos_turns(phase_turns(sc, (N / 2) * (N / 2) + ny * ny, t_rev, k0), s, c);
+        float2 a = fold_at(qa, s, c), b = make_float2(0.0f, 0.0f);  // Dx is 0 in column N/2 (nx = 0)
+        if (field != 1) {
+            sincos_turns(phase_turns(sc, ny * ny, t_rev, kN), s, c);
+            b = fold_at(qb, s, c);
+            if (field == 2) {
+                a = choppy((float)ny * k0, a);
+                b = choppy((float)ny * kN, b);
+            }
+        } else {
+            a = choppy((float)(-N / 2) * k0, a);
+        }
+        buf[lds_pad(ty)] = make_float2(a.x - b.y, a.y + b.x);
+    }
+}
+
+template <int N, int E, int C, int NB>
+__device__ __forceinline__ void cols_strip(const float4* __restrict__ uv, float2* __restrict__ z1,
+                                           float2* __restrict__ z2, const float2* __restrict__ tw,
+                                           const SpecConst& sc, double t_rev, int strip, float2* lds)
+{
+    constexpr int T = N / E, NT = C * T, LEN = strip_len(N);
+    using Sync = typename std::conditional<(T <= 64), WaveSync, BlockSync>::type;
     static_assert((N / 2) % C == 0, "strips of C columns tile the half plane");
+    static_assert(NB >= NT && NB % T == 0, "whole groups");
+    // Threads past the strip's groups only store; where the transforms meet
+    // block barriers (T > 64) they transform a column of their own for nothing
+    // (lds then holds NB/T buffers).
+    const bool active = NB == NT || T > 64 || (int)threadIdx.x < NT;
+    const int  g = threadIdx.x / T, j = threadIdx.x % T;
+    const int  tx = g < C ? strip * C + g : N / 2 - 1;
+    float2*    buf = lds + g * LEN;
+    float2     A[E], v[E];
+    auto put = [&](float2 (&x)[E]) {
 #pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-        const int k = threadIdx.x + it * NB;
-        if (k < C * (N / 2 + 1)) {
-            // rows ra and rb = -ra mod N of column c (ny -> -ny): their texel
-            // pairs share |k| and so one dispersion phase; rows 0 and N/2 are
-            // their own partners and are folded once
-            const int c   = k % C, ra = k / C;
-            const int rb  = (N - ra) & (N - 1);
-            const int tx  = strip * C + c;  // < N/2
-            const int mxc = (N - tx) & (N - 1);
-            const int nx = tx - N / 2, qx = mxc - N / 2;
-            float     kinv, sn, cs;
-            sincos_turns(turns(omega_fp64(sc, nx * nx + (ra - N / 2) * (ra - N / 2), kinv), t_rev), sn, cs);
-            float2 ay, ax, az;
-            pair_fold_sc(sc, at(tx, ra), at(mxc, rb), nx, ra - N / 2, qx, rb - N / 2, kinv, sn, cs, ay, ax, az);
-            lds[(0 * C + c) * LEN + lds_pad(ra)] = ay;
-            lds[(1 * C + c) * LEN + lds_pad(ra)] = ax;
-            lds[(2 * C + c) * LEN + lds_pad(ra)] = az;
-            if (rb != ra) {
-                pair_fold_sc(sc, at(tx, rb), at(mxc, ra), nx, rb - N / 2, qx, ra - N / 2, kinv, sn, cs, ay, ax, az);
-                lds[(0 * C + c) * LEN + lds_pad(rb)] = ay;
-                lds[(1 * C + c) * LEN + lds_pad(rb)] = ax;
-                lds[(2 * C + c) * LEN + lds_pad(rb)] = az;
-            }
-        }
-    }
-    if (strip == 0) strip_nyquist<N, C, NB, HT>(h0, sc, t_rev, lds);
-    __syncthreads();
-    strip_transform<N, C, Sync, NB>(tw, lds);
-    __syncthreads();
-    strip_store<N, C, NB>(z1, z2, strip, lds);
-}
-
-// cols_lds_strip for two frames (times ta, tb) of the same C columns, both
-// in LDS at once as 2C buffers per field (frame a's columns, then frame
-// b's): each texel pair's h0 values are loaded once for both frames, and the
-// dispersion is evaluated once for the two row pairs (ty, N - ty) and both
-// frames.  Block = 6*C*T threads (NB), the 6C transforms one
-// per T-thread group; lds holds 6*C*strip_len(N).
-template <int N, int C, class Sync, int NB = 6 * C * (N / 16)>
-__device__ __forceinline__ void cols_lds_strip_f2(const float4* __restrict__ h0, float2* __restrict__ z1a,
-                                                  float2* __restrict__ z2a, float2* __restrict__ z1b,
-                                                  float2* __restrict__ z2b, const float2* __restrict__ tw,
-                                                  const SpecConst& sc, double ta, double tb, int strip, float2* lds)
-{
-    constexpr int E = 16, T = N / E, NT = 6 * C * T, LEN = strip_len(N), CL = 2 * C;
-    constexpr int ITERS = (C * (N / 2 + 1) + NB - 1) / NB;  // row-pair tasks per thread
-    static_assert(NB >= NT, "block too small for the strip");
-    static_assert(NB == NT || !std::is_same<Sync, BlockSync>::value, "block barriers need every thread active");
-    static_assert((N / 2) % C == 0, "strips of C columns tile the half plane");
-    // frame f's folds of the texel pair at row y, all sharing the sin/cos of
-    // that frame: frame a to buffers 0..C-1 of each field, frame b to C..2C-1
-    auto fold2 = [&](float4 p, float4 q, int nx, int y, int qx, int qy, float kinv, float sa, float ca, float sb,
-                     float cb, int c) {
-        float2 ay, ax, az;
-        pair_fold_sc(sc, p, q, nx, y - N / 2, qx, qy, kinv, sa, ca, ay, ax, az);
-        lds[(0 * CL + c) * LEN + lds_pad(y)] = ay;
-        lds[(1 * CL + c) * LEN + lds_pad(y)] = ax;
-        lds[(2 * CL + c) * LEN + lds_pad(y)] = az;
-        pair_fold_sc(sc, p, q, nx, y - N / 2, qx, qy, kinv, sb, cb, ay, ax, az);
-        lds[(0 * CL + C + c) * LEN + lds_pad(y)] = ay;
-        lds[(1 * CL + C + c) * LEN + lds_pad(y)] = ax;
-        lds[(2 * CL + C + c) * LEN + lds_pad(y)] = az;
+        for (int r = 0; r < E; ++r) buf[lds_pad(j + r * T)] = x[r];
     };
+    auto get = [&](float2 (&x)[E]) {
 #pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-        const int k = threadIdx.x + it * NB;
-        if (k < C * (N / 2 + 1)) {
-            // rows ra and rb = -ra mod N share |k|: one dispersion evaluation
-            // and one sin/cos per frame for the four texels
-            const int c   = k % C, ra = k / C;
-            const int rb  = (N - ra) & (N - 1);
-            const int tx  = strip * C + c;  // < N/2
-            const int mxc = (N - tx) & (N - 1);
-            const int nx = tx - N / 2, qx = mxc - N / 2;
-            float        kinv, sa, ca, sb, cb;
-            const double w = omega_fp64(sc, nx * nx + (ra - N / 2) * (ra - N / 2), kinv);
-            sincos_turns(turns(w, ta), sa, ca);
-            sincos_turns(turns(w, tb), sb, cb);
-            fold2(h0[(size_t)ra * N + tx], h0[(size_t)rb * N + mxc], nx, ra, qx, rb - N / 2, kinv, sa, ca, sb, cb, c);
-            if (rb != ra)
-                fold2(h0[(size_t)rb * N + tx], h0[(size_t)ra * N + mxc], nx, rb, qx, ra - N / 2, kinv, sa, ca, sb, cb,
-                      c);
+        for (int r = 0; r < E; ++r) x[r] = buf[lds_pad(j + r * T)];
+    };
+    // strip is the same for every thread of the block
+    if (strip == 0) {
+        slot0_fold<N, NB>(uv, sc, t_rev, 2, lds);
+        __syncthreads();
+    }
+    if (active) {
+        const float4* col = uv + (size_t)tx * N;
+        const int     nx  = tx - N / 2;
+        float         kinv[E];
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            const int ny = j + r * T - N / 2;
+            float     s, c;
+            sincos_turns(phase_turns(sc, nx * nx + ny * ny, t_rev, kinv[r]), s, c);
+            A[r] = fold_at(col[j + r * T], s, c);
+            v[r] = choppy((float)ny * kinv[r], r == 0 && j == 0 ? fold_at(uv[uv_brow(N) + tx], s, c) : A[r]);
         }
+        if (tx == 0) get(v);
+        fft_inverse<N, E>(v, j, buf, tw, Sync{});
+        Sync{}();
+        put(v);
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            v[r] = A[r];
+            A[r] = choppy((float)nx * kinv[r], A[r]);
+        }
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < C * N / 4; k += NB) z2_store<N>(z2, k / C, strip * C + k % C, lds + (k % C) * LEN);
+    __syncthreads();
+    if (strip == 0) {
+        slot0_fold<N, NB>(uv, sc, t_rev, 0, lds);
+        __syncthreads();
+    }
+    if (active) {
+        if (tx == 0) get(v);
+        fft_inverse<N, E>(v, j, buf, tw, Sync{});
     }
     if (strip == 0) {
-        strip_nyquist<N, C, NB, false, CL>(h0, sc, ta, lds);
-        strip_nyquist<N, C, NB, false, CL>(h0, sc, tb, lds + C * LEN);
+        __syncthreads();
+        slot0_fold<N, NB>(uv, sc, t_rev, 1, lds);
+        __syncthreads();
     }
-    __syncthreads();
-    strip_transform<N, 2 * C, Sync, NB>(tw, lds);
-    __syncthreads();
-    strip_store<N, C, NB, CL>(z1a, z2a, strip, lds);
-    strip_store<N, C, NB, CL>(z1b, z2b, strip, lds + C * LEN);
-}
-
-// The same strip in two passes through half the LDS: block = 2*C*T threads,
-// lds holds 2*C*lds_len(N).  Phase A folds all three spectra; height and Dx go
-// to LDS, each thread keeps its Dz values in registers.  The first pass
-// transforms the 2C height/Dx columns and stores Z1; the second moves Dz into
-// LDS, transforms the C Dz columns (half the block) and stores Z2.  With half the LDS of
-// cols_lds_strip, two blocks fit a CU and one block's transforms overlap the
-// other's loads and stores.
-template <int N, int C>
-__device__ __forceinline__ void cols_lds2_strip(const float4* __restrict__ h0, float2* __restrict__ z1,
-                                                float2* __restrict__ z2, const float2* __restrict__ tw,
-                                                const SpecConst& sc, double t_rev, int strip, float2* lds)
-{
-    constexpr int E = 16, T = N / E, NT = 2 * C * T, LEN = lds_len(N);
-    constexpr int ITERS = C * N / NT;  // = N / (2T) = 8
-    static_assert(T <= 64 && 64 % T == 0 && (C * N) % NT == 0, "each transform group inside one wave");
-    float2 dzr[ITERS];
+    if (active) {
+        if (tx == 0) get(A);
+        fft_inverse<N, E>(A, j, buf, tw, Sync{});
+        // Z1 at tx and its mirror (slot 0: the real and the imaginary parts)
 #pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-        const int k   = threadIdx.x + it * NT;
-        const int c   = k % C, ty = k / C;
-        const int txc = min(strip * C + c, N / 2);
-        const int mxc = (N - txc) & (N - 1);
-        const int my  = (N - ty) & (N - 1);
-        float2 ay, ax;
-        pair_fold(sc, h0[(size_t)ty * N + txc], h0[(size_t)my * N + mxc], txc - N / 2, ty - N / 2, mxc - N / 2,
-                  my - N / 2, t_rev, ay, ax, dzr[it]);
-        lds[c * LEN + lds_pad(ty)]       = ay;
-        lds[(C + c) * LEN + lds_pad(ty)] = ax;
+        for (int r = 0; r < E; ++r) {
+            const float2 y = v[r], x = A[r];
+            v[r] = tx == 0 ? make_float2(y.x, x.x) : make_float2(y.x - x.y, y.y + x.x);
+            A[r] = tx == 0 ? make_float2(y.y, x.y) : make_float2(y.x + x.y, x.x - y.y);
+        }
+        Sync{}();
+        put(v);
     }
-    auto transform = [&](int groups) {
-        if ((int)threadIdx.x < groups * T) {  // whole waves
-            const int g = threadIdx.x / T, j = threadIdx.x % T;
-            float2*   buf = lds + g * LEN;
-            float2    v[E];
-#pragma unroll
-            for (int r = 0; r < E; ++r) v[r] = buf[lds_pad(j + r * T)];
-            fft_inverse<N, E>(v, j, buf, tw, WaveSync{});
-            WaveSync{}();
-#pragma unroll
-            for (int r = 0; r < E; ++r) buf[lds_pad(j + r * T)] = v[r];
+    auto store = [&](int side) {
+        for (int k = threadIdx.x; k < C * N / 2; k += NB) {
+            const int    c = k % C, m = k / C;
+            const float2 a = lds[c * LEN + lds_pad(2 * m)], b = lds[c * LEN + lds_pad(2 * m + 1)];
+            ztile<N>(z1, m)[strip * C + c + side * (N / 2)] = make_float4(a.x, a.y, b.x, b.y);
         }
     };
     __syncthreads();
-    transform(2 * C);
+    store(0);
     __syncthreads();
-    // Z1 tile m = k / C (rows 2m, 2m+1) of column c = k % C
-#pragma unroll
-    for (int it = 0; it < ITERS / 2; ++it) {
-        const int k = threadIdx.x + it * NT;
-        const int c = k % C, m = k / C;
-        const int tx = strip * C + c;
-        if (tx <= N / 2) {
-            const int    mxc = (N - tx) & (N - 1);
-            const float2 y0  = lds[c * LEN + lds_pad(2 * m)];
-            const float2 x0  = lds[(C + c) * LEN + lds_pad(2 * m)];
-            const float2 y1  = lds[c * LEN + lds_pad(2 * m + 1)];
-            const float2 x1  = lds[(C + c) * LEN + lds_pad(2 * m + 1)];
-            float4*      t1  = ztile<N>(z1, m);
-            t1[tx] = make_float4(y0.x - x0.y, y0.y + x0.x, y1.x - x1.y, y1.y + x1.x);
-            if (mxc != tx) t1[zpos<N>(mxc)] = make_float4(y0.x + x0.y, x0.x - y0.y, y1.x + x1.y, x1.x - y1.y);
-        }
-    }
+    if (active) put(A);
     __syncthreads();
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-        const int k = threadIdx.x + it * NT;
-        lds[(k % C) * LEN + lds_pad(k / C)] = dzr[it];
-    }
-    __syncthreads();
-    transform(C);
-    __syncthreads();
-    // Z2 tile m = k / C, m < N/4: Z2 rows 2m, 2m+1, Z2 row q pairing G_dz rows 2q and 2q+1
-#pragma unroll
-    for (int it = 0; it < ITERS / 4; ++it) {
-        const int k = threadIdx.x + it * NT;
-        const int c = k % C, m = k / C;
-        const int tx = strip * C + c;
-        if (tx <= N / 2) {
-            const int    mxc = (N - tx) & (N - 1);
-            const float2 a   = lds[c * LEN + lds_pad(4 * m)];
-            const float2 b   = lds[c * LEN + lds_pad(4 * m + 1)];
-            const float2 d   = lds[c * LEN + lds_pad(4 * m + 2)];
-            const float2 e   = lds[c * LEN + lds_pad(4 * m + 3)];
-            float4*      t2  = ztile<N>(z2, m);
-            t2[tx] = make_float4(a.x - b.y, a.y + b.x, d.x - e.y, d.y + e.x);
-            if (mxc != tx) t2[zpos<N>(mxc)] = make_float4(a.x + b.y, b.x - a.y, d.x + e.y, e.x - d.y);
-        }
-    }
-}
-
-// cols_lds2_strip for N >= 2048 (transform groups of several waves, block
-// barriers): block = 2*C*T threads, lds holds 2*C*lds_len(N), h0t is h0
-// transposed (the strip's columns contiguous).  Phase A folds all three
-// spectra; height and Dx go to LDS and each thread keeps its Dz values in
-// registers.  The first pass transforms the 2C height/Dx columns at radix 16
-// and stores Z1; the second moves Dz into LDS and transforms its C columns at
-// radix 8 (N/8 threads each), so every thread of the block takes part in both
-// passes and meets every barrier.  With half the LDS per column of
-// cols_lds_strip, a strip holds twice the columns: at N = 4096 two columns, so
-// each two-row tile row gets 32 contiguous bytes from one block instead of 16.
-template <int N, int C>
-__device__ __forceinline__ void cols_lds2b_strip(const float4* __restrict__ h0t, float2* __restrict__ z1,
-                                                 float2* __restrict__ z2, const float2* __restrict__ tw16,
-                                                 const float2* __restrict__ tw8, const SpecConst& sc, double t_rev,
-                                                 int strip, float2* lds)
-{
-    constexpr int T = N / 16, NT = 2 * C * T, LEN = lds_len(N);
-    constexpr int ITERS = C * N / NT;  // = 8
-    static_assert(T % 64 == 0 && NT <= 1024 && C * (N / 8) == NT, "whole waves; both passes use every thread");
-    float2 dzr[ITERS];
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-        const int k   = threadIdx.x + it * NT;
-        const int c   = k % C, ty = k / C;
-        const int txc = min(strip * C + c, N / 2);
-        const int mxc = (N - txc) & (N - 1);
-        const int my  = (N - ty) & (N - 1);
-        float2 ay, ax;
-        pair_fold(sc, h0t[(size_t)txc * N + ty], h0t[(size_t)mxc * N + my], txc - N / 2, ty - N / 2, mxc - N / 2,
-                  my - N / 2, t_rev, ay, ax, dzr[it]);
-        lds[c * LEN + lds_pad(ty)]       = ay;
-        lds[(C + c) * LEN + lds_pad(ty)] = ax;
-    }
-    __syncthreads();
-    {
-        const int g = threadIdx.x / T, j = threadIdx.x % T;
-        float2*   buf = lds + g * LEN;
-        float2    v[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = buf[lds_pad(j + r * T)];
-        fft_inverse<N, 16>(v, j, buf, tw16, BlockSync{});
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < 16; ++r) buf[lds_pad(j + r * T)] = v[r];
-    }
-    __syncthreads();
-    // Z1 tile m = k / C (rows 2m, 2m+1) of column c = k % C
-#pragma unroll
-    for (int it = 0; it < ITERS / 2; ++it) {
-        const int k = threadIdx.x + it * NT;
-        const int c = k % C, m = k / C;
-        const int tx = strip * C + c;
-        if (tx <= N / 2) {
-            const int    mxc = (N - tx) & (N - 1);
-            const float2 y0  = lds[c * LEN + lds_pad(2 * m)];
-            const float2 x0  = lds[(C + c) * LEN + lds_pad(2 * m)];
-            const float2 y1  = lds[c * LEN + lds_pad(2 * m + 1)];
-            const float2 x1  = lds[(C + c) * LEN + lds_pad(2 * m + 1)];
-            float4*      t1  = ztile<N>(z1, m);
-            t1[tx] = make_float4(y0.x - x0.y, y0.y + x0.x, y1.x - x1.y, y1.y + x1.x);
-            if (mxc != tx) t1[zpos<N>(mxc)] = make_float4(y0.x + x0.y, x0.x - y0.y, y1.x + x1.y, x1.x - y1.y);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-        const int k = threadIdx.x + it * NT;
-        lds[(k % C) * LEN + lds_pad(k / C)] = dzr[it];
-    }
-    __syncthreads();
-    {
-        constexpr int T8 = N / 8;
-        const int     g = threadIdx.x / T8, j = threadIdx.x % T8;
-        float2*       buf = lds + g * LEN;
-        float2        v[8];
-#pragma unroll
-        for (int r = 0; r < 8; ++r) v[r] = buf[lds_pad(j + r * T8)];
-        fft_inverse<N, 8>(v, j, buf, tw8, BlockSync{});
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < 8; ++r) buf[lds_pad(j + r * T8)] = v[r];
-    }
-    __syncthreads();
-    // Z2 tile m = k / C, m < N/4: Z2 rows 2m, 2m+1, Z2 row q pairing G_dz rows 2q and 2q+1
-#pragma unroll
-    for (int it = 0; it < ITERS / 4; ++it) {
-        const int k = threadIdx.x + it * NT;
-        const int c = k % C, m = k / C;
-        const int tx = strip * C + c;
-        if (tx <= N / 2) {
-            const int    mxc = (N - tx) & (N - 1);
-            const float2 a   = lds[c * LEN + lds_pad(4 * m)];
-            const float2 b   = lds[c * LEN + lds_pad(4 * m + 1)];
-            const float2 d   = lds[c * LEN + lds_pad(4 * m + 2)];
-            const float2 e   = lds[c * LEN + lds_pad(4 * m + 3)];
-            float4*      t2  = ztile<N>(z2, m);
-            t2[tx] = make_float4(a.x - b.y, a.y + b.x, d.x - e.y, d.y + e.x);
-            if (mxc != tx) t2[zpos<N>(mxc)] = make_float4(a.x + b.y, b.x - a.y, d.x + e.y, e.x - d.y);
-        }
-    }
+    store(1);
 }
 
 // ------------------------------------------------------------------ row pass + normals + Jacobian: one band

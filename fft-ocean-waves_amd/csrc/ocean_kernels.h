@@ -9,7 +9,7 @@
 namespace ocn {
 
 constexpr int kMaxFrames        = 32;  // frames per launch of the fused path
-constexpr int kNumColsVariants  = 21;  // column-pass (kernel, radix, columns/block) schedules
+constexpr int kNumColsVariants  = 22;  // column-pass (kernel, columns/block) schedules
 constexpr int kNumRowsVariants  = 9;   // row-pass schedules (radix, fused band, parallel bands)
 
 // Per-ocean spectrum constants, FP32 for the kernels plus the FP64 pieces of
@@ -40,8 +40,7 @@ struct FrameBatch {
 };
 
 struct FrameArgs {
-    const float4* h0;
-    const float4* h0t;        // h0 transposed ([x][y]) for the N >= 2048 column strips, else null
+    const float4* uv;         // folded spectrum (uv_entries(N) values)
     float2*       z1;         // nframes x N x N
     float2*       z2;         // nframes x N/2 x N
     const float2* tw[3];      // Stockham twiddles for radix 4, 8, 16
@@ -74,8 +73,12 @@ hipError_t static_scratch_resolve(int device);
 // The address static_scratch_resolve kept for `device`, or null.
 void*      static_scratch_ptr(int device);
 
-// h0 of the spectrum, and when h0t is given its transpose h0t[x * N + y] = h0[y * N + x]
-hipError_t launch_h0(int N, float4* h0, float4* h0t, const uint8_t* noise, const SpecConst& sc, hipStream_t s);
+// float4 entries of the folded spectrum the column pass reads (ocean_device.hpp),
+// rounded up to 256 bytes
+constexpr size_t uv_entries(int N) { return ((size_t)N * (N / 2 + 1) + N + N / 2 + 1 + 15) & ~size_t(15); }
+
+// h0 of the spectrum (N*N) and its folded form uv (uv_entries(N))
+hipError_t launch_h0(int N, float4* h0, float4* uv, const uint8_t* noise, const SpecConst& sc, hipStream_t s);
 hipError_t launch_spectrum_t(int N, const float4* h0, float2* hy, float2* hx, float2* hz, const SpecConst& sc,
                              double t_rev, hipStream_t s);
 // stages: bit 0 = spectrum + column transforms, bit 1 = row transforms +
@@ -85,7 +88,7 @@ hipError_t launch_ifft2(int N, const float2* src, float2* tmp, float* out, const
 hipError_t launch_normals(int N, const float* height, const float* dx, const float* dz, float4* normals,
                           float* jacobian, int mode, float lambda, float inv2d, hipStream_t s);
 bool       schedule_valid(int N, int cols_variant, int rows_variant);
-void       cols_variant_shape(int v, int* E, int* C);
+void       cols_variant_shape(int N, int v, int* E, int* C);
 int        rows_variant_radix(int v);
 int        rows_variant_band(int v);  // 0: separate normal-map kernel; R: fused bands of R rows
 bool       rows_variant_parallel(int v);  // fused bands whose rows are transformed at once

@@ -6,19 +6,18 @@
 //   butterfly_fft      (main.cpp:612-683, butterfly_cs.glsl,
 //                       inversion_cs.glsl)                      -> k_ifft2_rows + k_ifft2_cols_inv (pass API)
 //   generate_normal_map(main.cpp:687-707, normal_map_cs.glsl)   -> k_normals
-//   update() frame     (main.cpp:240-244)                       -> k_cols + k_rows + k_normals
+//   update() frame     (main.cpp:240-244)                       -> k_cols / k_cols_lds + k_rows_nrm /
+//                                                                  k_rows_nrm_par / k_rows + k_normals
 //
 // Fused frame data flow (per texel, FP32):
-//   h0 (float4: h0k, h0mk) --k_cols_fused--> Z1 (N x N float2), Z2 (N/2 x N float2)
-//                          --k_rows--> height, dx, dz (float)
-//                          --k_normals-----> normals (float4), Jacobian (float)
-// k_cols evaluates the spectrum at texel t and at its mirror t' = (-t mod N),
-// folds each field F into its Hermitian part A = (F(t) + conj F(t'))/2 (whose
-// inverse DFT is Re of F's inverse DFT, which is all inversion_cs.glsl keeps),
-// and runs the column (ty) transforms for the half plane tx in [0, N/2].  It
-// stores the packed rows Z1 = G_h + i G_dx (full width via G(-tx) = conj G(tx))
-// and Z2 = G_dz(2p) + i G_dz(2p + 1).  k_rows runs the row (tx)
-// transforms: Re/Im of each result are two real outputs at once.
+//   folded spectrum (float4 per half-plane texel) --columns--> Z1 (N x N float2), Z2 (N/2 x N float2)
+//                          --rows--> height, dx, dz (float), normals (float4), Jacobian (float)
+// The column pass evaluates each field's Hermitian part (whose inverse DFT is Re
+// of the field's inverse DFT, which is all inversion_cs.glsl keeps) from the
+// folded spectrum (ocean_device.hpp) and runs the column (ty) transforms for the
+// half plane tx in [0, N/2].  It stores the packed rows Z1 = G_h + i G_dx (full
+// width via G(-tx) = conj G(tx)) and Z2 = G_dz(2p) + i G_dz(2p + 1).  The row pass
+// runs the row (tx) transforms: Re/Im of each result are two real outputs at once.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -34,48 +33,69 @@ namespace ocn {
 // ------------------------------------------------------------------ A3 tilde_h0_k
 
 // tilde_h0_k_cs.glsl:74-94 with Philox uniforms (counter = (texel, ocean,
-// cascade, 0), key = seed).  Output: float4 (h0k.re, h0k.im, h0mk.re, h0mk.im).
-__global__ __launch_bounds__(256) void k_tilde_h0_k(float4* __restrict__ h0, SpecConst sc)
+// cascade, 0), key = seed), or NOISE: the reference's four 256x256 8-bit noise
+// images sampled NEAREST + CLAMP_TO_EDGE at gid/N (tilde_h0_k_cs.glsl:53-58,
+// main.cpp:1102-1116).  Output: h0, float4 (h0k.re, h0k.im, h0mk.re, h0mk.im),
+// and the folded spectrum uv that the column pass reads (fold_coeffs).
+// One thread per pair (texel of the half plane, its mirror), tiles of 16 x 16
+// pairs, which go through LDS to uv's columns in runs of 256 bytes.  The noise's
+// integer products bound the kernel at N <= 512, so the pairs are cut to fill
+// the grid exactly (512 blocks, two per CU, at N = 512) and share the amplitude,
+// which is even in k off the edges: the columns 0 and N/2, whose mirrors lie in
+// themselves, hold N + 2 pairs, and the N threads of column 0 take them all.
+// Against drawing h0 alone (and, from N = 2048, transposing it): N=512 3.9 -> 4.7
+// us, 1024 11.1 -> 12.6, 2048 57.8 -> 37.5.
+constexpr int kH0Tile = 16;
+template <bool NOISE>
+__global__ __launch_bounds__(kH0Tile* kH0Tile) void k_tilde_h0_k(float4* __restrict__ h0, float4* __restrict__ uv,
+                                                                 const uint8_t* __restrict__ noise, SpecConst sc)
 {
-    const int tx = blockIdx.x * blockDim.x + threadIdx.x;
-    const int ty = blockIdx.y;
-    if (tx >= sc.N) return;
-    const uint32_t idx = (uint32_t)ty * (uint32_t)sc.N + (uint32_t)tx;
-    const uint4 r  = philox4x32_10(make_uint4(idx, sc.ocean_id, sc.cascade_id, 0u), make_uint2(sc.key0, sc.key1));
-    const float4 xi = box_muller(u01(r.x), u01(r.y), u01(r.z), u01(r.w));
-    const float s  = phillips_amp(sc, tx, ty);
-    h0[idx] = make_float4(s * xi.x, s * xi.y, s * xi.z, s * xi.w);
-}
-
-// h0t[x * N + y] = h0[y * N + x] (N a multiple of 32): 32 x 32 tiles through
-// LDS, so both the reads and the writes are whole rows of a tile.  The column
-// strips at N >= 2048 read h0 down their columns from this copy.
-__global__ __launch_bounds__(256) void k_transpose_h0(const float4* __restrict__ h0, float4* __restrict__ h0t, int N)
-{
-    __shared__ float4 tile[32][33];
-    const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
-    const int x = threadIdx.x % 32, y = threadIdx.x / 32;  // 8 tile rows per pass
-    for (int r = y; r < 32; r += 8) tile[r][x] = h0[(size_t)(by + r) * N + bx + x];
+    __shared__ float4 tile[kH0Tile][kH0Tile + 1];  // [tx][ty]
+    const int N = sc.N, lx = threadIdx.x % kH0Tile, ly = threadIdx.x / kH0Tile;
+    const int x0 = blockIdx.x * kH0Tile, y0 = blockIdx.y * kH0Tile;
+    const int tx = x0 + lx, ty = y0 + ly;
+    // Column 0's threads: rows 0 and N/2, their own mirrors, take that row of
+    // both columns; a row below N/2 takes its pair of column 0, one above that
+    // of column N/2.
+    const bool self = tx == 0 && (ty & (N / 2 - 1)) == 0;
+    const int  my   = (N - ty) & (N - 1);
+    const int  px = tx == 0 && ty > N / 2 ? N / 2 : tx, py = ty;
+    const int  qx = self ? N / 2 : (N - px) & (N - 1), qy = self ? ty : my;
+    auto texel = [&](int x, int y, float s) {
+        float4 xi;
+        if constexpr (NOISE) {
+            const int o = min((y * 256) / N, 255) * 256 + min((x * 256) / N, 255);
+            xi = box_muller(noise[o] / 255.0f, noise[65536 + o] / 255.0f, noise[131072 + o] / 255.0f,
+                            noise[196608 + o] / 255.0f);
+        } else {
+            const uint4 r = philox4x32_10(make_uint4((uint32_t)y * (uint32_t)N + (uint32_t)x, sc.ocean_id,
+                                                     sc.cascade_id, 0u), make_uint2(sc.key0, sc.key1));
+            xi = box_muller(u01(r.x), u01(r.y), u01(r.z), u01(r.w));
+        }
+        return make_float4(s * xi.x, s * xi.y, s * xi.z, s * xi.w);
+    };
+    const float  s = phillips_amp(sc, px, py);
+    const float  t = tx != 0 && ty != 0 ? s : phillips_amp(sc, qx, qy);
+    const float4 p = texel(px, py, s), q = texel(qx, qy, t);
+    h0[(size_t)py * N + px] = p;
+    h0[(size_t)qy * N + qx] = q;
+    const int cm = sc.conj_mode;
+    if (tx != 0) {
+        tile[lx][ly] = fold_coeffs(p, q, cm, 1.0f);
+        if (ty == 0) uv[uv_brow(N) + tx] = fold_coeffs(p, q, cm, -1.0f);
+    } else {
+        const float4 pm = self ? p : q, qm = self ? q : p;  // h0 at the mirrors
+        uv[(size_t)px * N + py] = fold_coeffs(p, pm, cm, 1.0f);
+        uv[(size_t)qx * N + qy] = fold_coeffs(q, qm, cm, 1.0f);
+        if (px == 0) uv[uv_bcol(N) + py] = fold_coeffs(p, pm, cm, -1.0f);
+        if (qx == 0) uv[uv_bcol(N) + qy] = fold_coeffs(q, qm, cm, -1.0f);
+        if (ty == 0) {
+            uv[uv_brow(N)]         = fold_coeffs(p, pm, cm, -1.0f);
+            uv[uv_brow(N) + N / 2] = fold_coeffs(q, qm, cm, -1.0f);
+        }
+    }
     __syncthreads();
-    for (int r = y; r < 32; r += 8) h0t[(size_t)(bx + r) * N + by + x] = tile[x][r];
-}
-
-// Same with the reference's four 256x256 8-bit noise images sampled NEAREST +
-// CLAMP_TO_EDGE at gid/N (tilde_h0_k_cs.glsl:53-58, main.cpp:1102-1116).
-__global__ __launch_bounds__(256) void k_tilde_h0_k_noise(float4* __restrict__ h0, const uint8_t* __restrict__ noise,
-                                                          SpecConst sc)
-{
-    const int tx = blockIdx.x * blockDim.x + threadIdx.x;
-    const int ty = blockIdx.y;
-    if (tx >= sc.N) return;
-    int ix = (tx * 256) / sc.N, iy = (ty * 256) / sc.N;
-    ix = ix > 255 ? 255 : ix;
-    iy = iy > 255 ? 255 : iy;
-    const int o = iy * 256 + ix;
-    const float4 xi = box_muller(noise[o] / 255.0f, noise[65536 + o] / 255.0f, noise[131072 + o] / 255.0f,
-                                 noise[196608 + o] / 255.0f);
-    const float s = phillips_amp(sc, tx, ty);
-    h0[(size_t)ty * sc.N + tx] = make_float4(s * xi.x, s * xi.y, s * xi.z, s * xi.w);
+    if (x0 + ly != 0) uv[(size_t)(x0 + ly) * N + y0 + lx] = tile[ly][lx];
 }
 
 // Pass API: the three spectrum textures of tilde_h0_t (dy, dx, dz), float2 each.
@@ -98,196 +118,55 @@ __global__ __launch_bounds__(256) void k_tilde_h0_t(const float4* __restrict__ h
 
 // ------------------------------------------------------------------ fused frame, pass 1
 
-// Column pass.  1-D grid of (strip groups x frames x G) blocks.  Block = C
-// columns x T threads; thread (c, j) transforms column tx = strip*C + c of the
-// half plane (tx <= N/2), rows ty = j + r*T; consecutive threads read
-// consecutive columns, so a wave's loads cover 64/C rows of C adjacent texels.
-// The three transforms (height, Dx, Dz) share the column's LDS buffer.
-// Block order (after the XCD remap): group-major, then frame, then strip, so a
-// group's h0 columns (the same for every frame) and the Z lines its G strips
-// fill together are served by one XCD's L2.
-template <int N, int E, int C>
-__global__ __launch_bounds__(C*(N / E)) void k_cols(const float4* __restrict__ h0, float2* __restrict__ z1,
-                                                    float2* __restrict__ z2, const float2* __restrict__ tw,
-                                                    SpecConst sc, FrameBatch fb)
+// Column pass: 1-D grid of (strip groups x frames x G) blocks, one strip of one
+// frame each.  Block order (after the XCD remap): group-major, then frame, then
+// strip, so a group's columns of the folded spectrum (the same for every frame)
+// and the Z lines its G strips fill together are served by one XCD's L2.
+template <int N, int C>
+__device__ __forceinline__ void cols_block(const FrameBatch& fb, int& f, int& strip)
 {
-    constexpr int T = N / E;
     constexpr int G = strip_group<N, C>();
-    __shared__ float2 lds[C * lds_len(N)];
-    const int L     = xcd_logical(blockIdx.x, gridDim.x);
-    const int rest  = L / G;
-    const int f     = rest % fb.nframes;
-    const int strip = (rest / fb.nframes) * G + L % G;
-    if (strip > (N / 2) / C) return;  // padding of the last group (whole block)
-    const double t_rev = fb.t_rev[f];
-    z1 += (size_t)f * fb.z1_stride;
-    z2 += (size_t)f * fb.z2_stride;
-    const int  c     = threadIdx.x % C;
-    const int  j     = threadIdx.x / C;
-    const int  tx    = strip * C + c;
-    const bool valid = tx <= N / 2;
-    const int  txc   = valid ? tx : N / 2;
-    const int  mxc   = (N - txc) & (N - 1);
-    const int  nx = txc - N / 2, qx = mxc - N / 2;
-
-    float2 ay[E], ax[E], az[E];
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-        const int ty = j + r * T;
-        const int my = (N - ty) & (N - 1);
-        const float4 p = h0[(size_t)ty * N + txc];
-        const float4 q = h0[(size_t)my * N + mxc];
-        pair_fold(sc, p, q, nx, ty - N / 2, qx, my - N / 2, t_rev, ay[r], ax[r], az[r]);
-    }
-
-    float2* buf = lds + c * lds_len(N);
-    fft_inverse<N, E>(ay, j, buf, tw, BlockSync{});
-    fft_inverse<N, E>(ax, j, buf, tw, BlockSync{});
-    fft_inverse<N, E>(az, j, buf, tw, BlockSync{});
-    // G_dz back through LDS in natural order: Z2 pairs adjacent rows 2p, 2p+1,
-    // which sit in different threads.
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < E; ++r) buf[lds_pad(j + r * T)] = az[r];
-    __syncthreads();
-
-    if (!valid) return;
-    const bool mirror = mxc != tx;
-    // two-row tiles (zidx): threads j and j+1 of a column write the two rows
-    // of a tile, so the C columns of a strip fill runs of 2C values
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-        const int y = j + r * T;
-        z1[zidx<N>(y, tx)] = make_float2(ay[r].x - ax[r].y, ay[r].y + ax[r].x);
-        if (mirror) z1[zidx<N>(y, zpos<N>(mxc))] = make_float2(ay[r].x + ax[r].y, ax[r].x - ay[r].y);
-    }
-#pragma unroll
-    for (int r = 0; r < E / 2; ++r) {
-        const int    p  = j + r * T;
-        const float2 lo = buf[lds_pad(2 * p)], hi = buf[lds_pad(2 * p + 1)];  // rows 2p and 2p+1
-        z2[zidx<N>(p, tx)] = make_float2(lo.x - hi.y, lo.y + hi.x);
-        if (mirror) z2[zidx<N>(p, zpos<N>(mxc))] = make_float2(lo.x + hi.y, hi.x - lo.y);
-    }
+    const int L    = xcd_logical(blockIdx.x, gridDim.x);
+    const int rest = L / G;
+    f     = rest % fb.nframes;
+    strip = (rest / fb.nframes) * G + L % G;
 }
 
-// Column pass, LDS-staged variant (requires T = N/16 <= 64): the work and
-// block order of k_cols, with each strip done by cols_lds_strip (every thread
-// folds the spectrum into LDS, each transform runs inside one wave, every
-// thread stores).  Block = 3C*T threads.
-template <int N, int C, int W = 1>
-__global__ __launch_bounds__(W * 3 * C * (N / 16)) void k_cols_lds(const float4* __restrict__ h0,
+// Register strips (cols_strip): C columns x T = N/8 threads, four waves per SIMD.
+// Radix 8: a thread holds its column's three fields in 128 registers; at radix 16
+// they take 190-210 (two waves per SIMD; capped at three, they spill).  Against
+// the strips it replaced, us per frame (column pass alone): N=1024, 16 frames per
+// launch 4.56 -> 3.6 (4 columns); N=2048, 4 frames 26.8 -> 17.6; N=4096, 4 frames
+// 179 -> 151; the 192-cascade batch 627 -> 430 us.  It writes 12 B/texel at 3.5 TB/s
+// (N=1024): bound by the chain of each block's phases, four blocks per CU deep.
+template <int N, int C>
+__global__ __launch_bounds__(C*(N / 8), 4) void k_cols(const float4* __restrict__ uv, float2* __restrict__ z1,
+                                                       float2* __restrict__ z2, const float2* __restrict__ tw,
+                                                       SpecConst sc, FrameBatch fb)
+{
+    __shared__ float2 lds[C * strip_len(N)];
+    int f, strip;
+    cols_block<N, C>(fb, f, strip);
+    if (strip >= lds_strips<N, C>()) return;  // padding of the last group (whole block)
+    cols_strip<N, 8, C, C*(N / 8)>(uv, z1 + (size_t)f * fb.z1_stride, z2 + (size_t)f * fb.z2_stride, tw, sc,
+                                   fb.t_rev[f], strip, lds);
+}
+
+// LDS-staged strips (cols_lds_strip), single frames N=1024 26.4 -> 25.4 us, N=64
+// 32-frame launches 0.69 -> 0.52 us per frame on the folded spectrum: twice the transforms' 3C x T threads, the
+// extra ones folding and storing only.
+template <int N, int C>
+__global__ __launch_bounds__(2 * 3 * C * (N / 16)) void k_cols_lds(const float4* __restrict__ uv,
                                                                    float2* __restrict__ z1, float2* __restrict__ z2,
                                                                    const float2* __restrict__ tw, SpecConst sc,
                                                                    FrameBatch fb)
 {
-    // W = 2: twice the threads, the extra ones folding and storing only
-    constexpr int T = N / 16;
-    constexpr int G = strip_group<N, C>();
-    static_assert(T <= 64 && 64 % T == 0, "each transform group must lie inside one wave");
     __shared__ float2 lds[3 * C * strip_len(N)];
-    const int L     = xcd_logical(blockIdx.x, gridDim.x);
-    const int rest  = L / G;
-    const int f     = rest % fb.nframes;
-    const int strip = (rest / fb.nframes) * G + L % G;
+    int f, strip;
+    cols_block<N, C>(fb, f, strip);
     if (strip >= lds_strips<N, C>()) return;  // padding of the last group (whole block)
-    cols_lds_strip<N, C, WaveSync, W * 3 * C * T>(h0, z1 + (size_t)f * fb.z1_stride, z2 + (size_t)f * fb.z2_stride,
-                                                  tw, sc, fb.t_rev[f], strip, lds);
-}
-
-// k_cols_lds over pairs of frames: block (strip, frames 2i and 2i+1) holds
-// both frames of its C columns in LDS, loading each texel pair's h0 and
-// evaluating its dispersion once for both (cols_lds_strip_f2); an odd last
-// frame takes a block of its own.  Blocks of one strip group and consecutive
-// frame pairs are consecutive on one XCD, as in k_cols_lds.  Block = 6C*T
-// threads.
-template <int N, int C>
-__global__ __launch_bounds__(6 * C * (N / 16)) void k_cols_lds_f2(const float4* __restrict__ h0,
-                                                                  float2* __restrict__ z1, float2* __restrict__ z2,
-                                                                  const float2* __restrict__ tw, SpecConst sc,
-                                                                  FrameBatch fb)
-{
-    constexpr int T = N / 16, NB = 6 * C * T;
-    constexpr int G = strip_group<N, C>();
-    static_assert(T <= 64 && 64 % T == 0, "each transform group must lie inside one wave");
-    __shared__ float2 lds[6 * C * strip_len(N)];
-    const int L     = xcd_logical(blockIdx.x, gridDim.x);
-    const int pairs = (fb.nframes + 1) / 2;
-    const int rest  = L / G;
-    const int f     = 2 * (rest % pairs);
-    const int strip = (rest / pairs) * G + L % G;
-    if (strip >= lds_strips<N, C>()) return;  // padding of the last group (whole block)
-    float2* z1a = z1 + (size_t)f * fb.z1_stride;
-    float2* z2a = z2 + (size_t)f * fb.z2_stride;
-    if (f + 1 < fb.nframes)
-        cols_lds_strip_f2<N, C, WaveSync, NB>(h0, z1a, z2a, z1a + fb.z1_stride, z2a + fb.z2_stride, tw, sc,
-                                              fb.t_rev[f], fb.t_rev[f + 1], strip, lds);
-    else
-        cols_lds_strip<N, C, WaveSync, NB>(h0, z1a, z2a, tw, sc, fb.t_rev[f], strip, lds);
-}
-
-// k_cols_lds for N >= 2048, whose N/16-thread transform groups span several
-// waves: the same strip (cols_lds_strip) with block barriers between the
-// transform stages, reading the transposed h0 (h0t), where a strip's columns
-// are contiguous runs instead of one 16-byte value per 32 or 64 KB row
-// (sequences of frames: N=2048 70 -> 64 us, N=4096 363 -> 350 us per frame).
-// Block = 3C*T threads.
-template <int N, int C>
-__global__ __launch_bounds__(3 * C * (N / 16)) void k_cols_ldsb(const float4* __restrict__ h0t,
-                                                                float2* __restrict__ z1, float2* __restrict__ z2,
-                                                                const float2* __restrict__ tw, SpecConst sc,
-                                                                FrameBatch fb)
-{
-    constexpr int G = strip_group<N, C>();
-    static_assert(N / 16 > 64 && (N / 16) % 64 == 0, "transform groups of whole waves");
-    __shared__ float2 lds[3 * C * strip_len(N)];
-    const int L     = xcd_logical(blockIdx.x, gridDim.x);
-    const int rest  = L / G;
-    const int f     = rest % fb.nframes;
-    const int strip = (rest / fb.nframes) * G + L % G;
-    if (strip >= lds_strips<N, C>()) return;  // padding of the last group (whole block)
-    cols_lds_strip<N, C, BlockSync, 3 * C * (N / 16), true>(h0t, z1 + (size_t)f * fb.z1_stride,
-                                                            z2 + (size_t)f * fb.z2_stride, tw, sc, fb.t_rev[f], strip,
-                                                            lds);
-}
-
-// Two-pass variant of k_cols_ldsb (cols_lds2b_strip, N >= 2048): 2C*T threads,
-// half the LDS per column, the transposed h0.  Strips of C columns plus the
-// column N/2 (the last strip), in the block order of k_cols.
-template <int N, int C>
-__global__ __launch_bounds__(2 * C * (N / 16)) void k_cols_lds2b(const float4* __restrict__ h0t,
-                                                                 float2* __restrict__ z1, float2* __restrict__ z2,
-                                                                 const float2* __restrict__ tw16,
-                                                                 const float2* __restrict__ tw8, SpecConst sc,
-                                                                 FrameBatch fb)
-{
-    constexpr int G = strip_group<N, C>();
-    __shared__ float2 lds[2 * C * lds_len(N)];
-    const int L     = xcd_logical(blockIdx.x, gridDim.x);
-    const int rest  = L / G;
-    const int f     = rest % fb.nframes;
-    const int strip = (rest / fb.nframes) * G + L % G;
-    if (strip > (N / 2) / C) return;  // padding of the last group (whole block)
-    cols_lds2b_strip<N, C>(h0t, z1 + (size_t)f * fb.z1_stride, z2 + (size_t)f * fb.z2_stride, tw16, tw8, sc,
-                           fb.t_rev[f], strip, lds);
-}
-
-// Two-pass variant of k_cols_lds (cols_lds2_strip): 2C*T threads and half the
-// LDS, same block order.
-template <int N, int C>
-__global__ __launch_bounds__(2 * C * (N / 16)) void k_cols_lds2(const float4* __restrict__ h0,
-                                                                float2* __restrict__ z1, float2* __restrict__ z2,
-                                                                const float2* __restrict__ tw, SpecConst sc,
-                                                                FrameBatch fb)
-{
-    constexpr int G = strip_group<N, C>();
-    __shared__ float2 lds[2 * C * lds_len(N)];
-    const int L     = xcd_logical(blockIdx.x, gridDim.x);
-    const int rest  = L / G;
-    const int f     = rest % fb.nframes;
-    const int strip = (rest / fb.nframes) * G + L % G;
-    if (strip > (N / 2) / C) return;  // padding of the last group (whole block)
-    cols_lds2_strip<N, C>(h0, z1 + (size_t)f * fb.z1_stride, z2 + (size_t)f * fb.z2_stride, tw, sc, fb.t_rev[f],
-                          strip, lds);
+    cols_lds_strip<N, C, 2 * 3 * C * (N / 16)>(uv, z1 + (size_t)f * fb.z1_stride, z2 + (size_t)f * fb.z2_stride, tw,
+                                               sc, fb.t_rev[f], strip, lds);
 }
 
 // ------------------------------------------------------------------ fused frame, pass 2
@@ -708,23 +587,25 @@ __global__ __launch_bounds__(C*(N / E)) void k_ifft2_cols_inv(const float2* __re
 
 // ------------------------------------------------------------------ launchers
 
-// Column-pass schedules (radix E, columns per block C); the autotuner picks one
-// per N.  Row pass: radix E, three transforms per block.
-// kind 0: k_cols (register-resident, block-synchronised transforms);
-// kind 1: k_cols_lds (LDS-staged, one wave per transform, radix 16 only);
-// kind 2: k_cols_lds2 (the same in two passes through half the LDS);
-// kind 3: k_cols_lds with twice the threads (folds and stores split finer);
-// kind 4: k_cols_ldsb (LDS-staged, block-synchronised transforms, N >= 2048);
-// kind 5: k_cols_lds2b (the same in two passes through half the LDS, N >= 2048);
-// kind 6: k_cols_lds_f2 (k_cols_lds over pairs of frames).
+// Column-pass schedules: columns per block C of k_cols (radix 8), or lds: of
+// k_cols_lds (radix 16; the three transforms of a column side by side, folds
+// staged in LDS).  The numbers of earlier builds, which had a kernel for most
+// of them, stay valid for the sizes [min_N, max_N] that took them, in calls and
+// in saved autotune files; several now name one kernel.  A strip is at most
+// 1024 threads wide (cols_width).
 struct ColsVariant {
-    int E, C, kind;
+    int  C;
+    bool lds;
+    int  min_N, max_N;
 };
-constexpr ColsVariant kColsVariants[kNumColsVariants] = {{16, 1, 0}, {16, 2, 0}, {16, 4, 0}, {16, 8, 0}, {8, 2, 0},
-                                                         {8, 4, 0},  {8, 8, 0},  {16, 1, 1}, {16, 2, 1}, {16, 4, 1},
-                                                         {16, 2, 2}, {16, 4, 2}, {16, 8, 2}, {16, 1, 3}, {16, 2, 3},
-                                                         {16, 1, 4}, {16, 2, 4}, {16, 2, 5}, {16, 4, 5},
-                                                         {16, 4, 6}, {16, 8, 6}};
+constexpr ColsVariant kColsVariants[kNumColsVariants] = {
+    {1, false, 64, 4096},   {2, false, 64, 4096},   {4, false, 64, 4096},   {8, false, 64, 2048},
+    {2, false, 64, 4096},   {4, false, 64, 2048},   {8, false, 64, 1024},   {1, false, 64, 1024},
+    {2, false, 64, 1024},   {4, false, 64, 1024},   {2, false, 64, 1024},   {4, false, 64, 1024},
+    {8, false, 64, 1024},   {1, true, 64, 1024},    {2, true, 64, 1024},    {2, false, 2048, 4096},
+    {2, false, 2048, 2048}, {2, false, 2048, 4096}, {4, false, 2048, 2048}, {4, false, 64, 512},
+    {8, false, 64, 256},    {4, true, 64, 512}};
+constexpr int cols_width(int N, int C) { return C * (N / 8) <= 1024 ? C : 1024 / (N / 8); }
 // Row-pass schedules: band 0 = k_rows (radix E) followed by k_normals;
 // band R > 0 = k_rows_nrm with bands of R rows (radix E), normals fused;
 // par = k_rows_nrm_par (bands of R rows whose rows are transformed at once).
@@ -737,22 +618,7 @@ constexpr RowsVariant kRowsVariants[kNumRowsVariants] = {{16, 0, false, 1}, {8, 
                                                          {8, 8, false, 1},  {8, 16, false, 1}, {8, 32, false, 1},
                                                          {16, 4, true, 1},  {16, 2, true, 1},  {16, 2, true, 2}};
 
-template <int N, int E, int C, int K>
-constexpr bool cols_fits()
-{
-    if constexpr (K == 0)
-        return N >= 2 * E && C * (N / E) <= 1024 && C * lds_len(N) * 8 <= 160 * 1024 && C <= N / 2;
-    else if constexpr (K == 1 || K == 3 || K == 6)
-        return E == 16 && N / 16 <= 64 && (K == 1 ? 1 : 2) * 3 * C * (N / 16) <= 1024 &&
-               (K == 6 ? 2 : 1) * 3 * C * strip_len(N) * 8 <= 160 * 1024 && C <= N / 2;
-    else if constexpr (K == 4)
-        return E == 16 && N / 16 > 64 && 3 * C * (N / 16) <= 1024 && 3 * C * strip_len(N) * 8 <= 160 * 1024;
-    else if constexpr (K == 5)
-        return E == 16 && N / 16 > 64 && 2 * C * (N / 16) <= 1024 && 2 * C * lds_len(N) * 8 <= 160 * 1024;
-    else
-        return E == 16 && N >= 64 && N / 16 <= 64 && 2 * C * (N / 16) <= 1024 && 2 * C * lds_len(N) * 8 <= 160 * 1024 &&
-               C <= N / 2 && (C * N) % (2 * C * (N / 16)) == 0;
-}
+constexpr bool cols_fits(int N, int v) { return N >= kColsVariants[v].min_N && N <= kColsVariants[v].max_N; }
 template <int N, int E, int B, bool PAR = false, int W = 1>
 constexpr bool rows_fits()
 {
@@ -772,53 +638,18 @@ constexpr int radix_slot(int E) { return E == 16 ? 2 : E == 8 ? 1 : 0; }
 template <int N, int V>
 static hipError_t launch_cols_v(const FrameArgs& a, hipStream_t s)
 {
-    constexpr int E = kColsVariants[V].E, C = kColsVariants[V].C, K = kColsVariants[V].kind;
-    if constexpr (!cols_fits<N, E, C, K>()) {
+    if constexpr (!cols_fits(N, V)) {
         return hipErrorInvalidValue;
-    } else if constexpr (K == 1 || K == 3) {
-        constexpr int W      = K == 3 ? 2 : 1;
-        constexpr int G      = strip_group<N, C>();
-        constexpr int strips = lds_strips<N, C>();
-        constexpr int groups = (strips + G - 1) / G;
-        hipLaunchKernelGGL((k_cols_lds<N, C, W>), dim3(groups * G * a.nframes), dim3(W * 3 * C * (N / 16)), 0, s,
-                           a.h0, a.z1, a.z2, a.tw[radix_slot(16)], a.sc, a.fb);
-        return hipGetLastError();
-    } else if constexpr (K == 6) {
-        constexpr int G      = strip_group<N, C>();
-        constexpr int strips = lds_strips<N, C>();
-        constexpr int groups = (strips + G - 1) / G;
-        hipLaunchKernelGGL((k_cols_lds_f2<N, C>), dim3(groups * G * ((a.nframes + 1) / 2)), dim3(6 * C * (N / 16)), 0,
-                           s, a.h0, a.z1, a.z2, a.tw[radix_slot(16)], a.sc, a.fb);
-        return hipGetLastError();
-    } else if constexpr (K == 4) {
-        constexpr int G      = strip_group<N, C>();
-        constexpr int strips = lds_strips<N, C>();
-        constexpr int groups = (strips + G - 1) / G;
-        if (!a.h0t) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((k_cols_ldsb<N, C>), dim3(groups * G * a.nframes), dim3(3 * C * (N / 16)), 0, s, a.h0t,
-                           a.z1, a.z2, a.tw[radix_slot(16)], a.sc, a.fb);
-        return hipGetLastError();
-    } else if constexpr (K == 5) {
-        constexpr int G      = strip_group<N, C>();
-        constexpr int strips = (N / 2) / C + 1;
-        constexpr int groups = (strips + G - 1) / G;
-        if (!a.h0t) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((k_cols_lds2b<N, C>), dim3(groups * G * a.nframes), dim3(2 * C * (N / 16)), 0, s, a.h0t,
-                           a.z1, a.z2, a.tw[radix_slot(16)], a.tw[radix_slot(8)], a.sc, a.fb);
-        return hipGetLastError();
-    } else if constexpr (K == 2) {
-        constexpr int G      = strip_group<N, C>();
-        constexpr int strips = (N / 2) / C + 1;
-        constexpr int groups = (strips + G - 1) / G;
-        hipLaunchKernelGGL((k_cols_lds2<N, C>), dim3(groups * G * a.nframes), dim3(2 * C * (N / 16)), 0, s, a.h0,
-                           a.z1, a.z2, a.tw[radix_slot(16)], a.sc, a.fb);
-        return hipGetLastError();
     } else {
-        constexpr int G       = strip_group<N, C>();
-        constexpr int strips  = (N / 2) / C + 1;  // half plane tx in [0, N/2]
-        constexpr int groups  = (strips + G - 1) / G;
-        hipLaunchKernelGGL((k_cols<N, E, C>), dim3(groups * G * a.nframes), dim3(C * (N / E)), 0, s, a.h0, a.z1,
-                           a.z2, a.tw[radix_slot(E)], a.sc, a.fb);
+        constexpr int C = cols_width(N, kColsVariants[V].C);
+        constexpr int G = strip_group<N, C>(), groups = (lds_strips<N, C>() + G - 1) / G;
+        const dim3    grid(groups * G * a.nframes);
+        if constexpr (kColsVariants[V].lds)
+            hipLaunchKernelGGL((k_cols_lds<N, C>), grid, dim3(2 * 3 * C * (N / 16)), 0, s, a.uv, a.z1, a.z2,
+                               a.tw[radix_slot(16)], a.sc, a.fb);
+        else
+            hipLaunchKernelGGL((k_cols<N, C>), grid, dim3(C * (N / 8)), 0, s, a.uv, a.z1, a.z2, a.tw[radix_slot(8)],
+                               a.sc, a.fb);
         return hipGetLastError();
     }
 }
@@ -882,6 +713,7 @@ static hipError_t launch_frame_n(const FrameArgs& a, int stages, hipStream_t s)
         case 18: e = launch_cols_v<N, 18>(a, s); break;
         case 19: e = launch_cols_v<N, 19>(a, s); break;
         case 20: e = launch_cols_v<N, 20>(a, s); break;
+        case 21: e = launch_cols_v<N, 21>(a, s); break;
         default: e = hipErrorInvalidValue;
         }
         if (e != hipSuccess) return e;
@@ -922,11 +754,11 @@ template <int N>
 static bool variant_ok_n(int cols_v, int rows_v)
 {
     constexpr bool c[kNumColsVariants] = {
-#define OCN_FITS(v) cols_fits<N, kColsVariants[v].E, kColsVariants[v].C, kColsVariants[v].kind>()
+#define OCN_FITS(v) cols_fits(N, v)
         OCN_FITS(0), OCN_FITS(1), OCN_FITS(2), OCN_FITS(3), OCN_FITS(4),
         OCN_FITS(5), OCN_FITS(6), OCN_FITS(7), OCN_FITS(8), OCN_FITS(9),
         OCN_FITS(10), OCN_FITS(11), OCN_FITS(12), OCN_FITS(13), OCN_FITS(14), OCN_FITS(15), OCN_FITS(16),
-        OCN_FITS(17), OCN_FITS(18), OCN_FITS(19), OCN_FITS(20)};
+        OCN_FITS(17), OCN_FITS(18), OCN_FITS(19), OCN_FITS(20), OCN_FITS(21)};
 #undef OCN_FITS
 #define OCN_RFITS(v) \
     rows_fits<N, kRowsVariants[v].E, kRowsVariants[v].band, kRowsVariants[v].par, kRowsVariants[v].W>()
@@ -981,10 +813,10 @@ bool schedule_valid(int N, int cols_variant, int rows_variant)
 #undef CALL
 }
 
-void cols_variant_shape(int v, int* E, int* C)
+void cols_variant_shape(int N, int v, int* E, int* C)
 {
-    *E = kColsVariants[v].E;
-    *C = kColsVariants[v].C;
+    *E = kColsVariants[v].lds ? 16 : 8;
+    *C = cols_width(N, kColsVariants[v].C);
 }
 
 int rows_variant_radix(int v) { return kRowsVariants[v].E; }
@@ -1036,12 +868,11 @@ void* static_scratch_ptr(int device)
     return g_scratch_addr[device];
 }
 
-hipError_t launch_h0(int N, float4* h0, float4* h0t, const uint8_t* noise, const SpecConst& sc, hipStream_t s)
+hipError_t launch_h0(int N, float4* h0, float4* uv, const uint8_t* noise, const SpecConst& sc, hipStream_t s)
 {
-    dim3 grid((N + 255) / 256, N);
-    if (noise) hipLaunchKernelGGL(k_tilde_h0_k_noise, grid, dim3(256), 0, s, h0, noise, sc);
-    else hipLaunchKernelGGL(k_tilde_h0_k, grid, dim3(256), 0, s, h0, sc);
-    if (h0t) hipLaunchKernelGGL(k_transpose_h0, dim3(N / 32, N / 32), dim3(256), 0, s, h0, h0t, N);
+    const dim3 grid(N / 2 / kH0Tile, N / kH0Tile), block(kH0Tile * kH0Tile);
+    if (noise) hipLaunchKernelGGL(k_tilde_h0_k<true>, grid, block, 0, s, h0, uv, noise, sc);
+    else hipLaunchKernelGGL(k_tilde_h0_k<false>, grid, block, 0, s, h0, uv, noise, sc);
     return hipGetLastError();
 }
 

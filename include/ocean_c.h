@@ -302,9 +302,8 @@ int ocn_get_fields(const ocn_handle* h, ocn_fields* out);
 
 /* Device pointers of the spectrum textures: h0 (float4[N*N]) and the three
  * tilde_h0_t textures (float2[N*N] each; NULL until ocn_tilde_h0_t ran).
- * Any out-pointer may be NULL.  h0 is for reading: at N >= 2048 the frame
- * reads a transposed copy that ocn_tilde_h0_k and ocn_tilde_h0_k_from_noise
- * make along with it. */
+ * Any out-pointer may be NULL.  h0 is for reading: the frame reads a folded
+ * form that ocn_tilde_h0_k and ocn_tilde_h0_k_from_noise make along with it. */
 int ocn_get_spectrum(const ocn_handle* h, void** h0, void** hy, void** hx, void** hz);
 
 /* Copies the handle's output textures to host memory after the work queued on
@@ -357,8 +356,8 @@ int ocn_batch_update_graph(ocn_batch* b, double t, void* stream);
 int ocn_batch_set_schedule(ocn_batch* b, int N, int rows_band);
 int ocn_batch_get_schedule(const ocn_batch* b, int member, int* rows_band);
 /* Columns per block of the column pass for the members of size N: the
- * default 4096/N (N/2 at N = 64), whose three transforms per column fill a
- * 768-thread block, or half of it up to N = 1024 (more, smaller blocks).  The
+ * default 4096/N (N/2 at N = 64), whose transforms fill a 512-thread block
+ * (256 threads at N = 64), or half of it up to N = 1024 (more, smaller blocks).  The
  * outputs do not depend on it.  Waits for the device to be idle. */
 int ocn_batch_set_column_strips(ocn_batch* b, int N, int cols_per_block);
 int ocn_batch_get_column_strips(const ocn_batch* b, int member, int* cols_per_block);
@@ -370,7 +369,7 @@ int ocn_batch_autotune(ocn_batch* b, int reps, void* stream);
 
 /* Device pointers of one member's outputs (valid until ocn_batch_destroy;
  * displacement and render_normals are NULL unless the render export is on)
- * and its h0 spectrum (float4[N*N]). */
+ * and its h0 spectrum (float4[N*N], for reading, as ocn_get_spectrum's). */
 int ocn_batch_get_fields(const ocn_batch* b, int member, ocn_fields* out);
 /* Render export for every member on (1) or off (0): the row pass then also
  * writes each member's displacement and render_normals as ocn_update_into
