@@ -946,7 +946,8 @@ int ocn_get_schedule(const ocn_handle* h, int nframes, int* cols_variant, int* r
     if (cols_radix) *cols_radix = E;
     if (cols_per_block) *cols_per_block = C;
     if (rows_radix) *rows_radix = ocn::rows_variant_radix(rv);
-    if (rows_band) *rows_band = h->p.normal_mode == OCN_NORMALS_NEAREST ? ocn::rows_variant_band(rv) : 0;
+    if (rows_band)
+        *rows_band = ocn::rows_variant_band(h->p.N, rv, h->p.normal_mode != OCN_NORMALS_NEAREST, nframes);
     return OCN_OK;
 }
 
@@ -974,9 +975,8 @@ int ocn_autotune(ocn_handle* h, int nframes, int reps, void* stream)
     for (int cv = 0; cv < ocn::kNumColsVariants && rc == OCN_OK; ++cv)
         for (int rv = 0; rv < ocn::kNumRowsVariants && rc == OCN_OK; ++rv) {
             if (!ocn::schedule_valid(h->p.N, cv, rv)) continue;
-            // bilinear normals always run the separate normal-map kernel, so a
-            // fused row variant would time the same kernels as variant 0
-            if (h->p.normal_mode != OCN_NORMALS_NEAREST && ocn::rows_variant_band(rv) > 0) continue;
+            // bilinear normals take no walk: the parallel bands stand in for them
+            if (h->p.normal_mode != OCN_NORMALS_NEAREST && ocn::rows_variant_walk(rv)) continue;
             const int stages = OCN_STAGE_ALL;
             if ((rc = run_frames(h, t.data(), nframes, &out, nn, stages, cv, rv, s))) break;  // warm-up
             (void)hipEventRecord(e0, s);
@@ -1053,7 +1053,7 @@ int ocn_autotune_load(const char* path)
         const bool ok = dev >= 0 && N >= 64 && N <= 4096 && (N & (N - 1)) == 0 && frames_class(cls) == cls &&
                         (mode == OCN_NORMALS_NEAREST || mode == OCN_NORMALS_BILINEAR) &&
                         ocn::schedule_valid(N, cv, rv) &&
-                        (mode == OCN_NORMALS_NEAREST || ocn::rows_variant_band(rv) == 0);
+                        (mode == OCN_NORMALS_NEAREST || !ocn::rows_variant_walk(rv));
         if (!ok) {
             rc = fail(OCN_EINVAL, "%s:%d: not a valid (device, N, class, normal mode, schedule)", path, lineno);
             break;

@@ -264,34 +264,46 @@ __global__ __launch_bounds__(N / E >= 64 ? N / E : 64, 2) void k_rows_nrm(
 
 // ------------------------------------------------------------------ fused row pass, parallel bands
 
-// Row pass fused with the normal map (nearest taps) and the Jacobian for
-// launches of few frames: where the band walk of k_rows_nrm runs its rows one
-// after another (long bands, few groups), here one block owns a band of R
-// output rows [y0, y0 + R) and transforms all the rows its stencils need at
-// once: G1 = R + 2 Z1 rows (y0 - 1 .. y0 + R) and G2 = R/2 + 2 Z2 rows
-// (y0/2 - 1 .. y0/2 + R/2), one T-thread group (radix E) each.  The results
-// stay in the groups' LDS buffers in natural order; after one block barrier
-// every thread takes texels of the band, applies (-1)^(x+y) / N^2
-// (inversion_cs.glsl:35-41) to each value it reads and computes the Sobel
-// normal (normal_map_cs.glsl:37-53) and the Jacobian of the render
-// displacement (grid_tes.glsl:60-62) with the band walk's arithmetic.  1-D
-// grid of (N/R) x frames blocks; after the XCD remap neighbouring bands,
-// which read the same halo tiles, run on one XCD.
-template <int N, int E, int R>
+// Row pass fused with the normal map and the Jacobian for launches of few
+// frames: where the band walk of k_rows_nrm runs its rows one after another
+// (long bands, few groups), here one block owns a band of R output rows
+// [y0, y0 + R) and transforms all the rows its stencils need at once: Z1 rows
+// y0 - 1 .. y0 + R and Z2 rows y0/2 - 1 .. y0/2 + R/2, one T-thread group
+// (radix E) each.  The results stay in the groups' LDS buffers in natural
+// order; after one block barrier every thread takes texels of the band, applies
+// (-1)^(x+y) / N^2 (inversion_cs.glsl:35-41) to each value it reads and computes
+// the Sobel normal (normal_map_cs.glsl:37-53) and the Jacobian of the render
+// displacement (grid_tes.glsl:60-62) with the band walk's arithmetic.  1-D grid
+// of (N/R) x frames blocks; after the XCD remap neighbouring bands, which read
+// the same halo tiles, run on one XCD.
+//
+// RENDER adds the render export (disp, rnorm, either may be null), as in the walk.
+// BIL takes the height taps bilinearly at texel corners (OCN_NORMALS_BILINEAR):
+// the 2x2 box folded into the Sobel weights is [1 3 3 1] along one axis and
+// [1 1 -1 -1] along the other over x-2..x+1, y-2..y+1, so one more Z1 row is
+// transformed above the band.  Both used to take the unfused row pass and the
+// normal-map kernel, which read height, Dx and Dz back: 12 bytes a texel and a
+// launch more.  Whole frames, unfused -> here (us per frame): render export N=256
+// 17.0 -> 10.2 (single), 2.09 -> 1.66 (16 per launch), N=512 20.9 -> 13.5, N=1024
+// 38.4 -> 32.0; bilinear N=256 17.5 -> 9.2, N=512 21.5 -> 12.6 and 5.2 -> 3.9
+// (8 per launch), N=1024 33.4 -> 25.7 and 18.9 -> 13.0 (16), N=2048 88 -> 66 (4).
+template <int N, int E, int R, bool BIL = false>
 constexpr int par_groups()
 {
-    return (R + 2) + (R / 2 + 2);
+    return (R + 2 + (BIL ? 1 : 0)) + (R / 2 + 2);
 }
 
-template <int N, int E, int R, int W = 1>
-__global__ __launch_bounds__((W * par_groups<N, E, R>() * (N / E))) void k_rows_nrm_par(
+template <int N, int E, int R, int W, bool BIL, bool RENDER>
+__global__ __launch_bounds__((W * par_groups<N, E, R, BIL>() * (N / E))) void k_rows_nrm_par(
     const float2* __restrict__ z1, const float2* __restrict__ z2, float* __restrict__ height,
     float* __restrict__ dx, float* __restrict__ dz, float4* __restrict__ normals, float* __restrict__ jac,
-    const float2* __restrict__ tw, FrameBatch fb, float lambda, float inv2d)
+    const float2* __restrict__ tw, FrameBatch fb, float lambda, float inv2d, float4* __restrict__ disp,
+    float4* __restrict__ rnorm, float dscale)
 {
     // W = 2: twice the threads, the extra ones (after the G transform groups)
     // taking part in the stencils only
-    constexpr int T = N / E, G1 = R + 2, G = par_groups<N, E, R>(), LEN = lds_len(N), NT = W * G * T;
+    constexpr int UP = BIL ? 2 : 1;  // rows above the band
+    constexpr int T = N / E, G1 = R + UP + 1, G = par_groups<N, E, R, BIL>(), LEN = lds_len(N), NT = W * G * T;
     static_assert(R % 2 == 0 && N % R == 0, "bands of an even number of rows");
     static_assert(T % 64 == 0 || 64 % T == 0, "transform groups of whole waves or within one wave");
     static_assert(W == 1 || T <= 64, "extra threads only beside wave-local transforms");
@@ -310,13 +322,15 @@ __global__ __launch_bounds__((W * par_groups<N, E, R>() * (N / E))) void k_rows_
     dz += fo;
     if (normals) normals += fo;
     if (jac) jac += fo;
+    if (RENDER && disp) disp += fo;
+    if (RENDER && rnorm) rnorm += fo;
 
     if (W == 1 || (int)threadIdx.x < G * T) {
         const int g = threadIdx.x / T, j = threadIdx.x % T;
-        // group g < G1: Z1 row y0 - 1 + g; else Z2 row y0/2 - 1 + (g - G1) (periodic)
+        // group g < G1: Z1 row y0 - UP + g; else Z2 row y0/2 - 1 + (g - G1) (periodic)
         const bool    is1 = g < G1;
         const float2* src = is1 ? z1 : z2;
-        const int     row = is1 ? (y0 - 1 + g) & (N - 1) : ((y0 >> 1) - 1 + (g - G1)) & (N / 2 - 1);
+        const int     row = is1 ? (y0 - UP + g) & (N - 1) : ((y0 >> 1) - 1 + (g - G1)) & (N / 2 - 1);
         float2        v[E];
 #pragma unroll
         for (int r = 0; r < E; ++r) v[r] = src[zidx<N>(row, zpos_elem<N, E>(j, r))];
@@ -331,13 +345,14 @@ __global__ __launch_bounds__((W * par_groups<N, E, R>() * (N / E))) void k_rows_
     // Stencils: each thread walks whole columns x of the band, keeping the
     // signed values of x-1, x, x+1 for all band and halo rows in registers
     // (each LDS value is read once per column).  The sign (-1)^(x+y) / N^2 of
-    // texel (x, y): rows y0 - 1 + g alternate starting from that of
-    // (x, y0 - 1) (y0 is even); columns x +- 1 have the opposite sign of x.
+    // texel (x, y): rows y0 - UP + g alternate starting from that of
+    // (x, y0 - UP) (y0 is even); columns x +- 1 have the opposite sign of x.
     constexpr int G2 = G - G1;
     for (int x = threadIdx.x; x < N; x += NT) {
         const int   pl = lds_pad((x - 1) & (N - 1)), pm = lds_pad(x), pr = lds_pad((x + 1) & (N - 1));
-        const float s0 = ((x + 1) & 1) ? -scale : scale;  // (x, y0 - 1)
-        float2 hl[G1], hm[G1], hr[G1];  // (height, Dx) of rows y0 - 1 .. y0 + R at x - 1, x, x + 1
+        const float s0 = ((x + UP) & 1) ? -scale : scale;  // (x, y0 - UP)
+        float2 hl[G1], hm[G1], hr[G1];  // (height, Dx) of rows y0 - UP .. y0 + R at x - 1, x, x + 1
+        float  hll[BIL ? G1 : 1];       // height at x - 2
 #pragma unroll
         for (int g = 0; g < G1; ++g) {
             const float  sm = (g & 1) ? -s0 : s0;
@@ -345,48 +360,77 @@ __global__ __launch_bounds__((W * par_groups<N, E, R>() * (N / E))) void k_rows_
             hl[g] = make_float2(-sm * l.x, -sm * l.y);
             hm[g] = make_float2(sm * m.x, sm * m.y);
             hr[g] = make_float2(-sm * r.x, -sm * r.y);
+            if constexpr (BIL) hll[g] = sm * lds[g * LEN + lds_pad((x - 2) & (N - 1))].x;
         }
-        // Dz of rows y0 - 1 .. y0 + R: Z2 row y/2 (buffer G1 + (y+2)/2 - y0/2), part y & 1
-        float zl[G1], zm[G1], zr[G1];
+        // Dz of rows y0 - 1 .. y0 + R (index 0 .. R + 1): Z2 row y0/2 - 1 + q holds
+        // rows y0 - 2 + 2q (re) and y0 - 1 + 2q (im), i.e. indices 2q - 1, 2q
+        const float z0 = ((x + 1) & 1) ? -scale : scale;  // (x, y0 - 1)
+        float zl[R + 2], zm[R + 2], zr[R + 2];
 #pragma unroll
         for (int q = 0; q < G2; ++q) {
             const float2 l = lds[(G1 + q) * LEN + pl], m = lds[(G1 + q) * LEN + pm], r = lds[(G1 + q) * LEN + pr];
-            // Z2 row y0/2 - 1 + q holds rows y0 - 2 + 2q (re) and y0 - 1 + 2q (im), i.e. g = 2q - 1, 2q
 #pragma unroll
             for (int part = 0; part < 2; ++part) {
-                const int g = 2 * q - 1 + part;
-                if (g < 0 || g >= G1) continue;
-                const float sm = (g & 1) ? -s0 : s0;
-                zl[g] = -sm * (part ? l.y : l.x);
-                zm[g] = sm * (part ? m.y : m.x);
-                zr[g] = -sm * (part ? r.y : r.x);
+                const int i = 2 * q - 1 + part;
+                if (i < 0 || i >= R + 2) continue;
+                const float sm = (i & 1) ? -z0 : z0;
+                zl[i] = -sm * (part ? l.y : l.x);
+                zm[i] = sm * (part ? m.y : m.x);
+                zr[i] = -sm * (part ? r.y : r.x);
             }
         }
 #pragma unroll
         for (int k = 0; k < R; ++k) {
-            const int    g = k + 1;  // grid row y0 + k
+            const int    g = k + UP, i = k + 1;  // grid row y0 + k
             const size_t o = (size_t)(y0 + k) * N + x;
             if (normals) {
-                // v_s = h(y-1) + 2 h(y) + h(y+1), d_s = h(y-1) - h(y+1) at x-1, x, x+1;
-                // nx = v_s(x-1) - v_s(x+1), nz = d_s(x-1) + 2 d_s(x) + d_s(x+1)
-                const float vl  = hl[g - 1].x + 2.0f * hl[g].x + hl[g + 1].x;
-                const float vr  = hr[g - 1].x + 2.0f * hr[g].x + hr[g + 1].x;
-                const float nx  = vl - vr;
-                const float nz  = (hl[g - 1].x - hl[g + 1].x) + 2.0f * (hm[g - 1].x - hm[g + 1].x) +
-                                  (hr[g - 1].x - hr[g + 1].x);
+                float nx, nz;
+                if constexpr (BIL) {
+                    auto vs = [&](float a, float b, float c, float d) { return a + 3.0f * (b + c) + d; };
+                    auto ds = [&](float a, float b, float c, float d) { return (a + b) - (c + d); };
+                    const float v0 = vs(hll[g - 2], hll[g - 1], hll[g], hll[g + 1]);
+                    const float v1 = vs(hl[g - 2].x, hl[g - 1].x, hl[g].x, hl[g + 1].x);
+                    const float v2 = vs(hm[g - 2].x, hm[g - 1].x, hm[g].x, hm[g + 1].x);
+                    const float v3 = vs(hr[g - 2].x, hr[g - 1].x, hr[g].x, hr[g + 1].x);
+                    const float d0 = ds(hll[g - 2], hll[g - 1], hll[g], hll[g + 1]);
+                    const float d1 = ds(hl[g - 2].x, hl[g - 1].x, hl[g].x, hl[g + 1].x);
+                    const float d2 = ds(hm[g - 2].x, hm[g - 1].x, hm[g].x, hm[g + 1].x);
+                    const float d3 = ds(hr[g - 2].x, hr[g - 1].x, hr[g].x, hr[g + 1].x);
+                    nx = 0.25f * ds(v0, v1, v2, v3);
+                    nz = 0.25f * vs(d0, d1, d2, d3);
+                } else {
+                    // v_s = h(y-1) + 2 h(y) + h(y+1), d_s = h(y-1) - h(y+1) at x-1, x, x+1;
+                    // nx = v_s(x-1) - v_s(x+1), nz = d_s(x-1) + 2 d_s(x) + d_s(x+1)
+                    const float vl  = hl[g - 1].x + 2.0f * hl[g].x + hl[g + 1].x;
+                    const float vr  = hr[g - 1].x + 2.0f * hr[g].x + hr[g + 1].x;
+                    nx = vl - vr;
+                    nz = (hl[g - 1].x - hl[g + 1].x) + 2.0f * (hm[g - 1].x - hm[g + 1].x) +
+                         (hr[g - 1].x - hr[g + 1].x);
+                }
                 const float inv = rsqrtf(fmaf(nx, nx, fmaf(nz, nz, 1.0f)));
                 st_out(&normals[o], make_float4(nx * inv, inv, nz * inv, 1.0f));
             }
-            if (jac) {
+            if (jac || (RENDER && (disp || rnorm))) {
                 const float dxdx = (hr[g].y - hl[g].y) * inv2d;
-                const float dzdx = (zr[g] - zl[g]) * inv2d;
+                const float dzdx = (zr[i] - zl[i]) * inv2d;
                 const float dxdz = (hm[g + 1].y - hm[g - 1].y) * inv2d;
-                const float dzdz = (zm[g + 1] - zm[g - 1]) * inv2d;
-                st_out(&jac[o], (1.0f - lambda * dxdx) * (1.0f - lambda * dzdz) - lambda * lambda * dxdz * dzdx);
+                const float dzdz = (zm[i + 1] - zm[i - 1]) * inv2d;
+                const float J = (1.0f - lambda * dxdx) * (1.0f - lambda * dzdz) - lambda * lambda * dxdz * dzdx;
+                if (jac) st_out(&jac[o], J);
+                if (RENDER && disp)
+                    st_out(&disp[o], make_float4(-lambda * hm[g].y, dscale * hm[g].x, -lambda * zm[i], J));
+                if (RENDER && rnorm) {
+                    // n = dP/dv x dP/du (rows_nrm_band); its y component is J
+                    const float dhdx = (hr[g].x - hl[g].x) * inv2d, dhdz = (hm[g + 1].x - hm[g - 1].x) * inv2d;
+                    const float nx  = -dscale * (lambda * dhdz * dzdx + (1.0f - lambda * dzdz) * dhdx);
+                    const float nz  = -dscale * (lambda * dxdz * dhdx + dhdz * (1.0f - lambda * dxdx));
+                    const float inv = rsqrtf(fmaf(nx, nx, fmaf(J, J, nz * nz)));
+                    st_out(&rnorm[o], make_float4(nx * inv, J * inv, nz * inv, 1.0f));
+                }
             }
             st_out(&height[o], hm[g].x);
             st_out(&dx[o], hm[g].y);
-            st_out(&dz[o], zm[g]);
+            st_out(&dz[o], zm[i]);
         }
     }
 }
@@ -619,11 +663,11 @@ constexpr RowsVariant kRowsVariants[kNumRowsVariants] = {{16, 0, false, 1}, {8, 
                                                          {16, 4, true, 1},  {16, 2, true, 1},  {16, 2, true, 2}};
 
 constexpr bool cols_fits(int N, int v) { return N >= kColsVariants[v].min_N && N <= kColsVariants[v].max_N; }
-template <int N, int E, int B, bool PAR = false, int W = 1>
+template <int N, int E, int B, bool PAR = false, int W = 1, bool BIL = false>
 constexpr bool rows_fits()
 {
     if constexpr (PAR) {
-        constexpr int T = N / E, G = par_groups<N, E, B>();
+        constexpr int T = N / E, G = par_groups<N, E, B, BIL>();
         return N >= 2 * E && N % B == 0 && (T % 64 == 0 || 64 % T == 0) && (W == 1 || T <= 64) &&
                W * G * T <= 1024 && G * lds_len(N) * 8 <= 160 * 1024;
     } else if constexpr (B == 0) {
@@ -662,11 +706,21 @@ static hipError_t launch_rows_v(const FrameArgs& a, hipStream_t s)
     if constexpr (!rows_fits<N, E, B, P, W>()) {
         return hipErrorInvalidValue;
     } else if constexpr (P) {
-        constexpr int T = N / E;
-        hipLaunchKernelGGL((k_rows_nrm_par<N, E, B, W>), dim3((N / B) * a.nframes),
-                           dim3(W * par_groups<N, E, B>() * T), 0, s, a.z1, a.z2, a.height, a.dx, a.dz, a.normals,
-                           a.jacobian, a.tw[radix_slot(E)], a.fb, a.lambda, a.inv2d);
-        return hipGetLastError();
+        auto launch = [&](auto bil, auto ren) {
+            constexpr bool BIL = decltype(bil)::value, REN = decltype(ren)::value;
+            if constexpr (!rows_fits<N, E, B, true, W, BIL>()) {
+                return hipErrorInvalidValue;
+            } else {
+                hipLaunchKernelGGL((k_rows_nrm_par<N, E, B, W, BIL, REN>), dim3((N / B) * a.nframes),
+                                   dim3(W * par_groups<N, E, B, BIL>() * (N / E)), 0, s, a.z1, a.z2, a.height, a.dx,
+                                   a.dz, a.normals, a.jacobian, a.tw[radix_slot(E)], a.fb, a.lambda, a.inv2d, a.disp,
+                                   a.rnorm, a.dscale);
+                return hipGetLastError();
+            }
+        };
+        const bool ren = a.disp || a.rnorm;
+        if (a.normal_mode != 0) return ren ? launch(std::true_type{}, std::true_type{}) : launch(std::true_type{}, std::false_type{});
+        return ren ? launch(std::false_type{}, std::true_type{}) : launch(std::false_type{}, std::false_type{});
     } else if constexpr (B == 0) {
         hipLaunchKernelGGL((k_rows<N, E>), dim3(N / 2, a.nframes), dim3(3 * (N / E)), 0, s, a.z1, a.z2, a.height,
                            a.dx, a.dz, a.tw[radix_slot(E)], a.fb);
@@ -684,6 +738,26 @@ static hipError_t launch_rows_v(const FrameArgs& a, hipStream_t s)
                                a.lambda, a.inv2d, nullptr, nullptr, 0.0f);
         return hipGetLastError();
     }
+}
+
+// The row variant that a frame with bilinear normals takes for rv: the walks
+// read nearest taps only, so the parallel bands of 2 rows stand in for them; an
+// N whose bands do not fit a block with the extra row (4096) runs the unfused
+// radix-16 pass, and so does a single N = 2048 frame, whose textures the
+// normal-map kernel reads back from the Infinity Cache (75 us against 78 with
+// the bands, one block per CU; from 2 frames on 82 against 71).
+template <int N>
+constexpr int bilinear_rows(int rv, int nframes)
+{
+#define OCN_BFITS(v) \
+    (rows_fits<N, kRowsVariants[v].E, kRowsVariants[v].band, kRowsVariants[v].par, kRowsVariants[v].W, true>())
+    if (kRowsVariants[rv].band == 0) return rv;
+    if (!kRowsVariants[rv].par) {
+        if (N == 2048 && nframes == 1) return 0;
+        rv = 7;
+    }
+    return (rv == 6 ? OCN_BFITS(6) : rv == 7 ? OCN_BFITS(7) : OCN_BFITS(8)) ? rv : 0;
+#undef OCN_BFITS
 }
 
 template <int N>
@@ -718,13 +792,13 @@ static hipError_t launch_frame_n(const FrameArgs& a, int stages, hipStream_t s)
         }
         if (e != hipSuccess) return e;
     }
-    // The fused row variants cover the normal map and Jacobian (nearest taps
-    // only); with bilinear normals the unfused radix-16 row pass is used.  The
-    // parallel-band variants write no render export: with one requested the
-    // unfused radix-8 pass and the normal-map kernel write it.
-    int rv = a.rows_variant;
-    if (rv >= 0 && rv < kNumRowsVariants && kRowsVariants[rv].band > 0 && a.normal_mode != 0) rv = 0;
-    if (rv >= 0 && rv < kNumRowsVariants && kRowsVariants[rv].par && (a.disp || a.rnorm)) rv = 1;
+    // Bilinear normals and the parallel bands' render export are fused into the
+    // row pass of a whole frame only: the row or the normal-map stage by itself
+    // is the unfused kernel, which works from and on the output textures.
+    int        rv  = a.rows_variant;
+    const bool bil = a.normal_mode != 0, ren = a.disp || a.rnorm, whole = (stages & 6) == 6;
+    if (rv >= 0 && rv < kNumRowsVariants && bil) rv = whole ? bilinear_rows<N>(rv, a.nframes) : kRowsVariants[rv].band > 0 ? 0 : rv;
+    if (rv >= 0 && rv < kNumRowsVariants && kRowsVariants[rv].par && ren && !whole) rv = 1;
     const bool fused = rv >= 0 && rv < kNumRowsVariants && kRowsVariants[rv].band > 0;
     if (stages & 2) {
         switch (rv) {
@@ -821,9 +895,15 @@ void cols_variant_shape(int N, int v, int* E, int* C)
 
 int rows_variant_radix(int v) { return kRowsVariants[v].E; }
 
-int rows_variant_band(int v) { return kRowsVariants[v].band; }
+int rows_variant_band(int N, int v, bool bilinear, int nframes)
+{
+    if (!bilinear) return kRowsVariants[v].band;
+#define CALL(n) kRowsVariants[bilinear_rows<n>(v, nframes)].band
+    OCN_DISPATCH_N(N, CALL, 0)
+#undef CALL
+}
 
-bool rows_variant_parallel(int v) { return kRowsVariants[v].par; }
+bool rows_variant_walk(int v) { return kRowsVariants[v].band > 0 && !kRowsVariants[v].par; }
 
 hipError_t launch_ifft2(int N, const float2* src, float2* tmp, float* out, const float2* const* tw, hipStream_t s)
 {

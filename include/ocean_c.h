@@ -273,7 +273,7 @@ int ocn_frames_reserved(const ocn_handle* h, int* nframes);
  * it synchronises; it reserves nframes frames as ocn_reserve_frames does) and
  * records the fastest for (device, N, frames-per-launch class, normal mode);
  * later launches of any handle with that N and normal mode use it.  With
- * bilinear normals only the unfused row variants are timed.  ocn_set_schedule
+ * bilinear normals, which no row walk reads, the walks are not timed.  ocn_set_schedule
  * pins a variant pair on this handle; ocn_get_schedule reports the pair used
  * for launches of nframes frames and its shape (any out-pointer may be NULL);
  * rows_band > 0 means the normal map and Jacobian are fused into the row pass,
