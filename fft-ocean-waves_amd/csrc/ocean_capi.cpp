@@ -590,6 +590,8 @@ struct ocn_fit {
     std::vector<ocn::FitMember>           members;  // host copy of the device descriptors
     ocn::FitMember*                       d_members = nullptr;
     ocn::FitVars*                         d_vars    = nullptr;
+    ocn::FitRange*                        d_ranges  = nullptr;
+    float4*                               d_parts   = nullptr;
     int2*                                 d_cols    = nullptr;
     int                                   n_cols    = 0;
     char*                                 pool      = nullptr;
@@ -604,7 +606,7 @@ namespace {
 
 void fit_free(ocn_fit* f)
 {
-    void* ptrs[] = {f->d_members, f->d_vars, f->d_cols, f->pool};
+    void* ptrs[] = {f->d_members, f->d_vars, f->d_ranges, f->d_parts, f->d_cols, f->pool};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     for (auto& kv : f->tw)
@@ -640,8 +642,9 @@ int fit_run(ocn_fit* f, int mode, const ocn::AdamCfg& adam, const ocn::QnCfg& qn
             if (e == hipSuccess) f->targets_dirty[i] = 0;
         }
     if (e == hipSuccess)
-        e = ocn::launch_fit(f->d_members, (int)f->members.size(), f->d_cols, f->n_cols, mode, adam, qn,
-                            (hipStream_t)stream);
+        e = ocn::launch_fit({f->d_members, f->d_vars, f->d_ranges, f->d_cols, f->d_parts, (int)f->members.size(),
+                             f->n_cols},
+                            mode, adam, qn, (hipStream_t)stream);
     return e == hipSuccess ? OCN_OK : hip_fail(e, "fit launch");
 }
 
@@ -1606,9 +1609,9 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
     int        rc = OCN_OK;
     hipError_t e  = hipGetDevice(&f->device);
     if (e != hipSuccess) rc = hip_fail(e, "hipGetDevice");
-    // Per member, 256-byte aligned: xi 16, scratch 8, targets 4 K, dL/dh0 16 bytes per texel, partials,
+    // Per member, 256-byte aligned: xi 16, scratch 8, targets 4 K, dL/dh0 16 bytes per texel,
     // the targets' spectra T^ (8 bytes per frame and texel pair of the half plane), with equally spaced
-    // times the phase table (16 bytes per texel pair of the half plane), the noise coefficients (16 bytes
+    // times and split strips the phase table (16 bytes per texel pair of the half plane), the noise coefficients (16 bytes
     // per texel pair of the half plane) and the unit noise of the edge pairs (32 bytes each).
     // Small fits split each column strip's rows over up to four blocks so the
     // step launch has at least two blocks per CU of the 256.
@@ -1619,12 +1622,16 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
         while (row_parts < ocn::kFitMaxRowParts && items * row_parts < 512) row_parts *= 2;
     }
     auto   al    = [](size_t x) { return (x + 255) & ~size_t(255); };
-    auto   phase_bytes = [&](int N) { return uniform_times ? al(sizeof(float4) * ocn::fit_phase_entries(N)) : 0; };
+    // Equally spaced times: a step of whole strips is bound by memory and evaluates
+    // its pairs' phases, 16 of the 64 bytes a pair would read at K = 4 (256 oceans of
+    // N = 256, 96 -> 75 us; one of N = 1024, K = 8, 15.5 -> 15.0); one of split strips
+    // is bound by latency and reads them from a table (N = 512, K = 8: 7.8 us, 8.2
+    // evaluated).
+    const bool phase_table = uniform_times && row_parts > 1;
+    auto   phase_bytes = [&](int N) { return phase_table ? al(sizeof(float4) * ocn::fit_phase_entries(N)) : 0; };
     auto   bytes = [&](int N) {
         const size_t nn = (size_t)N * N;
         return al(nn * 16) + al(nn * 8) + al(nn * 4 * K) + al(nn * 16) +
-               al(sizeof(float) * ocn::fit_cols_items_per_member(N) * row_parts) +
-               al(sizeof(float) * 3 * ocn::fit_cols_items_per_member(N) * row_parts) +
                al(sizeof(float2) * K * ocn::fit_phase_entries(N)) + phase_bytes(N) +
                al(sizeof(float4) * ocn::fit_phase_entries(N)) + al(2 * sizeof(float4) * ocn::fit_edge_pairs(N));
     };
@@ -1640,9 +1647,10 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
     }
     if (!rc) rc = dalloc(&f->d_vars, (size_t)count, "fit variables");
     if (!rc) {
-        std::vector<ocn::FitVars> vars;
-        char*                     q = f->pool;
-        std::vector<int2>         cols;
+        std::vector<ocn::FitVars>  vars;
+        std::vector<ocn::FitRange> ranges;
+        char*                      q = f->pool;
+        std::vector<int2>          cols;
         for (int i = 0; i < count; ++i) {
             const ocn_params& p  = f->params[i];
             const size_t      nn = (size_t)p.N * p.N;
@@ -1665,29 +1673,28 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
             m.targets   = reinterpret_cast<const float*>(q), q += al(nn * 4 * K);
             m.grad_h0   = reinterpret_cast<float4*>(q), q += al(nn * 16);
             m.row_parts   = row_parts;
-            m.n_loss_part = ocn::fit_cols_items_per_member(p.N) * row_parts;  // one partial per step block
-            m.n_grad_part = m.n_loss_part;
-            m.loss_part = reinterpret_cast<float*>(q), q += al(sizeof(float) * m.n_loss_part);
-            m.grad_part = reinterpret_cast<float*>(q), q += al(sizeof(float) * 3 * m.n_grad_part);
             m.that      = reinterpret_cast<float2*>(q), q += al(sizeof(float2) * K * ocn::fit_phase_entries(p.N));
-            m.phase     = uniform_times ? reinterpret_cast<const float4*>(q) : nullptr, q += phase_bytes(p.N);
+            m.phase     = phase_table ? reinterpret_cast<const float4*>(q) : nullptr, q += phase_bytes(p.N);
             m.pq        = reinterpret_cast<const float4*>(q), q += al(sizeof(float4) * ocn::fit_phase_entries(p.N));
             m.edge      = reinterpret_cast<const float4*>(q), q += al(2 * sizeof(float4) * ocn::fit_edge_pairs(p.N));
             m.tw8       = f->tw[p.N][0];
             m.tw16      = f->tw[p.N][1];
-            m.vars      = f->d_vars + i;
             m.key0      = (uint32_t)p.seed;
             m.key1      = (uint32_t)(p.seed >> 32);
             m.ocean_id  = p.ocean_id;
             m.cascade_id = p.cascade_id;
             f->members.push_back(m);
             vars.push_back(initial_vars(p));
-            for (int k = 0; k < m.n_grad_part; ++k) cols.push_back(make_int2(i, k));
+            const int blocks = ocn::fit_cols_items_per_member(p.N) * row_parts;  // one partial each
+            ranges.push_back({(int)cols.size(), blocks, (double)K * (double)nn, p.gravity});
+            for (int k = 0; k < blocks; ++k) cols.push_back(make_int2(i, k));
         }
         f->n_cols = (int)cols.size();
         f->targets_dirty.assign(count, 1);
         if (!(rc = upload_vector(&f->d_members, f->members, "fit members")) &&
-            !(rc = upload_vector(&f->d_cols, cols, "fit column items"))) {
+            !(rc = upload_vector(&f->d_cols, cols, "fit column items")) &&
+            !(rc = upload_vector(&f->d_ranges, ranges, "fit ranges")) &&
+            !(rc = dalloc(&f->d_parts, cols.size(), "fit partial sums"))) {
             e = hipMemcpy(f->d_vars, vars.data(), sizeof(ocn::FitVars) * vars.size(), hipMemcpyHostToDevice);
             if (e != hipSuccess) rc = hip_fail(e, "hipMemcpy(fit variables)");
         }
@@ -1695,7 +1702,7 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
             if ((e = ocn::launch_fit_xi(f->members[i], nullptr)) != hipSuccess) rc = hip_fail(e, "fit noise launch");
             else if ((e = ocn::launch_fit_pq(f->members[i], nullptr)) != hipSuccess)
                 rc = hip_fail(e, "fit noise coefficients launch");
-            else if (uniform_times && (e = ocn::launch_fit_phase(f->members[i], nullptr)) != hipSuccess)
+            else if (phase_table && (e = ocn::launch_fit_phase(f->members[i], nullptr)) != hipSuccess)
                 rc = hip_fail(e, "fit phase launch");
         }
         if (!rc && (e = hipDeviceSynchronize()) != hipSuccess) rc = hip_fail(e, "hipDeviceSynchronize");
@@ -1768,7 +1775,7 @@ int ocn_fit_set_vars(ocn_fit* f, int member, const double vars[3])
     ocn::fit_vars_derive(v, f->params[member].gravity);
     hipError_t e = hipSetDevice(f->device);
     if (e == hipSuccess) e = hipDeviceSynchronize();
-    if (e == hipSuccess) e = hipMemcpy(f->members[member].vars, &v, sizeof(v), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(f->d_vars + member, &v, sizeof(v), hipMemcpyHostToDevice);
     return e == hipSuccess ? OCN_OK : hip_fail(e, "hipMemcpy(fit variables)");
 }
 
@@ -1823,7 +1830,7 @@ int ocn_fit_get(ocn_fit* f, int member, double vars[3], double grad[3], double* 
     ocn::FitVars v{};
     hipError_t   e = hipSetDevice(f->device);
     if (e == hipSuccess) e = hipStreamSynchronize((hipStream_t)stream);
-    if (e == hipSuccess) e = hipMemcpy(&v, f->members[member].vars, sizeof(v), hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = hipMemcpy(&v, f->d_vars + member, sizeof(v), hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_fail(e, "hipMemcpy(fit variables)");
     if (vars) {
         vars[0] = v.V;

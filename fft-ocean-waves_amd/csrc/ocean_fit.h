@@ -37,18 +37,41 @@ struct FitVars {
     float  Lp2, iLp2, Af, wx, wy, dv_scale, da_scale, sqA;
 };
 
-__host__ __device__ inline void fit_vars_derive(FitVars& v, double g)
+// The derived constants of each variable by itself (the reduction derives the
+// three side by side).
+__host__ __device__ inline void fit_derive_V(FitVars& v, double V, double g)
 {
-    const double Lp = v.V * v.V / g;
+    const double Lp = V * V / g;
     v.Lp2      = (float)(Lp * Lp);
     v.iLp2     = 1.0f / v.Lp2;
-    v.Af       = (float)v.A;
-    v.wx       = (float)cos(v.theta);
-    v.wy       = (float)sin(v.theta);
-    v.dv_scale = (float)(2.0 * g * g / (v.V * v.V * v.V * v.V * v.V));
-    v.da_scale = (float)(0.5 / v.A);
-    v.sqA      = (float)sqrt(v.A);
+    v.dv_scale = (float)(2.0 * g * g / (V * V * V * V * V));
 }
+__host__ __device__ inline void fit_derive_theta(FitVars& v, double theta)
+{
+    double s, c;
+    sincos(theta, &s, &c);
+    v.wx = (float)c;
+    v.wy = (float)s;
+}
+__host__ __device__ inline void fit_derive_A(FitVars& v, double A)
+{
+    v.Af       = (float)A;
+    v.da_scale = (float)(0.5 / A);
+    v.sqA      = (float)sqrt(A);
+}
+__host__ __device__ inline void fit_vars_derive(FitVars& v, double g)
+{
+    fit_derive_V(v, v.V, g);
+    fit_derive_theta(v, v.theta);
+    fit_derive_A(v, v.A);
+}
+
+// One member for the reduction: its partial sums are parts[start, start + count).
+struct FitRange {
+    int    start, count;
+    double knn;  // K * N * N
+    double g;
+};
 
 struct AdamCfg {
     double lr[3];
@@ -83,10 +106,10 @@ struct FitMember {
     // per pair at fit_edge_index.
     const float4* pq;
     const float4* edge;
-    // Equally spaced times: per column item and texel pair of its strip, the
-    // dispersion phase e^{i w t_0} and its step e^{i w dt} as (cos, sin,
-    // cos, sin), written once at creation (launch_fit_phase); entry
-    // (strip * N + ty) * C + c.  Null for other time sets.
+    // Equally spaced times and split strips: per column item and texel pair
+    // of its strip, the dispersion phase e^{i w t_0} and its step e^{i w dt} as
+    // (cos, sin, cos, sin), written once at creation (launch_fit_phase); entry
+    // (strip * N + ty) * C + c.  Null otherwise.
     const float4* phase;
     const float2* tw8;      // Stockham twiddles (N, 8) and (N, 16)
     const float2* tw16;
@@ -99,10 +122,6 @@ struct FitMember {
     // order).  Written by launch_fit_targets whenever the targets change.
     float2* that;
     float4* grad_h0;        // N*N: dL/dh0 as (dRe h0k, dIm h0k, dRe h0mk, dIm h0mk)
-    float*  loss_part;      // one partial sum per column item and row part
-    float*  grad_part;      // three partial sums per column item and row part
-    int     n_loss_part, n_grad_part;
-    FitVars* vars;
     uint32_t key0, key1, ocean_id, cascade_id;  // Philox noise of xi
 };
 
@@ -129,8 +148,17 @@ hipError_t launch_fit_targets(const FitMember& m, hipStream_t s);
 hipError_t launch_fit_pq(const FitMember& m, hipStream_t s);
 // Fills m.phase (a member with equally spaced times) from its constants.
 hipError_t launch_fit_phase(const FitMember& m, hipStream_t s);
-// cols_items: int2 (member, strip * row_parts + part): one block each for the step kernel
-hipError_t launch_fit(const FitMember* members, int n_members, const int2* cols_items, int n_cols, int mode,
-                      const AdamCfg& adam, const QnCfg& qn, hipStream_t s);
+// The device tables of a fit.  items: int2 (member, strip * row_parts + part), member
+// by member, one block each for the step kernel, which leaves its sums (loss,
+// dL/dV, dL/dtheta, dL/dA) at parts[item].
+struct FitTables {
+    const FitMember* members;
+    FitVars*         vars;
+    const FitRange*  ranges;
+    const int2*      items;
+    float4*          parts;
+    int              n_members, n_items;
+};
+hipError_t launch_fit(const FitTables& t, int mode, const AdamCfg& adam, const QnCfg& qn, hipStream_t s);
 
 }  // namespace ocn

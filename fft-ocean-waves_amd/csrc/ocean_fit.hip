@@ -94,18 +94,23 @@ __device__ __forceinline__ float2 phase_at(double w, double t_rev)
     return make_float2(c, s);
 }
 
-template <class T>
-__device__ __forceinline__ T block_sum(T x, T* red)
+// Sums of four values over the block, in one pass: across each wave, then over
+// the waves in order (the result is thread 0's).  red holds one float4 per wave.
+__device__ __forceinline__ float4 block_sum4(float4 t, float4* red)
 {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-    const int w = threadIdx.x / 64;
+    for (int o = 32; o > 0; o >>= 1) {
+        t.x += __shfl_xor(t.x, o);
+        t.y += __shfl_xor(t.y, o);
+        t.z += __shfl_xor(t.z, o);
+        t.w += __shfl_xor(t.w, o);
+    }
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64] = t;
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[w] = x;
-    __syncthreads();
-    T t = 0;
-    for (int i = 0; i < (int)(blockDim.x / 64); ++i) t += red[i];
-    return t;
+    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int i = 0; i < (int)(blockDim.x / 64); ++i)
+        s = make_float4(s.x + red[i].x, s.y + red[i].y, s.z + red[i].z, s.w + red[i].w);
+    return s;
 }
 
 // The fit's unit noise xi is stored in column strips: texel (x, y) at
@@ -184,16 +189,18 @@ __device__ __forceinline__ void param_add(const ParamGeo& g, float dl, float dv_
 // columns 0 and N/2, whose rows hold u and -u as texels of their own.  The
 // gradient of L = sum / (K N^2) with respect to the spectrum H(u) of the
 // texel is 2 D / (K N^4), and conj of it for -u: the pull-back takes it to
-// dL/dh0, then to dL/ds and the parameter partials.  Loss partials hold
-// sum_x (h_k - T_k)^2 (k_fit_reduce divides by K N^2).
-template <int N, bool UNIFORM, int R>
-__device__ __forceinline__ void fit_spectral(const FitMember& m, int item, int mode, float* red)
+// dL/dh0, then to dL/ds and the parameter partials.  Returns the thread's sums;
+// the loss's are of sum_x (h_k - T_k)^2 (k_fit_reduce divides by K N^2).
+// PHASE: where the frames' phases come from.
+enum { kPhaseEach, kPhaseTable, kPhaseStart };  // evaluated per frame; equally spaced times: table, or evaluated start
+template <int N, int PHASE, int R>
+__device__ __forceinline__ float4 fit_spectral(const FitMember& m, const FitVars& vars, int item, int mode)
 {
+    constexpr bool TABLE = PHASE == kPhaseTable, UNIFORM = PHASE != kPhaseEach;
     constexpr int C = fit_cols_per_block(N), NT = kFitColsThreads, IT = C * N / NT / R;
     static_assert((C * N) % (NT * R) == 0, "whole texel pairs per thread");
     // block `item` covers part `item % R` of the strip's C * N texel pairs
     const int strip = item / R, it0 = (item % R) * IT * NT;
-    const FitVars   vars = *m.vars;
     const SpecConst sc   = fit_spec(m, vars);
     const bool      grad = mode != kFitLoss;
     const bool      store_grad_h0 = mode == kFitGrad;
@@ -223,7 +230,7 @@ __device__ __forceinline__ void fit_spectral(const FitMember& m, int item, int m
         } else {
             na = m.pq[base + kk];
         }
-        if constexpr (UNIFORM) nph = m.phase[base + kk];
+        if constexpr (TABLE) nph = m.phase[base + kk];
 #pragma unroll
         for (int q = 0; q < 4; ++q)
             nT[q] = q < m.K ? m.that[(size_t)q * ne + base + kk] : make_float2(0.0f, 0.0f);
@@ -264,12 +271,13 @@ __device__ __forceinline__ void fit_spectral(const FitMember& m, int item, int m
         }
         PhaseWalk walk;
         double    w = 0.0;
-        if constexpr (UNIFORM) {
+        if constexpr (TABLE) {
             walk.load(ph);
         } else {
             const int nx = tx - N / 2, ny = ty - N / 2;
             float     kinv;
             w = omega_fp64(sc, nx * nx + ny * ny, kinv);
+            if constexpr (UNIFORM) walk.start(w, m.t_rev[0], m.dt_rev);
         }
         const float wt = self ? inv_nn : 2.0f * inv_nn;
         // With H = h0k e + C(h0mk) conj(e) at u and G the same at -u, the fold
@@ -334,18 +342,7 @@ __device__ __forceinline__ void fit_spectral(const FitMember& m, int item, int m
         if (self || paired) continue;
         if (gm.live) param_add(gm, dl_ds(gam, gbm, b), dv_scale, da_scale, dV, dT, dA);
     }
-    lsum = block_sum(lsum, red);
-    if (threadIdx.x == 0) m.loss_part[item] = lsum;
-    if (grad) {
-        dV = block_sum(dV, red);
-        dT = block_sum(dT, red);
-        dA = block_sum(dA, red);
-        if (threadIdx.x == 0) {
-            m.grad_part[3 * item + 0] = dV;
-            m.grad_part[3 * item + 1] = dT;
-            m.grad_part[3 * item + 2] = dA;
-        }
-    }
+    return make_float4(lsum, dV, dT, dA);
 }
 
 // T^ of one target frame, rows: R(t, y) = sum_x (-1)^(x+y) T(x, y) e^{-2 pi i t x / N}
@@ -394,10 +391,12 @@ __device__ __forceinline__ void fit_targets_col(const float2* __restrict__ R, fl
 }  // namespace
 
 template <int N, int R>
-__device__ __forceinline__ void fit_spectral_parts(const FitMember& m, int item, int mode, float* red)
+__device__ __forceinline__ float4 fit_spectral_parts(const FitMember& m, const FitVars& v, int item, int mode)
 {
-    if (m.uniform) fit_spectral<N, true, R>(m, item, mode, red);
-    else fit_spectral<N, false, R>(m, item, mode, red);
+    if (m.phase) return fit_spectral<N, kPhaseTable, R>(m, v, item, mode);
+    if constexpr (R == 1)  // split strips are few: equally spaced times always have the table
+        if (m.uniform) return fit_spectral<N, kPhaseStart, R>(m, v, item, mode);
+    return fit_spectral<N, kPhaseEach, R>(m, v, item, mode);
 }
 
 #define OCN_FIT_SWITCH(N_, CALL)                 \
@@ -411,17 +410,24 @@ __device__ __forceinline__ void fit_spectral_parts(const FitMember& m, int item,
     }
 
 __global__ __launch_bounds__(kFitColsThreads) void k_fit_spectral(const FitMember* __restrict__ members,
-                                                                  const int2* __restrict__ items, int mode)
+                                                                  const FitVars* __restrict__ vars,
+                                                                  const int2* __restrict__ items,
+                                                                  float4* __restrict__ parts, int mode)
 {
-    __shared__ float red[kFitColsThreads / 64];
-    const int2       it = items[xcd_logical(blockIdx.x, gridDim.x)];
-    const FitMember& m  = members[it.x];
+    __shared__ float4 red[kFitColsThreads / 64];
+    const int        idx = xcd_logical(blockIdx.x, gridDim.x);
+    const int2       it  = items[idx];
+    const FitMember& m   = members[it.x];
+    const FitVars&   v   = vars[it.x];
+    float4           s   = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #define OCN_CALL(n) \
-    if (m.row_parts == 4) fit_spectral_parts<n, 4>(m, it.y, mode, red); \
-    else if (m.row_parts == 2) fit_spectral_parts<n, 2>(m, it.y, mode, red); \
-    else fit_spectral_parts<n, 1>(m, it.y, mode, red)
+    if (m.row_parts == 4) s = fit_spectral_parts<n, 4>(m, v, it.y, mode); \
+    else if (m.row_parts == 2) s = fit_spectral_parts<n, 2>(m, v, it.y, mode); \
+    else s = fit_spectral_parts<n, 1>(m, v, it.y, mode)
     OCN_FIT_SWITCH(m.N, OCN_CALL)
 #undef OCN_CALL
+    s = block_sum4(s, red);
+    if (threadIdx.x == 0) parts[idx] = s;
 }
 
 template <int N>
@@ -465,29 +471,34 @@ __global__ __launch_bounds__(256) void k_fit_xi(float4* __restrict__ xi, int N, 
 //     reached it, and the trial becomes the anchor;
 // then the next trial is z_anchor + p, p = -H g_anchor cut to the radius.
 // Wind speed and amplitude stay positive (floors 1e-3 and 1e-6).
-__device__ void qn_step(FitVars& v, double L, const double g[3], const QnCfg& cfg)
+__device__ __forceinline__ void qn_step(FitVars& v, double L, const double g[3], const QnCfg& cfg)
 {
     double z[3], gz[3];
     z[0] = v.V / cfg.scale[0];
     z[1] = v.theta / cfg.scale[1];
     z[2] = v.A / cfg.scale[2];
+#pragma unroll
     for (int i = 0; i < 3; ++i) gz[i] = g[i] * cfg.scale[i];
-    auto H = [&](int i, int j) -> double& {
-        const int a = i < j ? i : j, b = i < j ? j : i;
-        return v.qH[a == 0 ? b : a == 1 ? 2 + b : 5];
+    // the symmetric inverse Hessian (xx, xy, xz, yy, yz, zz), in registers
+    double h0 = v.qH[0], h1 = v.qH[1], h2 = v.qH[2], h3 = v.qH[3], h4 = v.qH[4], h5 = v.qH[5];
+    auto   row = [&](int i, double x, double y, double z) {
+        return i == 0 ? h0 * x + h1 * y + h2 * z : i == 1 ? h1 * x + h3 * y + h4 * z : h2 * x + h4 * y + h5 * z;
     };
     bool anchor = false;
     if (v.qn == 0) {
-        for (int i = 0; i < 6; ++i) v.qH[i] = (i == 0 || i == 3 || i == 5) ? 1.0 : 0.0;
+        h0 = h3 = h5 = 1.0;
+        h1 = h2 = h4 = 0.0;
         v.qr   = cfg.radius;
         v.qk   = 0;
         anchor = true;
     } else if (!(L <= v.qL)) {
         double d2 = 0.0;
+#pragma unroll
         for (int i = 0; i < 3; ++i) d2 += (z[i] - v.qz[i]) * (z[i] - v.qz[i]);
         v.qr = 0.25 * sqrt(d2);
     } else {
         double s[3], y[3], sy = 0.0, ss = 0.0, yy = 0.0;
+#pragma unroll
         for (int i = 0; i < 3; ++i) {
             s[i] = z[i] - v.qz[i];
             y[i] = gz[i] - v.qg[i];
@@ -496,37 +507,35 @@ __device__ void qn_step(FitVars& v, double L, const double g[3], const QnCfg& cf
             yy += y[i] * y[i];
         }
         if (sy > 1e-12 * sqrt(ss * yy)) {
-            if (v.qk == 0)
-                for (int i = 0; i < 6; ++i) v.qH[i] *= sy / yy;
+            if (v.qk == 0) {
+                const double c = sy / yy;
+                h0 *= c, h1 *= c, h2 *= c, h3 *= c, h4 *= c, h5 *= c;
+            }
             // H <- (I - rho s y^T) H (I - rho y s^T) + rho s s^T
             const double rho = 1.0 / sy;
-            double       Hy[3], yHy = 0.0;
-            for (int i = 0; i < 3; ++i) {
-                Hy[i] = 0.0;
-                for (int j = 0; j < 3; ++j) Hy[i] += H(i, j) * y[j];
-                yHy += y[i] * Hy[i];
-            }
-            double nh[6];
-            for (int i = 0, k = 0; i < 3; ++i)
-                for (int j = i; j < 3; ++j, ++k)
-                    nh[k] = H(i, j) - rho * (s[i] * Hy[j] + Hy[i] * s[j]) + (rho * rho * yHy + rho) * s[i] * s[j];
-            for (int k = 0; k < 6; ++k) v.qH[k] = nh[k];
+            const double Hy[3] = {row(0, y[0], y[1], y[2]), row(1, y[0], y[1], y[2]), row(2, y[0], y[1], y[2])};
+            const double yHy = y[0] * Hy[0] + y[1] * Hy[1] + y[2] * Hy[2], c = rho * rho * yHy + rho;
+            auto         upd = [&](double h, int i, int j) { return h - rho * (s[i] * Hy[j] + Hy[i] * s[j]) + c * s[i] * s[j]; };
+            h0 = upd(h0, 0, 0), h1 = upd(h1, 0, 1), h2 = upd(h2, 0, 2);
+            h3 = upd(h3, 1, 1), h4 = upd(h4, 1, 2), h5 = upd(h5, 2, 2);
             v.qk += 1;
         }
         if (sqrt(ss) >= 0.99 * v.qr) v.qr = fmin(2.0 * v.qr, cfg.radius_max);
         anchor = true;
     }
     if (anchor) {
+#pragma unroll
         for (int i = 0; i < 3; ++i) {
             v.qz[i] = z[i];
             v.qg[i] = gz[i];
         }
         v.qL = L;
     }
+    v.qH[0] = h0, v.qH[1] = h1, v.qH[2] = h2, v.qH[3] = h3, v.qH[4] = h4, v.qH[5] = h5;
     double p[3], pp = 0.0;
+#pragma unroll
     for (int i = 0; i < 3; ++i) {
-        p[i] = 0.0;
-        for (int j = 0; j < 3; ++j) p[i] -= H(i, j) * v.qg[j];
+        p[i] = -row(i, v.qg[0], v.qg[1], v.qg[2]);
         pp += p[i] * p[i];
     }
     const double f = pp > v.qr * v.qr ? v.qr / sqrt(pp) : 1.0;
@@ -539,62 +548,133 @@ __device__ void qn_step(FitVars& v, double L, const double g[3], const QnCfg& cf
 // One block per member: loss and gradient from the partial sums (FP64), then
 // optionally one Adam step on (V, theta, A) (Kingma & Ba 2015, bias-corrected).
 // V and A stay positive (floors 1e-3 and 1e-6).
-__global__ __launch_bounds__(kFitReduceThreads) void k_fit_reduce(const FitMember* __restrict__ members, int mode,
-                                                                  AdamCfg cfg, QnCfg qcfg)
+// A small fit waits for this kernel at every step, so its chain is kept short:
+// the loads do not depend on one another, Adam's powers are taken while the
+// partial sums arrive, and waves 0..2 step and derive one variable each
+// (wave 3 writes the loss).  Single N=512, K=8 fit, Adam step 12.9 -> 9.6 us.
+//
+// The four sums of a member, in its block's thread 0 of every wave: per thread,
+// across each wave, then over the waves in order.
+struct FitSums {
+    double loss, dV, dT, dA;
+};
+__device__ __forceinline__ FitSums fit_sums(const FitRange& rg, const float4* __restrict__ parts, float4 p,
+                                            double (*red)[4])
 {
-    constexpr int     NW = kFitReduceThreads / 64;
-    __shared__ double red[4 * NW];
-    const FitMember&  m = members[blockIdx.x];
-    // thread 0 loads the member's variables before the partial sums, so the
-    // two loads' latencies overlap
-    FitVars v;
-    if (threadIdx.x == 0) v = *m.vars;
-    double t[4] = {0.0, 0.0, 0.0, 0.0};  // loss, dL/dV, dL/dtheta, dL/dA
-    for (int i = threadIdx.x; i < m.n_loss_part; i += blockDim.x) t[0] += (double)m.loss_part[i];
-    if (mode != kFitLoss)
-        for (int i = threadIdx.x; i < m.n_grad_part; i += blockDim.x) {
-            t[1] += (double)m.grad_part[3 * i + 0];
-            t[2] += (double)m.grad_part[3 * i + 1];
-            t[3] += (double)m.grad_part[3 * i + 2];
-        }
-    // the four sums in one pass: across each wave, then over the waves in order
+    double a[4] = {(double)p.x, (double)p.y, (double)p.z, (double)p.w};
+    for (int i = threadIdx.x + kFitReduceThreads; i < rg.count; i += kFitReduceThreads) {
+        p = parts[rg.start + i];
+        a[0] += (double)p.x;
+        a[1] += (double)p.y;
+        a[2] += (double)p.z;
+        a[3] += (double)p.w;
+    }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) t[j] += __shfl_xor(t[j], o);
+        for (int j = 0; j < 4; ++j) a[j] += __shfl_xor(a[j], o);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) red[4 * (threadIdx.x / 64) + j] = t[j];
+        for (int j = 0; j < 4; ++j) red[threadIdx.x / 64][j] = a[j];
     __syncthreads();
-    if (threadIdx.x != 0) return;
-    double sum[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int w = 0; w < NW; ++w)
+    FitSums s{0.0, 0.0, 0.0, 0.0};
+    for (int w = 0; w < kFitReduceThreads / 64; ++w) {
+        s.loss += red[w][0];
+        s.dV += red[w][1];
+        s.dT += red[w][2];
+        s.dA += red[w][3];
+    }
+    return s;
+}
+
+__device__ __forceinline__ float4 fit_first_part(const FitRange& rg, const float4* __restrict__ parts)
+{
+    return (int)threadIdx.x < rg.count ? parts[rg.start + threadIdx.x] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+
+__global__ __launch_bounds__(kFitReduceThreads) void k_fit_reduce(const FitRange* __restrict__ ranges,
+                                                                  FitVars* __restrict__ all_vars,
+                                                                  const float4* __restrict__ parts, int mode,
+                                                                  AdamCfg cfg)
+{
+    static_assert(kFitReduceThreads == 256, "one wave per variable and one for the loss");
+    __shared__ double red[kFitReduceThreads / 64][4];
+    const FitRange rg   = ranges[blockIdx.x];
+    FitVars&       vars = all_vars[blockIdx.x];
+    const int      wave = threadIdx.x / 64, var = wave < 3 ? wave : 0;
+    const bool     lead = (threadIdx.x & 63) == 0;
+    const float4   p    = fit_first_part(rg, parts);
+    double         x = 0.0, m = 0.0, s = 0.0, b1t = 1.0, b2t = 1.0;
+    int            step = 0;
+    if (mode == kFitAdam && wave < 3) {
+        x    = var == 0 ? vars.V : var == 1 ? vars.theta : vars.A;
+        m    = vars.m[var];
+        s    = vars.v[var];
+        step = vars.step + 1;
+        // both powers at once, in even and odd lanes
+        const double bt = 1.0 - pow((threadIdx.x & 1) ? cfg.beta2 : cfg.beta1, (double)step);
+        b1t = __shfl(bt, 0);
+        b2t = __shfl(bt, 1);
+    }
+    const FitSums sum = fit_sums(rg, parts, p, red);
+    if (!lead) return;
+    if (wave == 3) vars.loss = sum.loss / rg.knn;
+    if (wave == 3 || mode == kFitLoss) return;
+    const double g = var == 0 ? sum.dV : var == 1 ? sum.dT : sum.dA;
+    vars.grad[var] = g;
+    if (mode != kFitAdam) return;
+    m = cfg.beta1 * m + (1.0 - cfg.beta1) * g;
+    s = cfg.beta2 * s + (1.0 - cfg.beta2) * g * g;
+    x -= cfg.lr[var] * (m / b1t) / (sqrt(s / b2t) + cfg.eps);
+    vars.m[var] = m;
+    vars.v[var] = s;
+    if (var == 0) {
+        x         = fmax(x, 1e-3);
+        vars.V    = x;
+        vars.step = step;
+        fit_derive_V(vars, x, rg.g);
+    } else if (var == 1) {
+        vars.theta = x;
+        fit_derive_theta(vars, x);
+    } else {
+        x      = fmax(x, 1e-6);
+        vars.A = x;
+        fit_derive_A(vars, x);
+    }
+}
+
+// The same with a quasi-Newton step, by thread 0, which loads the member's
+// variables before the partial sums.
+__global__ __launch_bounds__(kFitReduceThreads) void k_fit_reduce_qn(const FitRange* __restrict__ ranges,
+                                                                     FitVars* __restrict__ all_vars,
+                                                                     const float4* __restrict__ parts, QnCfg cfg)
+{
+    __shared__ double red[kFitReduceThreads / 64][4];
+    const FitRange rg   = ranges[blockIdx.x];
+    FitVars&       vars = all_vars[blockIdx.x];
+    FitVars        v;  // all but Adam's moments
+    if (threadIdx.x == 0) {
+        v.V = vars.V, v.theta = vars.theta, v.A = vars.A;
+        v.qn = vars.qn, v.qk = vars.qk, v.qL = vars.qL, v.qr = vars.qr;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sum[j] += red[4 * w + j];
-    const double L = sum[0] / ((double)m.K * (double)m.N * (double)m.N);
-    if (mode == kFitLoss) {
-        m.vars->loss = L;
-        return;
+        for (int i = 0; i < 3; ++i) v.qz[i] = vars.qz[i], v.qg[i] = vars.qg[i];
+#pragma unroll
+        for (int i = 0; i < 6; ++i) v.qH[i] = vars.qH[i];
     }
-    const double g[3] = {sum[1], sum[2], sum[3]};
-    v.loss = L;
-    for (int i = 0; i < 3; ++i) v.grad[i] = g[i];
-    if (mode == kFitQn) {
-        qn_step(v, L, g, qcfg);
-    } else if (mode == kFitAdam) {
-        v.step += 1;
-        const double b1t = 1.0 - pow(cfg.beta1, (double)v.step), b2t = 1.0 - pow(cfg.beta2, (double)v.step);
-        double* x[3] = {&v.V, &v.theta, &v.A};
-        for (int i = 0; i < 3; ++i) {
-            v.m[i] = cfg.beta1 * v.m[i] + (1.0 - cfg.beta1) * g[i];
-            v.v[i] = cfg.beta2 * v.v[i] + (1.0 - cfg.beta2) * g[i] * g[i];
-            *x[i] -= cfg.lr[i] * (v.m[i] / b1t) / (sqrt(v.v[i] / b2t) + cfg.eps);
-        }
-        v.V = fmax(v.V, 1e-3);
-        v.A = fmax(v.A, 1e-6);
-    }
-    fit_vars_derive(v, m.g_d);
-    *m.vars = v;
+    const FitSums sum = fit_sums(rg, parts, fit_first_part(rg, parts), red);
+    if (threadIdx.x != 0) return;
+    const double L = sum.loss / rg.knn, g[3] = {sum.dV, sum.dT, sum.dA};
+    qn_step(v, L, g, cfg);
+    vars.loss = L;
+    vars.V = v.V, vars.theta = v.theta, vars.A = v.A;
+    vars.qn = v.qn, vars.qk = v.qk, vars.qL = v.qL, vars.qr = v.qr;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) vars.grad[i] = g[i], vars.qz[i] = v.qz[i], vars.qg[i] = v.qg[i];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) vars.qH[i] = v.qH[i];
+    fit_derive_V(vars, v.V, rg.g);
+    fit_derive_theta(vars, v.theta);
+    fit_derive_A(vars, v.A);
 }
 
 // The phase table of a member with equally spaced times: per column item and
@@ -692,13 +772,18 @@ hipError_t launch_fit_xi(const FitMember& m, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_fit(const FitMember* members, int n_members, const int2* cols_items, int n_cols, int mode,
-                      const AdamCfg& adam, const QnCfg& qn, hipStream_t s)
+hipError_t launch_fit(const FitTables& t, int mode, const AdamCfg& adam, const QnCfg& qn, hipStream_t s)
 {
-    if (n_members < 1 || n_cols < 1) return hipErrorInvalidValue;
+    if (t.n_members < 1 || t.n_items < 1) return hipErrorInvalidValue;
     // one launch over the column items: loss and gradient in the spectral domain
-    hipLaunchKernelGGL(k_fit_spectral, dim3(n_cols), dim3(kFitColsThreads), 0, s, members, cols_items, mode);
-    hipLaunchKernelGGL(k_fit_reduce, dim3(n_members), dim3(kFitReduceThreads), 0, s, members, mode, adam, qn);
+    hipLaunchKernelGGL(k_fit_spectral, dim3(t.n_items), dim3(kFitColsThreads), 0, s, t.members, t.vars, t.items, t.parts,
+                       mode);
+    if (mode == kFitQn)
+        hipLaunchKernelGGL(k_fit_reduce_qn, dim3(t.n_members), dim3(kFitReduceThreads), 0, s, t.ranges, t.vars,
+                           t.parts, qn);
+    else
+        hipLaunchKernelGGL(k_fit_reduce, dim3(t.n_members), dim3(kFitReduceThreads), 0, s, t.ranges, t.vars, t.parts,
+                           mode, adam);
     return hipGetLastError();
 }
 
