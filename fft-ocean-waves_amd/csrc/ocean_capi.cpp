@@ -636,11 +636,19 @@ int fit_run(ocn_fit* f, int mode, const ocn::AdamCfg& adam, const ocn::QnCfg& qn
 {
     if (!f) return fail(OCN_EINVAL, "fit is NULL");
     hipError_t e = hipSetDevice(f->device);
-    for (size_t i = 0; e == hipSuccess && i < f->members.size(); ++i)
-        if (f->targets_dirty[i]) {
-            e = ocn::launch_fit_targets(f->members[i], (hipStream_t)stream);
-            if (e == hipSuccess) f->targets_dirty[i] = 0;
+    // runs of neighbouring members of one size whose targets changed
+    const size_t n = f->members.size();
+    for (size_t i = 0; e == hipSuccess && i < n;) {
+        if (!f->targets_dirty[i]) {
+            ++i;
+            continue;
         }
+        size_t end = i + 1;
+        while (end < n && f->targets_dirty[end] && f->members[end].N == f->members[i].N) ++end;
+        e = ocn::launch_fit_targets(f->d_members, (int)i, (int)(end - i), f->members[i].N, f->K, (hipStream_t)stream);
+        if (e == hipSuccess) std::fill(f->targets_dirty.begin() + i, f->targets_dirty.begin() + end, 0);
+        i = end;
+    }
     if (e == hipSuccess)
         e = ocn::launch_fit({f->d_members, f->d_vars, f->d_ranges, f->d_cols, f->d_parts, (int)f->members.size(),
                              f->n_cols},
@@ -1609,7 +1617,7 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
     int        rc = OCN_OK;
     hipError_t e  = hipGetDevice(&f->device);
     if (e != hipSuccess) rc = hip_fail(e, "hipGetDevice");
-    // Per member, 256-byte aligned: xi 16, scratch 8, targets 4 K, dL/dh0 16 bytes per texel,
+    // Per member, 256-byte aligned: xi 16, targets 4 K, dL/dh0 16 bytes per texel,
     // the targets' spectra T^ (8 bytes per frame and texel pair of the half plane), with equally spaced
     // times and split strips the phase table (16 bytes per texel pair of the half plane), the noise coefficients (16 bytes
     // per texel pair of the half plane) and the unit noise of the edge pairs (32 bytes each).
@@ -1631,7 +1639,7 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
     auto   phase_bytes = [&](int N) { return phase_table ? al(sizeof(float4) * ocn::fit_phase_entries(N)) : 0; };
     auto   bytes = [&](int N) {
         const size_t nn = (size_t)N * N;
-        return al(nn * 16) + al(nn * 8) + al(nn * 4 * K) + al(nn * 16) +
+        return al(nn * 16) + al(nn * 4 * K) + al(nn * 16) +
                al(sizeof(float2) * K * ocn::fit_phase_entries(N)) + phase_bytes(N) +
                al(sizeof(float4) * ocn::fit_phase_entries(N)) + al(2 * sizeof(float4) * ocn::fit_edge_pairs(N));
     };
@@ -1669,7 +1677,6 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
             m.uniform = uniform_times ? 1 : 0;
             m.dt_rev  = uniform_dt / (2.0 * kPi);
             m.xi        = reinterpret_cast<const float4*>(q), q += al(nn * 16);
-            m.scratch   = reinterpret_cast<float2*>(q), q += al(nn * 8);
             m.targets   = reinterpret_cast<const float*>(q), q += al(nn * 4 * K);
             m.grad_h0   = reinterpret_cast<float4*>(q), q += al(nn * 16);
             m.row_parts   = row_parts;

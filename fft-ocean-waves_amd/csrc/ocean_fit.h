@@ -113,7 +113,6 @@ struct FitMember {
     const float4* phase;
     const float2* tw8;      // Stockham twiddles (N, 8) and (N, 16)
     const float2* tw16;
-    float2* scratch;        // N*N: the row transforms of a target frame (launch_fit_targets)
     const float* targets;   // K * N*N
     // Per target frame k, the sign-shifted 2-D DFT of the targets,
     // T^_k(n) = sum_x T_k(x) e^{-2 pi i n.x / N} over centred wave numbers n,
@@ -142,8 +141,9 @@ __host__ __device__ inline size_t fit_phase_entries(int N) { return (size_t)fit_
 enum FitMode { kFitLoss = 0, kFitGrad = 1, kFitAdam = 2, kFitQn = 3 };
 
 hipError_t launch_fit_xi(const FitMember& m, hipStream_t s);
-// T^ of every target frame of member m (m.scratch holds the row transforms).
-hipError_t launch_fit_targets(const FitMember& m, hipStream_t s);
+// T^ of every target frame of members first .. first + count - 1 of the device
+// table, all of size N.
+hipError_t launch_fit_targets(const FitMember* members, int first, int count, int N, int K, hipStream_t s);
 // Fills m.pq and m.edge from m.xi.
 hipError_t launch_fit_pq(const FitMember& m, hipStream_t s);
 // Fills m.phase (a member with equally spaced times) from its constants.

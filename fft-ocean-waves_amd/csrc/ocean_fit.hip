@@ -345,49 +345,6 @@ __device__ __forceinline__ float4 fit_spectral(const FitMember& m, const FitVars
     return make_float4(lsum, dV, dT, dA);
 }
 
-// T^ of one target frame, rows: R(t, y) = sum_x (-1)^(x+y) T(x, y) e^{-2 pi i t x / N}
-// (the conjugate of the inverse transform of the real input), one row per
-// block of N/8 threads; R in the member's Z buffer.
-template <int N>
-__device__ __forceinline__ void fit_targets_row(const float* __restrict__ tgt, float2* __restrict__ R,
-                                                const float2* __restrict__ tw8, float2* lds)
-{
-    constexpr int E = 8, T = N / E;
-    using Sync = typename std::conditional<(T <= 64), WaveSync, BlockSync>::type;
-    const int y = blockIdx.x, j = threadIdx.x;
-    float2    v[E];
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-        const int x = j + r * T;
-        const float t = tgt[(size_t)y * N + x];
-        v[r] = make_float2(((x + y) & 1) ? -t : t, 0.0f);
-    }
-    fft_inverse<N, E>(v, j, lds, tw8, Sync{});
-#pragma unroll
-    for (int r = 0; r < E; ++r) R[(size_t)y * N + j + r * T] = make_float2(v[r].x, -v[r].y);
-}
-
-// ... and columns t = 0..N/2 of R: T^(t, s) = sum_y R(t, y) e^{-2 pi i s y / N},
-// stored at the half-plane entries (strip t / C, c = t % C, row s).
-template <int N>
-__device__ __forceinline__ void fit_targets_col(const float2* __restrict__ R, float2* __restrict__ that,
-                                                const float2* __restrict__ tw8, float2* lds)
-{
-    constexpr int E = 8, T = N / E, C = fit_cols_per_block(N);
-    using Sync = typename std::conditional<(T <= 64), WaveSync, BlockSync>::type;
-    const int t = blockIdx.x, j = threadIdx.x;  // t <= N/2
-    float2    v[E];
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-        const float2 q = R[(size_t)(j + r * T) * N + t];
-        v[r] = make_float2(q.x, -q.y);
-    }
-    fft_inverse<N, E>(v, j, lds, tw8, Sync{});
-    const size_t col = (size_t)(t / C) * (N * C) + t % C;
-#pragma unroll
-    for (int r = 0; r < E; ++r) that[col + (size_t)(j + r * T) * C] = make_float2(v[r].x, -v[r].y);
-}
-
 }  // namespace
 
 template <int N, int R>
@@ -430,20 +387,72 @@ __global__ __launch_bounds__(kFitColsThreads) void k_fit_spectral(const FitMembe
     if (threadIdx.x == 0) parts[idx] = s;
 }
 
+// T^ of every frame of members first, first + 1, ... (blockIdx.z; all of size N),
+// rows: R(t, y) = sum_x (-1)^(x+y) T(x, y) e^{-2 pi i t x / N} for t <= N/2, the
+// conjugate of the inverse transform of the real input.  Rows 2q and 2q + 1 share
+// one transform (T = N/8 threads), as its real and imaginary parts.  R goes where
+// T^ will stand (that's layout, a column down a strip), so no other buffer is
+// needed and the frames and members of a call run side by side: two launches in
+// place of two per frame and member (N = 512, K = 8: 68 -> 18 us).
 template <int N>
-__global__ __launch_bounds__(N / 8) void k_fit_targets_rows(const float* __restrict__ tgt, float2* __restrict__ R,
-                                                            const float2* __restrict__ tw8)
+constexpr int fit_targets_threads() { return N / 8 < 64 ? 64 : N / 8; }
+template <int N>
+__global__ __launch_bounds__(fit_targets_threads<N>()) void k_fit_targets_rows(const FitMember* __restrict__ members,
+                                                                              int first)
 {
-    __shared__ float2 lds[lds_len(N)];
-    fit_targets_row<N>(tgt, R, tw8, lds);
+    constexpr int E = 8, T = N / E, GPB = fit_targets_threads<N>() / T, C = fit_cols_per_block(N);
+    using Sync = typename std::conditional<(T <= 64), WaveSync, BlockSync>::type;
+    __shared__ float2 lds[GPB * lds_len(N)];
+    const FitMember& m = members[first + blockIdx.z];
+    const int    g = threadIdx.x / T, j = threadIdx.x % T, y = 2 * (blockIdx.x * GPB + g);
+    const float* a = m.targets + ((size_t)blockIdx.y * N + y) * N;
+    float2*      R = m.that + blockIdx.y * fit_phase_entries(N);
+    float2*      buf = lds + g * lds_len(N);
+    float2       v[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int x = j + r * T;  // y is even: row y takes the sign (-1)^x, row y + 1 the other
+        v[r] = (x & 1) ? make_float2(-a[x], a[N + x]) : make_float2(a[x], -a[N + x]);
+    }
+    fft_inverse<N, E>(v, j, buf, m.tw8, Sync{});
+    Sync{}();
+#pragma unroll
+    for (int r = 0; r < E; ++r) buf[lds_pad(j + r * T)] = v[r];
+    Sync{}();
+    // entry k: strip k / 2C, row y + k % 2C / C, column c = k % C: runs of 2C entries
+    for (int k = j; k < 2 * C * (N / 2 / C + 1); k += T) {
+        const int strip = k / (2 * C), odd = k % (2 * C) / C, t = strip * C + k % C;
+        if (t > N / 2) continue;
+        const float2 p = buf[lds_pad(t)], q = buf[lds_pad((N - t) & (N - 1))];
+        R[((size_t)strip * N + y) * C + k % (2 * C)] = odd ? make_float2(0.5f * (p.y + q.y), 0.5f * (p.x - q.x))
+                                                           : make_float2(0.5f * (p.x + q.x), 0.5f * (q.y - p.y));
+    }
 }
 
+// ... and columns t = 0..N/2 of R in place: T^(t, s) = sum_y R(t, y) e^{-2 pi i s y / N}
+// at (strip t / C, row s, c = t % C).  Block: a strip, a group of N/8 threads per
+// column.
 template <int N>
-__global__ __launch_bounds__(N / 8) void k_fit_targets_cols(const float2* __restrict__ R, float2* __restrict__ that,
-                                                            const float2* __restrict__ tw8)
+__global__ __launch_bounds__(kFitColsWidth / 8) void k_fit_targets_cols(const FitMember* __restrict__ members,
+                                                                       int first)
 {
-    __shared__ float2 lds[lds_len(N)];
-    fit_targets_col<N>(R, that, tw8, lds);
+    constexpr int E = 8, T = N / E, C = fit_cols_per_block(N);
+    using Sync = typename std::conditional<(T <= 64), WaveSync, BlockSync>::type;
+    static_assert(T <= 64 || C == 1, "block barriers need every thread active");
+    __shared__ float2 lds[C * lds_len(N)];
+    const FitMember& m = members[first + blockIdx.z];
+    const int g = threadIdx.x / T, j = threadIdx.x % T, strip = blockIdx.x;
+    if (strip * C + g > N / 2) return;  // past the half plane (the last strip; whole group)
+    float2* R = m.that + blockIdx.y * fit_phase_entries(N) + (size_t)strip * (N * C) + g;
+    float2  v[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const float2 q = R[(size_t)(j + r * T) * C];
+        v[r] = make_float2(q.x, -q.y);
+    }
+    fft_inverse<N, E>(v, j, lds + g * lds_len(N), m.tw8, Sync{});
+#pragma unroll
+    for (int r = 0; r < E; ++r) R[(size_t)(j + r * T) * C] = make_float2(v[r].x, -v[r].y);
 }
 
 __global__ __launch_bounds__(256) void k_fit_xi(float4* __restrict__ xi, int N, uint32_t key0, uint32_t key1,
@@ -746,20 +755,19 @@ hipError_t launch_fit_pq(const FitMember& m, hipStream_t s)
 }
 
 template <int N>
-static hipError_t launch_fit_targets_n(const FitMember& m, hipStream_t s)
+static hipError_t launch_fit_targets_n(const FitMember* members, int first, int count, int K, hipStream_t s)
 {
-    const size_t nn = (size_t)N * N, ne = fit_phase_entries(N);
-    for (int f = 0; f < m.K; ++f) {
-        hipLaunchKernelGGL(k_fit_targets_rows<N>, dim3(N), dim3(N / 8), 0, s, m.targets + f * nn, m.scratch, m.tw8);
-        hipLaunchKernelGGL(k_fit_targets_cols<N>, dim3(N / 2 + 1), dim3(N / 8), 0, s, m.scratch, m.that + f * ne, m.tw8);
-    }
+    constexpr int NB = fit_targets_threads<N>(), pairs = NB / (N / 8);
+    hipLaunchKernelGGL(k_fit_targets_rows<N>, dim3(N / 2 / pairs, K, count), dim3(NB), 0, s, members, first);
+    hipLaunchKernelGGL(k_fit_targets_cols<N>, dim3(fit_cols_items_per_member(N), K, count), dim3(kFitColsWidth / 8), 0,
+                       s, members, first);
     return hipGetLastError();
 }
 
-hipError_t launch_fit_targets(const FitMember& m, hipStream_t s)
+hipError_t launch_fit_targets(const FitMember* members, int first, int count, int N, int K, hipStream_t s)
 {
-#define OCN_CALL(n) return launch_fit_targets_n<n>(m, s)
-    OCN_FIT_SWITCH(m.N, OCN_CALL)
+#define OCN_CALL(n) return launch_fit_targets_n<n>(members, first, count, K, s)
+    OCN_FIT_SWITCH(N, OCN_CALL)
 #undef OCN_CALL
     return hipErrorInvalidValue;
 }
