@@ -592,6 +592,8 @@ struct ocn_fit {
     ocn::FitVars*                         d_vars    = nullptr;
     ocn::FitRange*                        d_ranges  = nullptr;
     float4*                               d_parts   = nullptr;
+    ocn::FitReport*                       reports   = nullptr;  // pinned host memory (host address)
+    ocn::FitReport*                       d_reports = nullptr;  // its device address
     int2*                                 d_cols    = nullptr;
     int                                   n_cols    = 0;
     char*                                 pool      = nullptr;
@@ -609,6 +611,7 @@ void fit_free(ocn_fit* f)
     void* ptrs[] = {f->d_members, f->d_vars, f->d_ranges, f->d_parts, f->d_cols, f->pool};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
+    if (f->reports) (void)hipHostFree(f->reports);
     for (auto& kv : f->tw)
         for (float2* q : kv.second)
             if (q) (void)hipFree(q);
@@ -632,6 +635,11 @@ ocn::FitVars initial_vars(const ocn_params& p)
     return v;
 }
 
+void fit_report(ocn_fit* f, int member, const ocn::FitVars& v)
+{
+    f->reports[member] = {{v.V, v.theta, v.A}, {v.grad[0], v.grad[1], v.grad[2]}, v.loss, 0.0};
+}
+
 int fit_run(ocn_fit* f, int mode, const ocn::AdamCfg& adam, const ocn::QnCfg& qn, void* stream)
 {
     if (!f) return fail(OCN_EINVAL, "fit is NULL");
@@ -650,8 +658,8 @@ int fit_run(ocn_fit* f, int mode, const ocn::AdamCfg& adam, const ocn::QnCfg& qn
         i = end;
     }
     if (e == hipSuccess)
-        e = ocn::launch_fit({f->d_members, f->d_vars, f->d_ranges, f->d_cols, f->d_parts, (int)f->members.size(),
-                             f->n_cols},
+        e = ocn::launch_fit({f->d_members, f->d_vars, f->d_ranges, f->d_cols, f->d_parts, f->d_reports,
+                             (int)f->members.size(), f->n_cols},
                             mode, adam, qn, (hipStream_t)stream);
     return e == hipSuccess ? OCN_OK : hip_fail(e, "fit launch");
 }
@@ -1655,6 +1663,12 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
     }
     if (!rc) rc = dalloc(&f->d_vars, (size_t)count, "fit variables");
     if (!rc) {
+        e = hipHostMalloc((void**)&f->reports, sizeof(ocn::FitReport) * count, hipHostMallocMapped | hipHostMallocCoherent);
+        if (e != hipSuccess) f->reports = nullptr, rc = fail(OCN_ENOMEM, "hipHostMalloc(fit reports): %s", hipGetErrorString(e));
+        else if ((e = hipHostGetDevicePointer((void**)&f->d_reports, f->reports, 0)) != hipSuccess)
+            rc = hip_fail(e, "hipHostGetDevicePointer(fit reports)");
+    }
+    if (!rc) {
         std::vector<ocn::FitVars>  vars;
         std::vector<ocn::FitRange> ranges;
         char*                      q = f->pool;
@@ -1692,6 +1706,7 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
             m.cascade_id = p.cascade_id;
             f->members.push_back(m);
             vars.push_back(initial_vars(p));
+            fit_report(f, i, vars.back());
             const int blocks = ocn::fit_cols_items_per_member(p.N) * row_parts;  // one partial each
             ranges.push_back({(int)cols.size(), blocks, (double)K * (double)nn, p.gravity});
             for (int k = 0; k < blocks; ++k) cols.push_back(make_int2(i, k));
@@ -1783,6 +1798,7 @@ int ocn_fit_set_vars(ocn_fit* f, int member, const double vars[3])
     hipError_t e = hipSetDevice(f->device);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e == hipSuccess) e = hipMemcpy(f->d_vars + member, &v, sizeof(v), hipMemcpyHostToDevice);
+    if (e == hipSuccess) fit_report(f, member, v);
     return e == hipSuccess ? OCN_OK : hip_fail(e, "hipMemcpy(fit variables)");
 }
 
@@ -1834,19 +1850,17 @@ int ocn_fit_get(ocn_fit* f, int member, double vars[3], double grad[3], double* 
 {
     int rc = check_fit(f, member);
     if (rc) return rc;
-    ocn::FitVars v{};
-    hipError_t   e = hipSetDevice(f->device);
+    hipError_t e = hipSetDevice(f->device);
     if (e == hipSuccess) e = hipStreamSynchronize((hipStream_t)stream);
-    if (e == hipSuccess) e = hipMemcpy(&v, f->d_vars + member, sizeof(v), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return hip_fail(e, "hipMemcpy(fit variables)");
-    if (vars) {
-        vars[0] = v.V;
-        vars[1] = v.theta;
-        vars[2] = v.A;
+    // ... and, through the null stream, work queued on other blocking streams
+    if (e == hipSuccess && stream) e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize(fit)");
+    const volatile ocn::FitReport& r = f->reports[member];
+    for (int i = 0; i < 3; ++i) {
+        if (vars) vars[i] = r.var[i];
+        if (grad) grad[i] = r.grad[i];
     }
-    if (grad)
-        for (int i = 0; i < 3; ++i) grad[i] = v.grad[i];
-    if (loss) *loss = v.loss;
+    if (loss) *loss = r.loss;
     return OCN_OK;
 }
 

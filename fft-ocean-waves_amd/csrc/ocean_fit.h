@@ -137,6 +137,17 @@ __host__ __device__ inline int fit_edge_index(int N, int tx, int ty)
 // float4 entries of a member's phase table
 __host__ __device__ inline size_t fit_phase_entries(int N) { return (size_t)fit_cols_items_per_member(N) * N * fit_cols_per_block(N); }
 
+// What ocn_fit_get hands out of one member, in pinned host memory that the
+// reduction writes besides FitVars (and ocn_fit_set_vars, on the host): a get
+// waits for the stream and reads it, with no copy of its own (22 -> 2.0 us a call;
+// the writes to the host add 0.2-0.4 us to a step).
+struct FitReport {
+    double var[3];   // V, theta, A
+    double grad[3];
+    double loss;
+    double pad_;
+};
+
 // Modes of the fit launch sequence.
 enum FitMode { kFitLoss = 0, kFitGrad = 1, kFitAdam = 2, kFitQn = 3 };
 
@@ -157,6 +168,7 @@ struct FitTables {
     const FitRange*  ranges;
     const int2*      items;
     float4*          parts;
+    FitReport*       reports;
     int              n_members, n_items;
 };
 hipError_t launch_fit(const FitTables& t, int mode, const AdamCfg& adam, const QnCfg& qn, hipStream_t s);

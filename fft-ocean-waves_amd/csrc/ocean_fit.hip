@@ -603,13 +603,15 @@ __device__ __forceinline__ float4 fit_first_part(const FitRange& rg, const float
 
 __global__ __launch_bounds__(kFitReduceThreads) void k_fit_reduce(const FitRange* __restrict__ ranges,
                                                                   FitVars* __restrict__ all_vars,
-                                                                  const float4* __restrict__ parts, int mode,
+                                                                  const float4* __restrict__ parts,
+                                                                  FitReport* __restrict__ reports, int mode,
                                                                   AdamCfg cfg)
 {
     static_assert(kFitReduceThreads == 256, "one wave per variable and one for the loss");
     __shared__ double red[kFitReduceThreads / 64][4];
     const FitRange rg   = ranges[blockIdx.x];
     FitVars&       vars = all_vars[blockIdx.x];
+    FitReport&     rep  = reports[blockIdx.x];
     const int      wave = threadIdx.x / 64, var = wave < 3 ? wave : 0;
     const bool     lead = (threadIdx.x & 63) == 0;
     const float4   p    = fit_first_part(rg, parts);
@@ -627,18 +629,20 @@ __global__ __launch_bounds__(kFitReduceThreads) void k_fit_reduce(const FitRange
     }
     const FitSums sum = fit_sums(rg, parts, p, red);
     if (!lead) return;
-    if (wave == 3) vars.loss = sum.loss / rg.knn;
+    if (wave == 3) rep.loss = vars.loss = sum.loss / rg.knn;
     if (wave == 3 || mode == kFitLoss) return;
     const double g = var == 0 ? sum.dV : var == 1 ? sum.dT : sum.dA;
-    vars.grad[var] = g;
+    rep.grad[var] = vars.grad[var] = g;
     if (mode != kFitAdam) return;
     m = cfg.beta1 * m + (1.0 - cfg.beta1) * g;
     s = cfg.beta2 * s + (1.0 - cfg.beta2) * g * g;
     x -= cfg.lr[var] * (m / b1t) / (sqrt(s / b2t) + cfg.eps);
     vars.m[var] = m;
     vars.v[var] = s;
+    if (var == 0) x = fmax(x, 1e-3);
+    if (var == 2) x = fmax(x, 1e-6);
+    rep.var[var] = x;
     if (var == 0) {
-        x         = fmax(x, 1e-3);
         vars.V    = x;
         vars.step = step;
         fit_derive_V(vars, x, rg.g);
@@ -646,7 +650,6 @@ __global__ __launch_bounds__(kFitReduceThreads) void k_fit_reduce(const FitRange
         vars.theta = x;
         fit_derive_theta(vars, x);
     } else {
-        x      = fmax(x, 1e-6);
         vars.A = x;
         fit_derive_A(vars, x);
     }
@@ -656,7 +659,8 @@ __global__ __launch_bounds__(kFitReduceThreads) void k_fit_reduce(const FitRange
 // variables before the partial sums.
 __global__ __launch_bounds__(kFitReduceThreads) void k_fit_reduce_qn(const FitRange* __restrict__ ranges,
                                                                      FitVars* __restrict__ all_vars,
-                                                                     const float4* __restrict__ parts, QnCfg cfg)
+                                                                     const float4* __restrict__ parts,
+                                                                     FitReport* __restrict__ reports, QnCfg cfg)
 {
     __shared__ double red[kFitReduceThreads / 64][4];
     const FitRange rg   = ranges[blockIdx.x];
@@ -674,11 +678,13 @@ __global__ __launch_bounds__(kFitReduceThreads) void k_fit_reduce_qn(const FitRa
     if (threadIdx.x != 0) return;
     const double L = sum.loss / rg.knn, g[3] = {sum.dV, sum.dT, sum.dA};
     qn_step(v, L, g, cfg);
-    vars.loss = L;
+    FitReport& rep = reports[blockIdx.x];
+    rep.loss = vars.loss = L;
+    rep.var[0] = v.V, rep.var[1] = v.theta, rep.var[2] = v.A;
     vars.V = v.V, vars.theta = v.theta, vars.A = v.A;
     vars.qn = v.qn, vars.qk = v.qk, vars.qL = v.qL, vars.qr = v.qr;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) vars.grad[i] = g[i], vars.qz[i] = v.qz[i], vars.qg[i] = v.qg[i];
+    for (int i = 0; i < 3; ++i) rep.grad[i] = vars.grad[i] = g[i], vars.qz[i] = v.qz[i], vars.qg[i] = v.qg[i];
 #pragma unroll
     for (int i = 0; i < 6; ++i) vars.qH[i] = v.qH[i];
     fit_derive_V(vars, v.V, rg.g);
@@ -788,10 +794,10 @@ hipError_t launch_fit(const FitTables& t, int mode, const AdamCfg& adam, const Q
                        mode);
     if (mode == kFitQn)
         hipLaunchKernelGGL(k_fit_reduce_qn, dim3(t.n_members), dim3(kFitReduceThreads), 0, s, t.ranges, t.vars,
-                           t.parts, qn);
+                           t.parts, t.reports, qn);
     else
         hipLaunchKernelGGL(k_fit_reduce, dim3(t.n_members), dim3(kFitReduceThreads), 0, s, t.ranges, t.vars, t.parts,
-                           mode, adam);
+                           t.reports, mode, adam);
     return hipGetLastError();
 }
 
