@@ -22,10 +22,34 @@ constexpr int kBatchWideRowsThreads = kBatchWideN / 8;
 
 // Row-pass radix and default band height per N: radix 8 keeps the fused row
 // kernel at two waves per SIMD; short bands at small N keep a row block busy.
-// The band height of each member can be changed (ocn_batch_set_schedule,
-// ocn_batch_autotune) among the heights batch_band_valid accepts.
+// These suit many members; a batch whose walks would leave the GPU half empty
+// takes shorter bands (batch_band_shift).  The band height of each member can be
+// changed (ocn_batch_set_schedule, ocn_batch_autotune) among the heights
+// batch_band_valid accepts.
 __host__ __device__ constexpr int batch_rows_radix(int) { return 8; }
 __host__ __device__ constexpr int batch_rows_band(int N) { return N <= 64 ? 2 : N <= 512 ? 8 : N <= 1024 ? 16 : 32; }
+
+// How often a batch halves its members' default bands (never below 2 rows): until
+// its row walks, of N/8 threads each, make 1024 waves, half of the two waves per
+// SIMD that are resident.  A walk's rows follow one another, so few long walks
+// leave a small batch waiting (whole frames, us, default bands -> these): one ocean
+// of cascades 256 + 512 + 1024 105 -> 48, four of them 119 -> 91, 10 oceans of N = 256
+// 49 -> 32, two of 2048 202 -> 141.  At 2048 waves 100 oceans of N = 256 would halve too
+// and lose (94 -> 105).  rows_of(i), i < count: the member's N.
+template <class RowsOf>
+inline int batch_band_shift(int count, RowsOf rows_of)
+{
+    int shift = 0;
+    for (; shift < 4; ++shift) {
+        double waves = 0.0;
+        for (int i = 0; i < count; ++i) {
+            const int N = rows_of(i), R = batch_rows_band(N) >> shift;
+            waves += (double)N / (R < 2 ? 2 : R) * N / 512.0;
+        }
+        if (waves >= 1024.0) break;
+    }
+    return shift;
+}
 
 // Device-side descriptor of one batch member (one ocean cascade, one frame).
 struct BatchMember {

@@ -1219,8 +1219,8 @@ int ocn_batch_create(const ocn_params* params, int count, ocn_batch** out)
         if (!(rc = upload_table(&t[0], stockham_twiddles(p.N, 8)))) rc = upload_table(&t[1], stockham_twiddles(p.N, 16));
     }
     if (!rc) {
-        char*             q = b->pool;
-        std::vector<int2> cols;
+        char*     q     = b->pool;
+        const int shift = ocn::batch_band_shift(count, [&](int i) { return b->params[i].N; });
         for (int i = 0; i < count; ++i) {
             const ocn_params& p  = b->params[i];
             const size_t      nn = (size_t)p.N * p.N;
@@ -1240,7 +1240,7 @@ int ocn_batch_create(const ocn_params* params, int count, ocn_batch** out)
             m.lambda  = (float)p.choppiness;
             m.inv2d   = (float)((double)p.N / (2.0 * p.L));
             m.dscale  = (float)p.displacement_scale;
-            m.band    = ocn::batch_rows_band(p.N);
+            m.band    = std::max(2, ocn::batch_rows_band(p.N) >> shift);
             m.cols    = ocn::batch_cols_per_block(p.N);
             b->members.push_back(m);
         }
