@@ -442,14 +442,21 @@ __global__ __launch_bounds__((W * par_groups<N, E, R, BIL>() * (N / E))) void k_
 // of the render displacement (-l Dx, -l Dz) (grid_tes.glsl:60-62), by periodic
 // central differences with spacing L/N.
 //
-// Tiled: a block owns a 64 x 16 texel tile and first stages height/dx/dz for
+// Tiled: a block owns a 64 x H texel tile and first stages height/dx/dz for
 // the tile plus a 2-texel periodic halo in LDS with coalesced row loads (the
 // bilinear taps reach two texels down/left, the others one), then every tap
-// comes from LDS.  1-D grid of (N/64) x (N/16) x frames blocks; frame f reads
+// comes from LDS.  1-D grid of (N/64) x (N/H) x frames blocks; frame f reads
 // and writes at offset f*stride.  After the XCD remap, tiles of neighbouring
 // rows run on the same XCD, so the halo rows are L2 hits.
-constexpr int kNrmW = 64, kNrmH = 16, kNrmHalo = 2;
-constexpr int kNrmLW = kNrmW + 2 * kNrmHalo, kNrmLH = kNrmH + 2 * kNrmHalo;
+constexpr int kNrmW = 64, kNrmHalo = 2;
+constexpr int kNrmLW = kNrmW + 2 * kNrmHalo;
+// H = 16 reads 1.25 rows per row kept and is what memory wants where the grid
+// fills the chip (N = 4096: 131 us, H = 4 196; N = 2048: 24 against 32).  A grid
+// below four blocks per CU waits for the chain of one block instead, seven
+// staging loads and four texels in each thread; H = 4 cuts it to three and one:
+// back to back N = 64 5.7 -> 3.2 us, N = 256 6.0 -> 3.4, N = 512 6.5 -> 4.8 (H = 8:
+// 4.1, 4.3, 5.2).  N = 1024 sits at four blocks: 9.3 with 16, 10.5 with 4.
+constexpr int normals_tile_rows(int N, int nframes) { return (N / kNrmW) * (N / 16) * nframes >= 1024 ? 16 : 4; }
 
 // texture() of the staged tile under NEAREST + REPEAT (s[y][x], halo-offset
 // coordinates) or LINEAR + REPEAT at a texel corner: 2x2 box over (x-1..x, y-1..y).
@@ -458,14 +465,16 @@ __device__ __forceinline__ float stap(const float (*s)[kNrmLW], int y, int x, in
     return mode ? 0.25f * (s[y - 1][x - 1] + s[y - 1][x] + s[y][x - 1] + s[y][x]) : s[y][x];
 }
 
+template <int H>
 __global__ __launch_bounds__(256) void k_normals(const float* __restrict__ height, const float* __restrict__ dx,
                                                  const float* __restrict__ dz, float4* __restrict__ normals,
                                                  float* __restrict__ jac, int N, int mode, float lambda,
                                                  float inv2d, size_t stride, float4* __restrict__ disp,
                                                  float4* __restrict__ rnorm, float dscale)
 {
-    __shared__ float sh[kNrmLH][kNrmLW], sx[kNrmLH][kNrmLW], sz[kNrmLH][kNrmLW];
-    const int tiles_x = N / kNrmW, tiles_y = N / kNrmH;
+    constexpr int LH = H + 2 * kNrmHalo;
+    __shared__ float sh[LH][kNrmLW], sx[LH][kNrmLW], sz[LH][kNrmLW];
+    const int tiles_x = N / kNrmW, tiles_y = N / H;
     const int L  = xcd_logical(blockIdx.x, gridDim.x);
     const int bx = L % tiles_x;
     const int by = (L / tiles_x) % tiles_y;
@@ -479,8 +488,8 @@ __global__ __launch_bounds__(256) void k_normals(const float* __restrict__ heigh
     if (disp) disp += fo;
     if (rnorm) rnorm += fo;
     const bool need_h = normals || disp || rnorm, need_xz = jac || disp || rnorm;
-    const int x0 = bx * kNrmW, y0 = by * kNrmH;
-    for (int k = threadIdx.x; k < kNrmLH * kNrmLW; k += 256) {
+    const int x0 = bx * kNrmW, y0 = by * H;
+    for (int k = threadIdx.x; k < LH * kNrmLW; k += 256) {
         const int ly = k / kNrmLW, lx = k % kNrmLW;
         const size_t gi = (size_t)((y0 + ly - kNrmHalo) & (N - 1)) * N + ((x0 + lx - kNrmHalo) & (N - 1));
         if (need_h) sh[ly][lx] = height[gi];
@@ -492,7 +501,7 @@ __global__ __launch_bounds__(256) void k_normals(const float* __restrict__ heigh
     __syncthreads();
     const int cx = (threadIdx.x & 63) + kNrmHalo;
 #pragma unroll
-    for (int k = 0; k < kNrmH / 4; ++k) {
+    for (int k = 0; k < H / 4; ++k) {
         const int ly = (threadIdx.x >> 6) + 4 * k;
         const int cy = ly + kNrmHalo;
         const size_t i = (size_t)(y0 + ly) * N + x0 + (threadIdx.x & 63);
@@ -526,6 +535,15 @@ __global__ __launch_bounds__(256) void k_normals(const float* __restrict__ heigh
             }
         }
     }
+}
+
+static void normals_pass(int N, int nframes, const float* height, const float* dx, const float* dz, float4* normals,
+                         float* jac, int mode, float lambda, float inv2d, size_t stride, float4* disp, float4* rnorm,
+                         float dscale, hipStream_t s)
+{
+    const int H = normals_tile_rows(N, nframes);
+    hipLaunchKernelGGL(H == 16 ? k_normals<16> : k_normals<4>, dim3((N / kNrmW) * (N / H) * nframes), dim3(256), 0, s,
+                       height, dx, dz, normals, jac, N, mode, lambda, inv2d, stride, disp, rnorm, dscale);
 }
 
 // ------------------------------------------------------------------ A5+A6 pass API (general complex input)
@@ -816,9 +834,8 @@ static hipError_t launch_frame_n(const FrameArgs& a, int stages, hipStream_t s)
         if (e != hipSuccess) return e;
     }
     if ((stages & 4) && !fused && (a.normals || a.jacobian || a.disp || a.rnorm)) {
-        hipLaunchKernelGGL(k_normals, dim3((N / kNrmW) * (N / kNrmH) * a.nframes), dim3(256), 0, s, a.height, a.dx, a.dz,
-                           a.normals, a.jacobian, N, a.normal_mode, a.lambda, a.inv2d, a.fb.out_stride, a.disp,
-                           a.rnorm, a.dscale);
+        normals_pass(N, a.nframes, a.height, a.dx, a.dz, a.normals, a.jacobian, a.normal_mode, a.lambda, a.inv2d,
+                     a.fb.out_stride, a.disp, a.rnorm, a.dscale, s);
         e = hipGetLastError();
     }
     return e;
@@ -966,8 +983,7 @@ hipError_t launch_spectrum_t(int N, const float4* h0, float2* hy, float2* hx, fl
 hipError_t launch_normals(int N, const float* height, const float* dx, const float* dz, float4* normals,
                           float* jacobian, int mode, float lambda, float inv2d, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_normals, dim3((N / kNrmW) * (N / kNrmH)), dim3(256), 0, s, height, dx, dz, normals, jacobian, N, mode,
-                       lambda, inv2d, (size_t)0, (float4*)nullptr, (float4*)nullptr, 0.0f);
+    normals_pass(N, 1, height, dx, dz, normals, jacobian, mode, lambda, inv2d, 0, nullptr, nullptr, 0.0f, s);
     return hipGetLastError();
 }
 
