@@ -153,8 +153,9 @@ int frames_class(int nframes)
 // the folds over the block, the shorter chain while a launch has less than
 // about four blocks per CU; beyond that k_cols, which does less work per column
 // in a third of the LDS, is faster.  Both sides of the line (us per frame,
-// whole frames, k_cols_lds / k_cols): N=256, 32 frames 1.02 / 1.05; N=512, 4
-// frames 5.36 / 5.60, 8 frames 5.22 / 4.53; N=1024, 1 frame 25.4 / 25.7, 2
+// whole frames, k_cols_lds / k_cols): N=256, 32 frames 1.04 / 1.08; N=512, 4
+// frames 5.56 / 5.99, 5 frames 5.65 / 5.43 (render export 7.25 / 6.96), 6 frames
+// 5.52 / 4.97, 8 frames 5.22 / 4.53; N=1024, 1 frame 25.4 / 25.7, 2
 // frames 18.9 / 19.5, 4 frames 16.4 / 15.1, 16 frames 11.6 / 11.3.
 std::pair<int, int> default_schedule(int N, int nframes)
 {
@@ -171,7 +172,7 @@ std::pair<int, int> default_schedule(int N, int nframes)
     case 64: cv = 14; rv = batch ? 1 : 8; break;
     case 128: cv = 14; rv = batch ? 2 : 8; break;
     case 256: cv = nframes >= 5 && nframes <= 16 ? 21 : 14; rv = 8; break;
-    case 512: cv = nframes <= 2 ? 14 : nframes <= 6 ? 21 : 12; rv = batch ? 7 : 8; break;
+    case 512: cv = nframes <= 2 ? 14 : nframes <= 4 ? 21 : 12; rv = batch ? 7 : 8; break;
     case 1024:
         cv = !batch ? 13 : nframes <= 2 ? 14 : 9;
         rv = !batch ? 7 : nframes <= 6 ? 7 : nframes <= 9 ? 3 : nframes <= 16 ? 4 : 5;
