@@ -400,13 +400,16 @@ int run_frames(ocn_handle* h, const double* t, int nframes, const ocn_fields* ou
 // Infinity Cache holds beside the spectrum, however many frames were reserved:
 // beyond that the row pass reads them from HBM (us per frame: N=1024 32 frames
 // 13.8, 16 frames 11.2; N=2048 8 frames 61, 4 frames 50; N=4096 4 frames 300, single
-// frames 268; below the line a longer launch is the faster one).
+// frames 268; below the line a longer launch is the faster one).  A single stage
+// keeps the caller's chunks: another stage's call finds every frame of a chunk
+// in its own slot.
 int frames_in_chunks(ocn_handle* h, float2* z1, float2* z2, const double* t_host, int nframes,
                      const ocn_fields* out, int stage, int chunk, hipStream_t s)
 {
     const size_t nn = (size_t)h->p.N * h->p.N;
     int cv, rv, rc;
-    chunk = std::min(chunk, (int)std::max<size_t>(1, ((size_t)1 << 24) / nn));
+    const int both = OCN_STAGE_COLUMNS | OCN_STAGE_ROWS;
+    if ((stage & both) == both) chunk = std::min(chunk, (int)std::max<size_t>(1, ((size_t)1 << 24) / nn));
     for (int f0 = 0; f0 < nframes; f0 += chunk) {
         const int nf = std::min(chunk, nframes - f0);
         pick_schedule(h, nf, &cv, &rv);

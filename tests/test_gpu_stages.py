@@ -1,0 +1,45 @@
+"""The stages of ocn_update_stage called one by one over as many frames as the
+handle reserved, more than one launch of whole frames takes (2^24 texels: 4
+frames at N=2048): the row stage finds every frame's intermediates where the
+column stage left them, so the outputs are those of ocn_update_frames."""
+import numpy as np
+import pytest
+
+import pyocean
+from ocean_testutil import assert_field_close
+
+pytestmark = pytest.mark.gpu
+
+SIZES = {"height": 4, "dx": 4, "dz": 4, "normals": 16, "jacobian": 4}
+
+
+def test_stages_one_by_one_over_more_frames_than_a_launch():
+    N, F = 2048, 5
+    print("stages N=%d frames=%d" % (N, F), flush=True)
+    hip = pyocean.Hip()
+    times = 0.5 + np.arange(F) * 0.25
+    bufs = {k: hip.malloc(F * N * N * b) for k, b in SIZES.items()}
+    fl = pyocean.OcnFields(*[bufs[k] for k in SIZES])
+
+    def slots():
+        hip.sync()
+        return {k: [hip.download(bufs[k] + f * N * N * b, (N, N, 4) if b == 16 else (N, N)) for f in range(F)]
+                for k, b in SIZES.items()}
+
+    try:
+        with pyocean.Ocean(pyocean.make_params(N=N, L=1000.0, seed=4)) as oc:
+            oc.tilde_h0_k()
+            oc.reserve_frames(F)
+            oc.update_frames(times, fl)
+            want = slots()
+            for v, b in zip(bufs.values(), SIZES.values()):
+                hip.upload(v, np.zeros(F * N * N * b // 4, np.float32))
+            oc.update_stage(times, fl, 1)
+            oc.update_stage(times, fl, 2 | 4)
+            got = slots()
+    finally:
+        for v in bufs.values():
+            hip.free(v)
+    for k in SIZES:
+        for f in range(F):
+            assert_field_close("%s f%d" % (k, f), got[k][f], want[k][f])
