@@ -52,11 +52,11 @@ CANON_STAGE = {"k_cols": 40, "k_rows": 36, "k_normals": 20, "k_rows_nrm": 56}
 # launch's column pass wrote stay in the 256 MB Infinity Cache for its row
 # pass as long as they fit there beside h0: 16 N=1024 frames (192 MB) ran at
 # 12.4 us per frame over the 600-frame sequence, against 13.8 in 8-frame and
-# 15.0 in 32-frame launches (384 MB, read back from HBM).  N=2048 runs
-# fastest in 4-frame launches, N=4096 in 8-frame ones, smaller N in 32-frame
-# ones.
+# 15.0 in 32-frame launches (384 MB, read back from HBM).  The library cuts
+# launches to 2^24 texels (4 frames at N=2048, 1 at N=4096); smaller N run
+# fastest in 32-frame ones.
 def launch_frames_for(n):
-    return 16 if n == 1024 else 4 if n == 2048 else 8 if n == 4096 else 32
+    return 16 if n == 1024 else 4 if n == 2048 else 1 if n == 4096 else 32
 
 
 LAUNCH_FRAMES = launch_frames_for(1024)
@@ -65,7 +65,7 @@ LAUNCH_FRAMES = launch_frames_for(1024)
 # (each scaled by what the counter reads for a device-to-device copy of known
 # size: fetch x 2.0, write x 1.0) for this workload, keyed by kernel and the
 # (column, row) schedule it ran under; see
-# profiles/k_rows_nrm_k_cols_lds_n1024_batched_pmc_traffic.md.  Reported only
+# profiles/k_rows_nrm_k_cols_n1024_batched_pmc_traffic.md.  Reported only
 # when the schedule in use matches, otherwise null.
 MEASURED_TRAFFIC = {
     ("k_rows_nrm", 9, 4, 16): 13.5 + 32.1,

@@ -98,7 +98,7 @@ public:
     void tilde_h0_t(double t) { check(ocn_tilde_h0_t(h_, t, stream_)); }
     void butterfly_fft(Field f) { check(ocn_butterfly_fft(h_, static_cast<int>(f), stream_)); }
     void generate_normal_map() { check(ocn_generate_normal_map(h_, stream_)); }
-    // ... or fused (the same outputs in three kernels).
+    // ... or fused (the same outputs in two or three kernels).
     void update(double t) { check(ocn_update(h_, t, stream_)); }
     void update_into(double t, const ocn_fields& out) { check(ocn_update_into(h_, t, &out, stream_)); }
     void update_frames(const std::vector<double>& t, const ocn_fields& out)

@@ -209,7 +209,8 @@ int ocn_generate_normal_map(ocn_handle* h, void* stream);
 /* ---------------------------------------------------------------- fused frame */
 
 /* One frame (main.cpp:240-244): tilde_h0_t, the three butterfly_fft calls and
- * generate_normal_map, fused into three kernels, into the handle's fields. */
+ * generate_normal_map, fused into two kernels (three where the normal map runs
+ * by itself), into the handle's fields. */
 int ocn_update(ocn_handle* h, double t, void* stream);
 
 /* Same into caller buffers (height, dx, dz required; normals, jacobian optional). */
@@ -232,7 +233,9 @@ int ocn_update_stage(ocn_handle* h, const double* t_host, int nframes, const ocn
 /* nframes frames at times t_host[0..nframes) into consecutive output slices:
  * frame f writes out->height + f*N*N, ..., out->normals + f*N*N*4, ...
  * (the per-frame slices of a recorded sequence).  The frames run in launches
- * of at most ocn_frames_reserved() frames each (1 after ocn_create); the call
+ * of at most ocn_frames_reserved() frames each (1 after ocn_create) and 2^24
+ * texels (N = 4096: 1 frame, 2048: 4, 1024: 16, so that a launch's
+ * intermediates stay in the 256 MB Infinity Cache); the call
  * never allocates, so reserve once before the first multi-frame update. */
 int ocn_update_frames(ocn_handle* h, const double* t_host, int nframes, const ocn_fields* out, void* stream);
 
