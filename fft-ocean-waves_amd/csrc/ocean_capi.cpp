@@ -140,6 +140,14 @@ int frames_class(int nframes)
     return nframes <= 1 ? 1 : nframes <= 4 ? 4 : nframes <= 8 ? 8 : nframes <= 16 ? 16 : ocn::kMaxFrames;
 }
 
+// Frames of one launch of whole frames, at most.  Its intermediates are kept to
+// 2^24 texels (201 MB), what the 256 MB Infinity Cache holds beside the spectrum,
+// however many frames were reserved: beyond that the row pass reads them from
+// HBM (us per frame: N=1024 32 frames 13.8, 16 frames 11.2; N=2048 8 frames 61, 4
+// frames 50; N=4096 4 frames 300, single frames 268; below the line a longer
+// launch is the faster one).
+int launch_cap(int N) { return std::min(ocn::kMaxFrames, std::max(1, (1 << 24) / (N * N))); }
+
 // Built-in schedules: the fastest (column variant, row variant) measured on
 // MI355X per N and frames per launch; the autotuner may replace them.  Column
 // variants (kColsVariants): 13, 14 and 21 k_cols_lds with 1, 2 and 4 columns
@@ -396,20 +404,16 @@ int run_frames(ocn_handle* h, const double* t, int nframes, const ocn_fields* ou
 // most `chunk` frames, intermediates at z1 / z2 (room for `chunk` frames).
 // Each launch takes the schedule for its own frame count, so a short last
 // launch gets the short bands that fill the GPU.
-// A launch's intermediates are kept to 2^24 texels (201 MB), what the 256 MB
-// Infinity Cache holds beside the spectrum, however many frames were reserved:
-// beyond that the row pass reads them from HBM (us per frame: N=1024 32 frames
-// 13.8, 16 frames 11.2; N=2048 8 frames 61, 4 frames 50; N=4096 4 frames 300, single
-// frames 268; below the line a longer launch is the faster one).  A single stage
-// keeps the caller's chunks: another stage's call finds every frame of a chunk
-// in its own slot.
+// Whole frames run in launches of at most launch_cap(N); a single stage keeps
+// the caller's chunks, so that another stage's call finds every frame of a
+// chunk in its own slot.
 int frames_in_chunks(ocn_handle* h, float2* z1, float2* z2, const double* t_host, int nframes,
                      const ocn_fields* out, int stage, int chunk, hipStream_t s)
 {
     const size_t nn = (size_t)h->p.N * h->p.N;
     int cv, rv, rc;
     const int both = OCN_STAGE_COLUMNS | OCN_STAGE_ROWS;
-    if ((stage & both) == both) chunk = std::min(chunk, (int)std::max<size_t>(1, ((size_t)1 << 24) / nn));
+    if ((stage & both) == both) chunk = std::min(chunk, launch_cap(h->p.N));
     for (int f0 = 0; f0 < nframes; f0 += chunk) {
         const int nf = std::min(chunk, nframes - f0);
         pick_schedule(h, nf, &cv, &rv);
@@ -990,6 +994,8 @@ int ocn_autotune(ocn_handle* h, int nframes, int reps, void* stream)
     if ((rc = set_device(h)) || (rc = reserve_z(h, nframes))) return rc;
     hipStream_t s = (hipStream_t)stream;
     const size_t nn = (size_t)h->p.N * h->p.N;
+    const int asked = nframes;
+    nframes = std::min(nframes, launch_cap(h->p.N));  // the launches that frames will run in
     float* outb = nullptr;
     if ((rc = dalloc(&outb, nn * 8 * nframes, "autotune outputs"))) return rc;
     ocn_fields out{outb, outb + nn * nframes, outb + 2 * nn * nframes, outb + 3 * nn * nframes,
@@ -1032,7 +1038,7 @@ int ocn_autotune(ocn_handle* h, int nframes, int reps, void* stream)
     if (bc < 0) return fail(OCN_ENOTSUP, "no schedule available for N=%d", h->p.N);
     {
         std::lock_guard<std::mutex> lk(g_sched_mu);
-        g_sched[{h->device, h->p.N, frames_class(nframes), h->p.normal_mode}] = {bc, br};
+        for (int n : {nframes, asked}) g_sched[{h->device, h->p.N, frames_class(n), h->p.normal_mode}] = {bc, br};
     }
     h->tuned = false;  // use the tuned table entry for this frame count class
     return OCN_OK;

@@ -272,7 +272,8 @@ int ocn_frames_reserved(const ocn_handle* h, int* nframes);
  * counterpart: the reference has one fixed 32x32 dispatch shape (main.cpp:18).
  *
  * ocn_autotune times every variant available for this N on the handle's
- * device (nframes frames per launch, reps launches each, on `stream`, which
+ * device (nframes frames per launch, or as many as a launch of whole frames
+ * takes (ocn_update_frames), reps launches each, on `stream`, which
  * it synchronises; it reserves nframes frames as ocn_reserve_frames does) and
  * records the fastest for (device, N, frames-per-launch class, normal mode);
  * later launches of any handle with that N and normal mode use it.  With

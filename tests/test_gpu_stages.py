@@ -43,3 +43,13 @@ def test_stages_one_by_one_over_more_frames_than_a_launch():
     for k in SIZES:
         for f in range(F):
             assert_field_close("%s f%d" % (k, f), got[k][f], want[k][f])
+
+
+def test_autotune_beyond_a_launch_tunes_the_launches_that_run():
+    """Tuned for 8 frames at N=2048, whose launches hold 4: both launch sizes take the pair found."""
+    print("autotune N=2048 frames=8", flush=True)
+    with pyocean.Ocean(pyocean.make_params(N=2048, L=1000.0, seed=4, normal_mode=1)) as oc:
+        oc.tilde_h0_k()
+        oc.autotune(8, 1)
+        a, b = oc.schedule(8), oc.schedule(4)
+        assert (a["cols_variant"], a["rows_variant"]) == (b["cols_variant"], b["rows_variant"])
