@@ -213,6 +213,8 @@ struct ocn_handle {
     int        device   = 0;
     bool       h0_ready = false;
     int        zcap     = 0;        // frames the intermediate buffers hold
+    int        turn_frames = 0;     // frames_on_handle: whole frames whose launches took the slots in turn,
+    double     turn_t[ocn::kMaxFrames];  // and their times
     int        cols_variant = 0;
     int        rows_variant = 0;
     bool       tuned = false;       // schedule set by ocn_autotune / ocn_set_schedule
@@ -404,16 +406,11 @@ int run_frames(ocn_handle* h, const double* t, int nframes, const ocn_fields* ou
 // most `chunk` frames, intermediates at z1 / z2 (room for `chunk` frames).
 // Each launch takes the schedule for its own frame count, so a short last
 // launch gets the short bands that fill the GPU.
-// Whole frames run in launches of at most launch_cap(N); a single stage keeps
-// the caller's chunks, so that another stage's call finds every frame of a
-// chunk in its own slot.
 int frames_in_chunks(ocn_handle* h, float2* z1, float2* z2, const double* t_host, int nframes,
                      const ocn_fields* out, int stage, int chunk, hipStream_t s)
 {
     const size_t nn = (size_t)h->p.N * h->p.N;
     int cv, rv, rc;
-    const int both = OCN_STAGE_COLUMNS | OCN_STAGE_ROWS;
-    if ((stage & both) == both) chunk = std::min(chunk, launch_cap(h->p.N));
     for (int f0 = 0; f0 < nframes; f0 += chunk) {
         const int nf = std::min(chunk, nframes - f0);
         pick_schedule(h, nf, &cv, &rv);
@@ -427,6 +424,37 @@ int frames_in_chunks(ocn_handle* h, float2* z1, float2* z2, const double* t_host
         if ((rc = run_frames_z(h, z1, z2, t_host + f0, nf, &sl, nn, stage, cv, rv, s))) return rc;
     }
     return OCN_OK;
+}
+
+// The same on the handle's own intermediates, in launches of the reserved frames:
+// frame f of a launch has slot f of Z1 / Z2.
+// Whole frames run in launches of at most launch_cap(N) instead, which take the
+// first slots in turn (in slots of their own they would fill the Infinity Cache one
+// after another: N=2048, 8 frames reserved, 61 us a frame against 50).  Any other
+// set of stages keeps the reserved launches: calls that divide a frame's stages
+// between them then take one schedule, and agree on which of them writes the
+// normals.  Rows called without columns read every frame of a launch in its slot:
+// after whole frames that took the slots in turn, the columns of the frames that
+// the last reserved launch would have held are run again first.
+int frames_on_handle(ocn_handle* h, const double* t_host, int nframes, const ocn_fields* out, int stage,
+                     hipStream_t s)
+{
+    const int reserved = std::min(ocn::kMaxFrames, h->zcap);
+    const int chunk    = stage == OCN_STAGE_ALL ? std::min(reserved, launch_cap(h->p.N)) : reserved;
+    int       rc       = OCN_OK;
+    if (stage & OCN_STAGE_COLUMNS) {
+        h->turn_frames = 0;
+    } else if ((stage & OCN_STAGE_ROWS) && h->turn_frames > 0) {
+        rc = frames_in_chunks(h, h->z1, h->z2, h->turn_t, h->turn_frames, out, OCN_STAGE_COLUMNS, reserved, s);
+        h->turn_frames = 0;
+    }
+    if (!rc) rc = frames_in_chunks(h, h->z1, h->z2, t_host, nframes, out, stage, chunk, s);
+    if (!rc && chunk < reserved && nframes > chunk) {
+        const int last = (nframes - 1) / reserved * reserved;
+        h->turn_frames = nframes - last;
+        std::copy(t_host + last, t_host + nframes, h->turn_t);
+    }
+    return rc;
 }
 
 // Checks shared by the frame entry points (before any HIP call).
@@ -889,8 +917,7 @@ int ocn_update_stage(ocn_handle* h, const double* t_host, int nframes, const ocn
     if (nframes == 0) return OCN_OK;
     if ((rc = set_device(h))) return rc;
     // launches of at most the reserved frame count: nothing is allocated here
-    const int chunk = std::min(ocn::kMaxFrames, h->zcap);
-    return frames_in_chunks(h, h->z1, h->z2, t_host, nframes, out, stage, chunk, (hipStream_t)stream);
+    return frames_on_handle(h, t_host, nframes, out, stage, (hipStream_t)stream);
 }
 
 int ocn_update_frames_noalloc(ocn_handle* h, const double* t_host, int nframes, const ocn_fields* out, void* stream)

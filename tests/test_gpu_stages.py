@@ -53,3 +53,48 @@ def test_autotune_beyond_a_launch_tunes_the_launches_that_run():
         oc.autotune(8, 1)
         a, b = oc.schedule(8), oc.schedule(4)
         assert (a["cols_variant"], a["rows_variant"]) == (b["cols_variant"], b["rows_variant"])
+
+
+RENDER = {"displacement": 16, "render_normals": 16}
+
+
+@pytest.mark.parametrize("N,reserve,frames", [(1024, 32, 20), (2048, 8, 6)])
+def test_stage_subsets_over_more_frames_than_a_launch(N, reserve, frames):
+    """With the render export, whose normals the row stage by itself leaves to the
+    normal-map stage under some schedules and writes under others: columns and rows
+    in one call and the normal map in another, and the rows and the normal map again
+    after whole frames, give every frame of the whole frames."""
+    sizes = dict(SIZES, **RENDER)
+    looked_at = sorted({0, frames // 2, frames - 4, frames - 1})
+    print("stage subsets N=%d reserve=%d frames=%d" % (N, reserve, frames), flush=True)
+    hip = pyocean.Hip()
+    times = 0.5 + np.arange(frames) * 0.25
+    bufs = {k: hip.malloc(frames * N * N * b) for k, b in sizes.items()}
+    fl = pyocean.OcnFields(*[bufs[k] for k in sizes])
+    zeros = np.zeros(frames * N * N * 4, np.float32)
+
+    def taken(*calls):
+        for k, b in sizes.items():
+            hip.upload(bufs[k], zeros[:frames * N * N * b // 4])
+        for c in calls:
+            c()
+        hip.sync()
+        return {k: {f: hip.download(bufs[k] + f * N * N * b, (N, N, 4) if b == 16 else (N, N)) for f in looked_at}
+                for k, b in sizes.items()}
+
+    try:
+        with pyocean.Ocean(pyocean.make_params(N=N, L=1000.0, seed=4)) as oc:
+            oc.tilde_h0_k()
+            oc.reserve_frames(reserve)
+            want = taken(lambda: oc.update_frames(times, fl))
+            apart = taken(lambda: oc.update_stage(times, fl, 1 | 2), lambda: oc.update_stage(times, fl, 4))
+            # (taken clears the outputs first: the second call alone writes what is compared)
+            oc.update_frames(times, fl)
+            again = taken(lambda: oc.update_stage(times, fl, 2 | 4))
+    finally:
+        for v in bufs.values():
+            hip.free(v)
+    for name, got in (("columns and rows, then normals", apart), ("rows and normals after whole frames", again)):
+        for k in sizes:
+            for f in looked_at:
+                assert_field_close("%s: %s f%d" % (name, k, f), got[k][f], want[k][f])
