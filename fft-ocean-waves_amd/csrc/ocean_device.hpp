@@ -357,46 +357,66 @@ __device__ __forceinline__ void cols_lds_strip(const float4* __restrict__ uv, fl
     constexpr int ITERS = (C * H + NB - 1) / NB;  // row-pair tasks per thread
     static_assert(NB >= NT && T <= 64 && 64 % T == 0, "transforms inside one wave");
     static_assert((N / 2) % C == 0, "strips of C columns tile the half plane");
+    // Row 0 and, in strip 0 (FIRST), column 0 take their B coefficients by the load's
+    // address: a load in a branch is another trip to memory, and every column has a row 0.
+    auto folds = [&](auto first) {
+        constexpr bool FIRST = decltype(first)::value;
 #pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-        const int k = threadIdx.x + it * NB;
-        if (k < C * H) {
-            const int    c = k / H, ra = k % H, rb = (N - ra) & (N - 1);
-            const int    tx = strip * C + c, nx = tx - N / 2, ny = ra - N / 2;
-            const float4 qa = uv[(size_t)tx * N + ra], qb = uv[(size_t)tx * N + rb];
-            float        kinv, s, cs;
-            sincos_turns(turns(omega_fp64(sc, nx * nx + ny * ny, kinv), t_rev), s, cs);
-            const float2 A = fold_at(qa, s, cs), B = fold_at(qb, s, cs);
-            // Dx takes B's coefficients in column 0, Dz in row 0 (folded spectrum, above)
-            const float2 Ax = tx == 0 ? fold_at(uv[uv_bcol(N) + ra], s, cs) : A;
-            const float2 Bx = tx == 0 ? fold_at(uv[uv_bcol(N) + rb], s, cs) : B;
-            const float2 Az = ra == 0 ? fold_at(uv[uv_brow(N) + tx], s, cs) : A;
-            const float  mx = (float)nx * kinv, mz = (float)ny * kinv;
-            lds[(0 * C + c) * LEN + lds_pad(ra)] = A;
-            lds[(1 * C + c) * LEN + lds_pad(ra)] = choppy(mx, Ax);
-            lds[(2 * C + c) * LEN + lds_pad(ra)] = choppy(mz, Az);
-            if (rb != ra) {  // rows 0 and N/2 are their own partners
-                lds[(0 * C + c) * LEN + lds_pad(rb)] = B;
-                lds[(1 * C + c) * LEN + lds_pad(rb)] = choppy(mx, Bx);
-                lds[(2 * C + c) * LEN + lds_pad(rb)] = choppy(-mz, B);
+        for (int it = 0; it < ITERS; ++it) {
+            const int k = threadIdx.x + it * NB;
+            if (k < C * H) {
+                const int    c = k / H, ra = k % H, rb = (N - ra) & (N - 1);
+                const int    tx = strip * C + c, nx = tx - N / 2, ny = ra - N / 2;
+                const size_t col = (size_t)tx * N;
+                const float4 qa = uv[col + ra], qb = uv[col + rb];
+                const float4 qz = uv[ra == 0 ? uv_brow(N) + tx : col + ra];
+                const size_t bx = FIRST && tx == 0 ? uv_bcol(N) : col;
+                const float4 xa = FIRST ? uv[bx + ra] : qa, xb = FIRST ? uv[bx + rb] : qb;
+                float        kinv, s, cs;
+                sincos_turns(turns(omega_fp64(sc, nx * nx + ny * ny, kinv), t_rev), s, cs);
+                const float2 B = fold_at(qb, s, cs);
+                const float  mx = (float)nx * kinv, mz = (float)ny * kinv;
+                lds[(0 * C + c) * LEN + lds_pad(ra)] = fold_at(qa, s, cs);
+                lds[(1 * C + c) * LEN + lds_pad(ra)] = choppy(mx, fold_at(xa, s, cs));
+                lds[(2 * C + c) * LEN + lds_pad(ra)] = choppy(mz, fold_at(qz, s, cs));
+                if (rb != ra) {  // rows 0 and N/2 are their own partners
+                    lds[(0 * C + c) * LEN + lds_pad(rb)] = B;
+                    lds[(1 * C + c) * LEN + lds_pad(rb)] = choppy(mx, fold_at(xb, s, cs));
+                    lds[(2 * C + c) * LEN + lds_pad(rb)] = choppy(-mz, B);
+                }
             }
         }
-    }
+    };
     if (strip == 0) {
         // column slot 0 += i * (the Nyquist column's folds), its rows spread
-        // over the whole block; its Dx spectrum is 0 (nx = 0)
-        __syncthreads();
-        for (int ty = threadIdx.x; ty < N; ty += NB) {
-            const int ny = ty - N / 2;
-            float     kinv, s, cs;
+        // over the whole block; its Dx spectrum is 0 (nx = 0).  They are made first, so
+        // that only the sums are left behind the barrier.
+        constexpr int NI = (N + NB - 1) / NB;
+        float2        h[NI], z[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int    ty = (threadIdx.x + i * NB) & (N - 1), ny = ty - N / 2;
+            const float4 q  = uv[(size_t)(N / 2) * N + ty];
+            const float4 qz = uv[ty == 0 ? uv_brow(N) + N / 2 : (size_t)(N / 2) * N + ty];
+            float        kinv, s, cs;
             sincos_turns(phase_turns(sc, ny * ny, t_rev, kinv), s, cs);
-            const float2 h = fold_at(uv[(size_t)(N / 2) * N + ty], s, cs);
-            const float2 z = choppy((float)ny * kinv, ty == 0 ? fold_at(uv[uv_brow(N) + N / 2], s, cs) : h);
-            float2&      ah = lds[0 * C * LEN + lds_pad(ty)];
-            float2&      az = lds[2 * C * LEN + lds_pad(ty)];
-            ah = make_float2(ah.x - h.y, ah.y + h.x);
-            az = make_float2(az.x - z.y, az.y + z.x);
+            h[i] = fold_at(q, s, cs);
+            z[i] = choppy((float)ny * kinv, fold_at(qz, s, cs));
         }
+        folds(std::true_type{});
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int ty = threadIdx.x + i * NB;
+            if (ty < N) {
+                float2& ah = lds[0 * C * LEN + lds_pad(ty)];
+                float2& az = lds[2 * C * LEN + lds_pad(ty)];
+                ah = make_float2(ah.x - h[i].y, ah.y + h[i].x);
+                az = make_float2(az.x - z[i].y, az.y + z[i].x);
+            }
+        }
+    } else {
+        folds(std::false_type{});
     }
     __syncthreads();
     if (NB == NT || (int)threadIdx.x < NT) {

@@ -152,21 +152,32 @@ __global__ __launch_bounds__(C*(N / 8), 4) void k_cols(const float4* __restrict_
                                    fb.t_rev[f], strip, lds);
 }
 
-// LDS-staged strips (cols_lds_strip), single frames N=1024 26.4 -> 25.4 us, N=64
-// 32-frame launches 0.69 -> 0.52 us per frame on the folded spectrum: twice the transforms' 3C x T threads, the
-// extra ones folding and storing only.
+// LDS-staged strips (cols_lds_strip), for launches of few frames: a short chain from
+// the first load to the last store.  Threads for the strip's C (N/2 + 1) row pairs, and
+// with them its stores, in one round where a block of 1024 holds them, else twice the
+// transforms' 3C x T; those past the transforms fold and store only.  A second round
+// puts another trip to memory and another dispersion phase behind the first: with
+// twice the transforms' threads at every size, single frames (us) N=64 8.5 -> 7.6, 128
+// 8.8 -> 8.0, 256 9.5 -> 8.8, 512 12.9 -> 12.6, 1024 27.0 -> 26.6.
 template <int N, int C>
-__global__ __launch_bounds__(2 * 3 * C * (N / 16)) void k_cols_lds(const float4* __restrict__ uv,
-                                                                   float2* __restrict__ z1, float2* __restrict__ z2,
-                                                                   const float2* __restrict__ tw, SpecConst sc,
-                                                                   FrameBatch fb)
+constexpr int cols_lds_threads()
+{
+    constexpr int one = (C * (N / 2 + 1) + 63) / 64 * 64;
+    return one <= 1024 ? one : 2 * 3 * C * (N / 16);
+}
+template <int N, int C>
+__global__ __launch_bounds__((cols_lds_threads<N, C>())) void k_cols_lds(const float4* __restrict__ uv,
+                                                                        float2* __restrict__ z1,
+                                                                        float2* __restrict__ z2,
+                                                                        const float2* __restrict__ tw, SpecConst sc,
+                                                                        FrameBatch fb)
 {
     __shared__ float2 lds[3 * C * strip_len(N)];
     int f, strip;
     cols_block<N, C>(fb, f, strip);
     if (strip >= lds_strips<N, C>()) return;  // padding of the last group (whole block)
-    cols_lds_strip<N, C, 2 * 3 * C * (N / 16)>(uv, z1 + (size_t)f * fb.z1_stride, z2 + (size_t)f * fb.z2_stride, tw,
-                                               sc, fb.t_rev[f], strip, lds);
+    cols_lds_strip<N, C, cols_lds_threads<N, C>()>(uv, z1 + (size_t)f * fb.z1_stride, z2 + (size_t)f * fb.z2_stride,
+                                                   tw, sc, fb.t_rev[f], strip, lds);
 }
 
 // ------------------------------------------------------------------ fused frame, pass 2
@@ -707,7 +718,7 @@ static hipError_t launch_cols_v(const FrameArgs& a, hipStream_t s)
         constexpr int G = strip_group<N, C>(), groups = (lds_strips<N, C>() + G - 1) / G;
         const dim3    grid(groups * G * a.nframes);
         if constexpr (kColsVariants[V].lds)
-            hipLaunchKernelGGL((k_cols_lds<N, C>), grid, dim3(2 * 3 * C * (N / 16)), 0, s, a.uv, a.z1, a.z2,
+            hipLaunchKernelGGL((k_cols_lds<N, C>), grid, dim3(cols_lds_threads<N, C>()), 0, s, a.uv, a.z1, a.z2,
                                a.tw[radix_slot(16)], a.sc, a.fb);
         else
             hipLaunchKernelGGL((k_cols<N, C>), grid, dim3(C * (N / 8)), 0, s, a.uv, a.z1, a.z2, a.tw[radix_slot(8)],
