@@ -289,6 +289,14 @@ __global__ __launch_bounds__(N / E >= 64 ? N / E : 64, 2) void k_rows_nrm(
 // the same halo tiles, run on one XCD.
 //
 // RENDER adds the render export (disp, rnorm, either may be null), as in the walk.
+// Launches of 2^19 to 2^22 texels write it by plain stores: an export of 134 MB, half
+// of the Infinity Cache, stays there.  With all outputs non-temporal, frames written
+// to the same buffers over and over were slower than the unfused passes (N=512, 8
+// frames, us per frame: unfused 5.8, non-temporal 6.3, plain 5.5; into buffers that
+// change 6.4, 5.4, 5.1; N=1024, 2 frames 24.3, 25.2, 23.4).  Larger exports do not stay
+// in the cache (N=512, 32 frames: non-temporal 4.13, plain 4.34); smaller ones would
+// stay in the L2s and be written back at the launch's end (N=512, single frames 13.5,
+// 14.2).
 // BIL takes the height taps bilinearly at texel corners (OCN_NORMALS_BILINEAR):
 // the 2x2 box folded into the Sobel weights is [1 3 3 1] along one axis and
 // [1 1 -1 -1] along the other over x-2..x+1, y-2..y+1, so one more Z1 row is
@@ -309,7 +317,7 @@ __global__ __launch_bounds__((W * par_groups<N, E, R, BIL>() * (N / E))) void k_
     const float2* __restrict__ z1, const float2* __restrict__ z2, float* __restrict__ height,
     float* __restrict__ dx, float* __restrict__ dz, float4* __restrict__ normals, float* __restrict__ jac,
     const float2* __restrict__ tw, FrameBatch fb, float lambda, float inv2d, float4* __restrict__ disp,
-    float4* __restrict__ rnorm, float dscale)
+    float4* __restrict__ rnorm, float dscale, bool plain)
 {
     // W = 2: twice the threads, the extra ones (after the G transform groups)
     // taking part in the stencils only
@@ -353,6 +361,10 @@ __global__ __launch_bounds__((W * par_groups<N, E, R, BIL>() * (N / E))) void k_
     }
     __syncthreads();
 
+    auto put = [&](float4* p, float4 v) {
+        if (plain) *p = v;
+        else st_out(p, v);
+    };
     // Stencils: each thread walks whole columns x of the band, keeping the
     // signed values of x-1, x, x+1 for all band and halo rows in registers
     // (each LDS value is read once per column).  The sign (-1)^(x+y) / N^2 of
@@ -428,15 +440,14 @@ __global__ __launch_bounds__((W * par_groups<N, E, R, BIL>() * (N / E))) void k_
                 const float dzdz = (zm[i + 1] - zm[i - 1]) * inv2d;
                 const float J = (1.0f - lambda * dxdx) * (1.0f - lambda * dzdz) - lambda * lambda * dxdz * dzdx;
                 if (jac) st_out(&jac[o], J);
-                if (RENDER && disp)
-                    st_out(&disp[o], make_float4(-lambda * hm[g].y, dscale * hm[g].x, -lambda * zm[i], J));
+                if (RENDER && disp) put(&disp[o], make_float4(-lambda * hm[g].y, dscale * hm[g].x, -lambda * zm[i], J));
                 if (RENDER && rnorm) {
                     // n = dP/dv x dP/du (rows_nrm_band); its y component is J
                     const float dhdx = (hr[g].x - hl[g].x) * inv2d, dhdz = (hm[g + 1].x - hm[g - 1].x) * inv2d;
                     const float nx  = -dscale * (lambda * dhdz * dzdx + (1.0f - lambda * dzdz) * dhdx);
                     const float nz  = -dscale * (lambda * dxdz * dhdx + dhdz * (1.0f - lambda * dxdx));
                     const float inv = rsqrtf(fmaf(nx, nx, fmaf(J, J, nz * nz)));
-                    st_out(&rnorm[o], make_float4(nx * inv, J * inv, nz * inv, 1.0f));
+                    put(&rnorm[o], make_float4(nx * inv, J * inv, nz * inv, 1.0f));
                 }
             }
             st_out(&height[o], hm[g].x);
@@ -737,13 +748,14 @@ static hipError_t launch_rows_v(const FrameArgs& a, hipStream_t s)
     } else if constexpr (P) {
         auto launch = [&](auto bil, auto ren) {
             constexpr bool BIL = decltype(bil)::value, REN = decltype(ren)::value;
+            const int      texels = a.nframes * N * N;
             if constexpr (!rows_fits<N, E, B, true, W, BIL>()) {
                 return hipErrorInvalidValue;
             } else {
                 hipLaunchKernelGGL((k_rows_nrm_par<N, E, B, W, BIL, REN>), dim3((N / B) * a.nframes),
                                    dim3(W * par_groups<N, E, B, BIL>() * (N / E)), 0, s, a.z1, a.z2, a.height, a.dx,
                                    a.dz, a.normals, a.jacobian, a.tw[radix_slot(E)], a.fb, a.lambda, a.inv2d, a.disp,
-                                   a.rnorm, a.dscale);
+                                   a.rnorm, a.dscale, texels > (1 << 19) && texels <= (1 << 22));
                 return hipGetLastError();
             }
         };
