@@ -165,6 +165,10 @@ int launch_cap(int N) { return std::min(ocn::kMaxFrames, std::max(1, (1 << 24) /
 // frames 5.56 / 5.99, 5 frames 5.65 / 5.43 (render export 7.25 / 6.96), 6 frames
 // 5.52 / 4.97, 8 frames 5.22 / 4.53; N=1024, 1 frame 25.4 / 25.7, 2
 // frames 18.9 / 19.5, 4 frames 16.4 / 15.1, 16 frames 11.6 / 11.3.
+// At N=1024 and 4 columns 512 blocks are resident: 4 frames fill them, 3 and 5 leave
+// part of a round empty and take 2 columns, in blocks half as large (4 columns / 2,
+// frames into the same buffers: 3 frames 17.7 / 16.9, 4 frames 14.9 / 15.2, 5 frames
+// 14.4 / 14.0; into buffers that change 16.7 / 16.1, 14.4 / 14.3, 14.1 / 13.8).
 std::pair<int, int> default_schedule(int N, int nframes)
 {
     const bool batch = nframes > 1;
@@ -182,7 +186,7 @@ std::pair<int, int> default_schedule(int N, int nframes)
     case 256: cv = nframes >= 5 && nframes <= 16 ? 21 : 14; rv = 8; break;
     case 512: cv = nframes <= 2 ? 14 : nframes <= 4 ? 21 : 12; rv = batch ? 7 : 8; break;
     case 1024:
-        cv = !batch ? 13 : nframes <= 2 ? 14 : 9;
+        cv = !batch ? 13 : nframes <= 2 ? 14 : nframes == 3 || nframes == 5 ? 8 : 9;
         rv = !batch ? 7 : nframes <= 6 ? 7 : nframes <= 9 ? 3 : nframes <= 16 ? 4 : 5;
         break;
     // N=2048: 2 columns per block up to a few frames (single frames 79.4 -> 65.1
