@@ -94,16 +94,22 @@ __device__ __forceinline__ float2 phase_at(double w, double t_rev)
     return make_float2(c, s);
 }
 
-// Sums of four values over the block, in one pass: across each wave, then over
-// the waves in order (the result is thread 0's).  red holds one float4 per wave.
-__device__ __forceinline__ float4 block_sum4(float4 t, float4* red)
+// Sums of four values over the block (of the first alone unless `all`; the others
+// are 0 then), in one pass: across each wave, then over the waves in order (the result
+// is thread 0's).  red holds one float4 per wave.
+__device__ __forceinline__ float4 block_sum4(float4 t, bool all, float4* red)
 {
+    if (all) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        t.x += __shfl_xor(t.x, o);
-        t.y += __shfl_xor(t.y, o);
-        t.z += __shfl_xor(t.z, o);
-        t.w += __shfl_xor(t.w, o);
+        for (int o = 32; o > 0; o >>= 1) {
+            t.x += __shfl_xor(t.x, o);
+            t.y += __shfl_xor(t.y, o);
+            t.z += __shfl_xor(t.z, o);
+            t.w += __shfl_xor(t.w, o);
+        }
+    } else {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) t.x += __shfl_xor(t.x, o);
     }
     if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64] = t;
     __syncthreads();
@@ -383,7 +389,7 @@ __global__ __launch_bounds__(kFitColsThreads) void k_fit_spectral(const FitMembe
     else s = fit_spectral_parts<n, 1>(m, v, it.y, mode)
     OCN_FIT_SWITCH(m.N, OCN_CALL)
 #undef OCN_CALL
-    s = block_sum4(s, red);
+    s = block_sum4(s, mode != kFitLoss, red);
     if (threadIdx.x == 0) parts[idx] = s;
 }
 
@@ -568,7 +574,7 @@ struct FitSums {
     double loss, dV, dT, dA;
 };
 __device__ __forceinline__ FitSums fit_sums(const FitRange& rg, const float4* __restrict__ parts, float4 p,
-                                            double (*red)[4])
+                                            bool all, double (*red)[4])
 {
     double a[4] = {(double)p.x, (double)p.y, (double)p.z, (double)p.w};
     for (int i = threadIdx.x + kFitReduceThreads; i < rg.count; i += kFitReduceThreads) {
@@ -578,10 +584,15 @@ __device__ __forceinline__ FitSums fit_sums(const FitRange& rg, const float4* __
         a[2] += (double)p.z;
         a[3] += (double)p.w;
     }
+    if (all) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
+        for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) a[j] += __shfl_xor(a[j], o);
+            for (int j = 0; j < 4; ++j) a[j] += __shfl_xor(a[j], o);
+    } else {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) a[0] += __shfl_xor(a[0], o);
+    }
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
         for (int j = 0; j < 4; ++j) red[threadIdx.x / 64][j] = a[j];
@@ -627,7 +638,7 @@ __global__ __launch_bounds__(kFitReduceThreads) void k_fit_reduce(const FitRange
         b1t = __shfl(bt, 0);
         b2t = __shfl(bt, 1);
     }
-    const FitSums sum = fit_sums(rg, parts, p, red);
+    const FitSums sum = fit_sums(rg, parts, p, mode != kFitLoss, red);
     if (!lead) return;
     if (wave == 3) rep.loss = vars.loss = sum.loss / rg.knn;
     if (wave == 3 || mode == kFitLoss) return;
@@ -674,7 +685,7 @@ __global__ __launch_bounds__(kFitReduceThreads) void k_fit_reduce_qn(const FitRa
 #pragma unroll
         for (int i = 0; i < 6; ++i) v.qH[i] = vars.qH[i];
     }
-    const FitSums sum = fit_sums(rg, parts, fit_first_part(rg, parts), red);
+    const FitSums sum = fit_sums(rg, parts, fit_first_part(rg, parts), true, red);
     if (threadIdx.x != 0) return;
     const double L = sum.loss / rg.knn, g[3] = {sum.dV, sum.dT, sum.dA};
     qn_step(v, L, g, cfg);
