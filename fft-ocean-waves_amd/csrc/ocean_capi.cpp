@@ -1674,23 +1674,25 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
     if (e != hipSuccess) rc = hip_fail(e, "hipGetDevice");
     // Per member, 256-byte aligned: xi 16, targets 4 K, dL/dh0 16 bytes per texel,
     // the targets' spectra T^ (8 bytes per frame and texel pair of the half plane), with equally spaced
-    // times and split strips the phase table (16 bytes per texel pair of the half plane), the noise coefficients (16 bytes
+    // times and fewer than 512 strips the phase table (16 bytes per texel pair of the half plane), the noise coefficients (16 bytes
     // per texel pair of the half plane) and the unit noise of the edge pairs (32 bytes each).
     // Small fits split each column strip's rows over up to four blocks so the
-    // step launch has at least two blocks per CU of the 256.
-    int row_parts = 1;
-    {
-        long items = 0;
-        for (const ocn_params& p : f->params) items += ocn::fit_cols_items_per_member(p.N);
-        while (row_parts < ocn::kFitMaxRowParts && items * row_parts < 512) row_parts *= 2;
-    }
+    // step launch has at least two blocks per CU of the 256.  A few strips more than
+    // that would leave a few CUs with a third block and the others waiting for them:
+    // such fits split their strips in two (us, whole strips -> halves: one N = 1024
+    // ocean, K = 4, loss 11.8 -> 11.1, Adam step 12.6 -> 12.5; 16 oceans of N = 256 12.3
+    // -> 11.0, 13.4 -> 12.7; from 600 strips on even).
+    long items = 0;
+    for (const ocn_params& p : f->params) items += ocn::fit_cols_items_per_member(p.N);
+    int row_parts = items >= 512 && items < 600 ? 2 : 1;
+    while (row_parts < ocn::kFitMaxRowParts && items * row_parts < 512) row_parts *= 2;
     auto   al    = [](size_t x) { return (x + 255) & ~size_t(255); };
-    // Equally spaced times: a step of whole strips is bound by memory and evaluates
+    // Equally spaced times: from 512 strips on a step is bound by memory and evaluates
     // its pairs' phases, 16 of the 64 bytes a pair would read at K = 4 (256 oceans of
-    // N = 256, 96 -> 75 us; one of N = 1024, K = 8, 15.5 -> 15.0); one of split strips
+    // N = 256, 96 -> 75 us; one of N = 1024, K = 8, 15.5 -> 15.0); one of fewer strips
     // is bound by latency and reads them from a table (N = 512, K = 8: 7.8 us, 8.2
     // evaluated).
-    const bool phase_table = uniform_times && row_parts > 1;
+    const bool phase_table = uniform_times && items < 512;
     auto   phase_bytes = [&](int N) { return phase_table ? al(sizeof(float4) * ocn::fit_phase_entries(N)) : 0; };
     auto   bytes = [&](int N) {
         const size_t nn = (size_t)N * N;

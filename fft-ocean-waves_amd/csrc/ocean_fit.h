@@ -106,9 +106,9 @@ struct FitMember {
     // per pair at fit_edge_index.
     const float4* pq;
     const float4* edge;
-    // Equally spaced times and split strips: per column item and texel pair
-    // of its strip, the dispersion phase e^{i w t_0} and its step e^{i w dt} as
-    // (cos, sin, cos, sin), written once at creation (launch_fit_phase); entry
+    // Equally spaced times and a fit of fewer than 512 strips: per column item
+    // and texel pair of its strip, the dispersion phase e^{i w t_0} and its step
+    // e^{i w dt} as (cos, sin, cos, sin), written once at creation (launch_fit_phase); entry
     // (strip * N + ty) * C + c.  Null otherwise.
     const float4* phase;
     const float2* tw8;      // Stockham twiddles (N, 8) and (N, 16)

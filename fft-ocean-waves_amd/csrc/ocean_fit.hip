@@ -357,7 +357,7 @@ template <int N, int R>
 __device__ __forceinline__ float4 fit_spectral_parts(const FitMember& m, const FitVars& v, int item, int mode)
 {
     if (m.phase) return fit_spectral<N, kPhaseTable, R>(m, v, item, mode);
-    if constexpr (R == 1)  // split strips are few: equally spaced times always have the table
+    if constexpr (R <= 2)  // quartered strips are few: equally spaced times always have the table
         if (m.uniform) return fit_spectral<N, kPhaseStart, R>(m, v, item, mode);
     return fit_spectral<N, kPhaseEach, R>(m, v, item, mode);
 }
