@@ -1010,8 +1010,8 @@ int ocn_get_schedule(const ocn_handle* h, int nframes, int* cols_variant, int* r
     if (cols_radix) *cols_radix = E;
     if (cols_per_block) *cols_per_block = C;
     if (rows_radix) *rows_radix = ocn::rows_variant_radix(rv);
-    if (rows_band)
-        *rows_band = ocn::rows_variant_band(h->p.N, rv, h->p.normal_mode != OCN_NORMALS_NEAREST, nframes);
+    // what a row stage by itself does: with bilinear normals only whole frames fuse the normal map
+    if (rows_band) *rows_band = h->p.normal_mode == OCN_NORMALS_NEAREST ? ocn::rows_variant_band(rv) : 0;
     return OCN_OK;
 }
 

@@ -90,8 +90,7 @@ hipError_t launch_normals(int N, const float* height, const float* dx, const flo
 bool       schedule_valid(int N, int cols_variant, int rows_variant);
 void       cols_variant_shape(int N, int v, int* E, int* C);
 int        rows_variant_radix(int v);
-// 0: separate normal-map kernel; R: fused bands of R rows
-int        rows_variant_band(int N, int v, bool bilinear, int nframes);
+int        rows_variant_band(int v);  // 0: separate normal-map kernel; R: fused bands of R rows
 bool       rows_variant_walk(int v);  // fused bands walked row by row (nearest taps only)
 
 }  // namespace ocn

@@ -935,13 +935,7 @@ void cols_variant_shape(int N, int v, int* E, int* C)
 
 int rows_variant_radix(int v) { return kRowsVariants[v].E; }
 
-int rows_variant_band(int N, int v, bool bilinear, int nframes)
-{
-    if (!bilinear) return kRowsVariants[v].band;
-#define CALL(n) kRowsVariants[bilinear_rows<n>(v, nframes)].band
-    OCN_DISPATCH_N(N, CALL, 0)
-#undef CALL
-}
+int rows_variant_band(int v) { return kRowsVariants[v].band; }
 
 bool rows_variant_walk(int v) { return kRowsVariants[v].band > 0 && !kRowsVariants[v].par; }
 

@@ -279,9 +279,12 @@ int ocn_frames_reserved(const ocn_handle* h, int* nframes);
  * later launches of any handle with that N and normal mode use it.  With
  * bilinear normals, which no row walk reads, the walks are not timed.  ocn_set_schedule
  * pins a variant pair on this handle; ocn_get_schedule reports the pair used
- * for launches of nframes frames and its shape (any out-pointer may be NULL);
- * rows_band > 0 means the normal map and Jacobian are fused into the row pass,
- * which walks bands of that many rows. */
+ * for launches of nframes frames and its shape (any out-pointer may be NULL).
+ * rows_band > 0 means that OCN_STAGE_ROWS writes the normal map and Jacobian
+ * too, in bands of that many rows (where the render export is asked for, the
+ * parallel bands leave all of it to OCN_STAGE_NORMALS, which writes whatever
+ * the row stage did not); it is 0 with bilinear normals, which only whole
+ * frames fuse into the row pass. */
 int ocn_autotune(ocn_handle* h, int nframes, int reps, void* stream);
 /* The autotuner's table as a text file, so a tuned schedule outlives the
  * process: ocn_autotune_save writes every entry ocn_autotune recorded in this

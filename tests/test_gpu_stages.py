@@ -98,3 +98,38 @@ def test_stage_subsets_over_more_frames_than_a_launch(N, reserve, frames):
         for k in sizes:
             for f in looked_at:
                 assert_field_close("%s: %s f%d" % (name, k, f), got[k][f], want[k][f])
+
+
+@pytest.mark.parametrize("N,frames", [(256, 1), (1024, 2), (2048, 2)])
+def test_bilinear_stages_follow_the_reported_schedule(N, frames):
+    """A caller that calls the normal-map stage where ocn_get_schedule says that the
+    row stage does not write the normals gets them with bilinear taps too."""
+    print("bilinear stages N=%d frames=%d" % (N, frames), flush=True)
+    hip = pyocean.Hip()
+    times = 0.5 + np.arange(frames) * 0.25
+    bufs = {k: hip.malloc(frames * N * N * b) for k, b in SIZES.items()}
+    fl = pyocean.OcnFields(*[bufs[k] for k in SIZES])
+
+    def taken():
+        hip.sync()
+        return {k: hip.download(bufs[k], (frames, N, N) + ((4,) if b == 16 else ())) for k, b in SIZES.items()}
+
+    try:
+        with pyocean.Ocean(pyocean.make_params(N=N, L=1000.0, seed=4, normal_mode=1)) as oc:
+            oc.tilde_h0_k()
+            oc.reserve_frames(frames)
+            oc.update_frames(times, fl)
+            want = taken()
+            for k, b in SIZES.items():
+                hip.upload(bufs[k], np.zeros(frames * N * N * b // 4, np.float32))
+            oc.update_stage(times, fl, 1)
+            oc.update_stage(times, fl, 2)
+            if oc.schedule(frames)["rows_band"] == 0:
+                oc.update_stage(times, fl, 4)
+            got = taken()
+    finally:
+        for v in bufs.values():
+            hip.free(v)
+    for k in SIZES:
+        for f in range(frames):
+            assert_field_close("%s f%d" % (k, f), got[k][f], want[k][f])
