@@ -494,6 +494,7 @@ struct ocn_batch {
     bool                                   render      = false;
     std::map<int, std::array<float2*, 2>>  tw;  // per N: radix-8 and radix-16 Stockham twiddles
     bool                                   h0_ready  = false;
+    mutable std::vector<char>              h0_out;  // members whose h0 a caller has the address of
     hipGraph_t                             graph     = nullptr;
     hipGraphExec_t                         exec      = nullptr;
     hipGraphNode_t                         node_cols = nullptr;
@@ -623,6 +624,31 @@ int batch_ready(const ocn_batch* b, double t)
     if (!b->h0_ready) return fail(OCN_ESTATE, "the spectra do not exist yet: call ocn_batch_tilde_h0_k first");
     hipError_t e = hipSetDevice(b->device);
     return e == hipSuccess ? OCN_OK : hip_fail(e, "hipSetDevice");
+}
+
+// Ahead of a frame's columns: the folded spectrum of the members whose h0 the caller
+// may have written to (ocn_batch_get_h0).
+hipError_t batch_fold(const ocn_batch* b, hipStream_t s)
+{
+    hipError_t e = hipSuccess;
+    if (b->h0_out.empty()) return e;
+    for (int N = ocn::kBatchMinN; N <= ocn::kBatchMaxN; N *= 2) {
+        ocn::FoldList list;
+        int           n = 0;
+        for (size_t i = 0; e == hipSuccess && i < b->members.size(); ++i) {
+            if (b->h0_out[i] && b->params[i].N == N) {
+                list.h0[n]        = b->members[i].h0;
+                list.uv[n]        = b->members[i].uv;
+                list.conj_mode[n] = b->params[i].conj_mode;
+                ++n;
+            }
+            if (n == ocn::kFoldList || (n > 0 && i + 1 == b->members.size())) {
+                e = ocn::launch_fold(N, list, n, s);
+                n = 0;
+            }
+        }
+    }
+    return e;
 }
 
 }  // namespace
@@ -1347,8 +1373,10 @@ int ocn_batch_update(ocn_batch* b, double t, void* stream)
     TraceRange trace("ocn_batch_update");
     int rc = batch_ready(b, t);
     if (rc) return rc;
-    hipError_t e = ocn::launch_batch_frame(b->d_members, b->d_cols, b->n_cols, b->d_rows, b->n_rows, b->d_wide,
-                                           b->n_wide, t / (2.0 * kPi), b->render, (hipStream_t)stream);
+    hipError_t e = batch_fold(b, (hipStream_t)stream);
+    if (e == hipSuccess)
+        e = ocn::launch_batch_frame(b->d_members, b->d_cols, b->n_cols, b->d_rows, b->n_rows, b->d_wide, b->n_wide,
+                                    t / (2.0 * kPi), b->render, (hipStream_t)stream);
     return e == hipSuccess ? OCN_OK : hip_fail(e, "batch update launch");
 }
 
@@ -1399,6 +1427,7 @@ int ocn_batch_update_graph(ocn_batch* b, double t, void* stream)
     } else if ((e = hipGraphExecKernelNodeSetParams(b->exec, b->node_cols, &kc)) != hipSuccess) {
         return hip_fail(e, "hipGraphExecKernelNodeSetParams");
     }
+    if ((e = batch_fold(b, (hipStream_t)stream)) != hipSuccess) return hip_fail(e, "batch fold launch");
     e = hipGraphLaunch(b->exec, (hipStream_t)stream);
     return e == hipSuccess ? OCN_OK : hip_fail(e, "hipGraphLaunch");
 }
@@ -1607,6 +1636,8 @@ int ocn_batch_get_h0(const ocn_batch* b, int member, void** h0)
     if (!h0) return fail(OCN_EINVAL, "h0 is NULL");
     if (member < 0 || member >= (int)b->members.size())
         return fail(OCN_EINVAL, "member %d out of range [0, %zu)", member, b->members.size());
+    b->h0_out.resize(b->members.size());
+    b->h0_out[member] = 1;
     *h0 = b->members[member].h0;
     return OCN_OK;
 }

@@ -79,6 +79,14 @@ constexpr size_t uv_entries(int N) { return ((size_t)N * (N / 2 + 1) + N + N / 2
 
 // h0 of the spectrum (N*N) and its folded form uv (uv_entries(N))
 hipError_t launch_h0(int N, float4* h0, float4* uv, const uint8_t* noise, const SpecConst& sc, hipStream_t s);
+// uv of the first `count` spectra of a list, all of size N, from h0 as it stands
+constexpr int kFoldList = 128;
+struct FoldList {
+    float4* h0[kFoldList];
+    float4* uv[kFoldList];
+    int     conj_mode[kFoldList];
+};
+hipError_t launch_fold(int N, const FoldList& list, int count, hipStream_t s);
 hipError_t launch_spectrum_t(int N, const float4* h0, float2* hy, float2* hx, float2* hz, const SpecConst& sc,
                              double t_rev, hipStream_t s);
 // stages: bit 0 = spectrum + column transforms, bit 1 = row transforms +

@@ -45,10 +45,12 @@ namespace ocn {
 // themselves, hold N + 2 pairs, and the N threads of column 0 take them all.
 // Against drawing h0 alone (and, from N = 2048, transposing it): N=512 3.9 -> 4.7
 // us, 1024 11.1 -> 12.6, 2048 57.8 -> 37.5.
+// SRC kStored takes h0 as it stands and makes uv alone.
 constexpr int kH0Tile = 16;
-template <bool NOISE>
-__global__ __launch_bounds__(kH0Tile* kH0Tile) void k_tilde_h0_k(float4* __restrict__ h0, float4* __restrict__ uv,
-                                                                 const uint8_t* __restrict__ noise, SpecConst sc)
+enum H0Source { kPhilox, kNoiseImages, kStored };
+template <H0Source SRC>
+__device__ __forceinline__ void h0_tile(float4* __restrict__ h0, float4* __restrict__ uv,
+                                        const uint8_t* __restrict__ noise, const SpecConst& sc)
 {
     __shared__ float4 tile[kH0Tile][kH0Tile + 1];  // [tx][ty]
     const int N = sc.N, lx = threadIdx.x % kH0Tile, ly = threadIdx.x / kH0Tile;
@@ -62,8 +64,9 @@ __global__ __launch_bounds__(kH0Tile* kH0Tile) void k_tilde_h0_k(float4* __restr
     const int  px = tx == 0 && ty > N / 2 ? N / 2 : tx, py = ty;
     const int  qx = self ? N / 2 : (N - px) & (N - 1), qy = self ? ty : my;
     auto texel = [&](int x, int y, float s) {
+        if constexpr (SRC == kStored) return h0[(size_t)y * N + x];
         float4 xi;
-        if constexpr (NOISE) {
+        if constexpr (SRC == kNoiseImages) {
             const int o = min((y * 256) / N, 255) * 256 + min((x * 256) / N, 255);
             xi = box_muller(noise[o] / 255.0f, noise[65536 + o] / 255.0f, noise[131072 + o] / 255.0f,
                             noise[196608 + o] / 255.0f);
@@ -77,8 +80,10 @@ __global__ __launch_bounds__(kH0Tile* kH0Tile) void k_tilde_h0_k(float4* __restr
     const float  s = phillips_amp(sc, px, py);
     const float  t = tx != 0 && ty != 0 ? s : phillips_amp(sc, qx, qy);
     const float4 p = texel(px, py, s), q = texel(qx, qy, t);
-    h0[(size_t)py * N + px] = p;
-    h0[(size_t)qy * N + qx] = q;
+    if constexpr (SRC != kStored) {
+        h0[(size_t)py * N + px] = p;
+        h0[(size_t)qy * N + qx] = q;
+    }
     const int cm = sc.conj_mode;
     if (tx != 0) {
         tile[lx][ly] = fold_coeffs(p, q, cm, 1.0f);
@@ -96,6 +101,22 @@ __global__ __launch_bounds__(kH0Tile* kH0Tile) void k_tilde_h0_k(float4* __restr
     }
     __syncthreads();
     if (x0 + ly != 0) uv[(size_t)(x0 + ly) * N + y0 + lx] = tile[ly][lx];
+}
+
+template <H0Source SRC>
+__global__ __launch_bounds__(kH0Tile* kH0Tile) void k_tilde_h0_k(float4* __restrict__ h0, float4* __restrict__ uv,
+                                                                 const uint8_t* __restrict__ noise, SpecConst sc)
+{
+    h0_tile<SRC>(h0, uv, noise, sc);
+}
+
+// uv of the spectra of a list (blockIdx.z), all of size N, as they stand.
+__global__ __launch_bounds__(kH0Tile* kH0Tile) void k_fold(FoldList list, int N)
+{
+    SpecConst sc{};
+    sc.N         = N;
+    sc.conj_mode = list.conj_mode[blockIdx.z];
+    h0_tile<kStored>(list.h0[blockIdx.z], list.uv[blockIdx.z], nullptr, sc);
 }
 
 // Pass API: the three spectrum textures of tilde_h0_t (dy, dx, dz), float2 each.
@@ -985,8 +1006,14 @@ void* static_scratch_ptr(int device)
 hipError_t launch_h0(int N, float4* h0, float4* uv, const uint8_t* noise, const SpecConst& sc, hipStream_t s)
 {
     const dim3 grid(N / 2 / kH0Tile, N / kH0Tile), block(kH0Tile * kH0Tile);
-    if (noise) hipLaunchKernelGGL(k_tilde_h0_k<true>, grid, block, 0, s, h0, uv, noise, sc);
-    else hipLaunchKernelGGL(k_tilde_h0_k<false>, grid, block, 0, s, h0, uv, noise, sc);
+    if (noise) hipLaunchKernelGGL(k_tilde_h0_k<kNoiseImages>, grid, block, 0, s, h0, uv, noise, sc);
+    else hipLaunchKernelGGL(k_tilde_h0_k<kPhilox>, grid, block, 0, s, h0, uv, noise, sc);
+    return hipGetLastError();
+}
+
+hipError_t launch_fold(int N, const FoldList& list, int count, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_fold, dim3(N / 2 / kH0Tile, N / kH0Tile, count), dim3(kH0Tile * kH0Tile), 0, s, list, N);
     return hipGetLastError();
 }
 

@@ -377,7 +377,10 @@ int ocn_batch_autotune(ocn_batch* b, int reps, void* stream);
 
 /* Device pointers of one member's outputs (valid until ocn_batch_destroy;
  * displacement and render_normals are NULL unless the render export is on)
- * and its h0 spectrum (float4[N*N], for reading, as ocn_get_spectrum's). */
+ * and its h0 spectrum (float4[N*N]).  h0 may be written to: from the
+ * ocn_batch_get_h0 call on every ocn_batch_update and ocn_batch_update_graph
+ * takes that member's h0 as it stands, by a pass over it ahead of the frame
+ * (24 bytes a texel). */
 int ocn_batch_get_fields(const ocn_batch* b, int member, ocn_fields* out);
 /* Render export for every member on (1) or off (0): the row pass then also
  * writes each member's displacement and render_normals as ocn_update_into
