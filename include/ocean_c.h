@@ -254,15 +254,17 @@ int ocn_update_frames(ocn_handle* h, const double* t_host, int nframes, const oc
 int ocn_update_frames_noalloc(ocn_handle* h, const double* t_host, int nframes, const ocn_fields* out, void* stream);
 
 /* Sizes the handle's intermediate buffers for launches of up to nframes frames
- * (1..32; 12 bytes per texel and frame): a setup call, which allocates and,
+ * (1..32; 12 bytes per texel and frame: 201 MB a frame at N = 4096, where
+ * whole frames run one by one and use the first): a setup call, which allocates and,
  * when it grows the buffers, waits for the device and frees the old ones.
  * Graphs captured from this handle before a growth must be captured again.
  * A smaller nframes than the current reservation keeps the buffers.  No
  * reference counterpart (the reference runs one frame per update(),
  * main.cpp:240-244, on textures allocated once, main.cpp:1089-1099). */
 int ocn_reserve_frames(ocn_handle* h, int nframes);
-/* Frames per launch the handle's buffers hold (the launch size of
- * ocn_update_frames). */
+/* Frames per launch the handle's buffers hold: the launch size of
+ * ocn_update_stage, and with its limit of 2^24 texels of ocn_update_frames
+ * (which leaves the buffers beyond that to the stages). */
 int ocn_frames_reserved(const ocn_handle* h, int* nframes);
 
 /* ---------------------------------------------------------------- schedules */
@@ -279,7 +281,8 @@ int ocn_frames_reserved(const ocn_handle* h, int* nframes);
  * later launches of any handle with that N and normal mode use it.  With
  * bilinear normals, which no row walk reads, the walks are not timed.  ocn_set_schedule
  * pins a variant pair on this handle; ocn_get_schedule reports the pair used
- * for launches of nframes frames and its shape (any out-pointer may be NULL).
+ * for launches of nframes frames and its shape (any out-pointer may be NULL;
+ * whole frames run in launches of at most 2^24 texels, see ocn_update_frames).
  * rows_band > 0 means that OCN_STAGE_ROWS writes the normal map and Jacobian
  * too, in bands of that many rows (where the render export is asked for, the
  * parallel bands leave all of it to OCN_STAGE_NORMALS, which writes whatever
