@@ -50,11 +50,10 @@ CANON_STAGE = {"k_cols": 40, "k_rows": 36, "k_normals": 20, "k_rows_nrm": 56}
 # Frames per kernel launch of the sequence (ocn_reserve_frames), by N.  The
 # row pass writes its outputs with non-temporal stores, so the intermediates a
 # launch's column pass wrote stay in the 256 MB Infinity Cache for its row
-# pass as long as they fit there beside h0: 16 N=1024 frames (192 MB) ran at
-# 12.4 us per frame over the 600-frame sequence, against 13.8 in 8-frame and
-# 15.0 in 32-frame launches (384 MB, read back from HBM).  The library cuts
-# launches to 2^24 texels (4 frames at N=2048, 1 at N=4096); smaller N run
-# fastest in 32-frame ones.
+# pass as long as they fit there beside the spectrum: 16 N=1024 frames (192 MB)
+# run at 12.0 us per frame over the 600-frame sequence, 8 at 13.4.  The library
+# cuts launches to 2^24 texels (4 frames at N=2048, 1 at N=4096), beyond which
+# the row pass reads them back from HBM; smaller N run fastest in 32-frame ones.
 def launch_frames_for(n):
     return 16 if n == 1024 else 4 if n == 2048 else 1 if n == 4096 else 32
 
@@ -68,9 +67,7 @@ LAUNCH_FRAMES = launch_frames_for(1024)
 # profiles/k_rows_nrm_k_cols_n1024_batched_pmc_traffic.md.  Reported only
 # when the schedule in use matches, otherwise null.
 MEASURED_TRAFFIC = {
-    ("k_rows_nrm", 9, 4, 16): 13.5 + 32.1,
-    ("k_rows_nrm", 9, 3, 8): 15.8 + 32.0,
-    ("k_rows_nrm", 9, 5, 32): 12.9 + 32.0,
+    ("k_rows_nrm", 9, 4, 16): 13.4 + 32.1,
 }
 
 
@@ -621,10 +618,10 @@ def main():
     fps = args.steps / (ms / 1e3)
 
     # Per-kernel durations: HIP events on the launch stream around `reps`
-    # launches of each kernel alone, each launch covering LAUNCH_FRAMES frames
-    # exactly as the timed region launches them.
+    # launches of each kernel alone, each launch covering as many frames as the
+    # timed region's launches, which the library cuts to 2^24 texels.
     stage_ms = {}
-    lf = min(LAUNCH_FRAMES, slots)
+    lf = min(LAUNCH_FRAMES, slots, max(1, 2 ** 24 // nn))
     tl = np.arange(lf, dtype=np.float64) / 60.0
     reps = 40
     sched = oc.schedule(lf)

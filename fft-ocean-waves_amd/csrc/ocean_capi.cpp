@@ -131,7 +131,8 @@ ocn::SpecConst spec_const(const ocn_params& p)
 }
 
 // Schedules the autotuner found, per (device, N, frames-per-launch class,
-// normal mode): the fused row variants only run with nearest-tap normals.
+// normal mode): the row walks run with nearest-tap normals only, bilinear ones
+// take parallel bands in their place.
 std::mutex                                               g_sched_mu;
 std::map<std::tuple<int, int, int, int>, std::pair<int, int>> g_sched;
 
@@ -141,8 +142,9 @@ int frames_class(int nframes)
 }
 
 // Frames of one launch of whole frames, at most.  Its intermediates are kept to
-// 2^24 texels (201 MB), what the 256 MB Infinity Cache holds beside the spectrum,
-// however many frames were reserved: beyond that the row pass reads them from
+// 2^24 texels (201 MB), what the 256 MB Infinity Cache holds beside the spectrum up to
+// N=2048 (34 MB; at N=4096, with 134 MB of spectrum, one frame is over it), however
+// many frames were reserved: beyond that the row pass reads them from
 // HBM (us per frame: N=1024 32 frames 13.8, 16 frames 11.2; N=2048 8 frames 61, 4
 // frames 50; N=4096 4 frames 300, single frames 268; below the line a longer
 // launch is the faster one).
