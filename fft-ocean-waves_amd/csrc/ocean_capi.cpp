@@ -1066,7 +1066,12 @@ int ocn_autotune(ocn_handle* h, int nframes, int reps, void* stream)
     (void)hipEventCreate(&e1);
     float best = 1e30f;
     int   bc = -1, br = -1;
-    for (int cv = 0; cv < ocn::kNumColsVariants && rc == OCN_OK; ++cv)
+    std::vector<std::pair<int, int>> shapes;  // of the column variants timed: several numbers name one kernel
+    for (int cv = 0; cv < ocn::kNumColsVariants && rc == OCN_OK; ++cv) {
+        int E, C;
+        ocn::cols_variant_shape(h->p.N, cv, &E, &C);
+        if (!ocn::schedule_valid(h->p.N, cv, 0) || std::count(shapes.begin(), shapes.end(), std::make_pair(E, C))) continue;
+        shapes.push_back({E, C});
         for (int rv = 0; rv < ocn::kNumRowsVariants && rc == OCN_OK; ++rv) {
             if (!ocn::schedule_valid(h->p.N, cv, rv)) continue;
             // bilinear normals take no walk: the parallel bands stand in for them
@@ -1090,6 +1095,7 @@ int ocn_autotune(ocn_handle* h, int nframes, int reps, void* stream)
                 br   = rv;
             }
         }
+    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     (void)hipFree(outb);

@@ -273,7 +273,7 @@ int ocn_frames_reserved(const ocn_handle* h, int* nframes);
  * columns per workgroup) have several compiled variants per N.  No reference
  * counterpart: the reference has one fixed 32x32 dispatch shape (main.cpp:18).
  *
- * ocn_autotune times every variant available for this N on the handle's
+ * ocn_autotune times every kernel shape available for this N on the handle's
  * device (nframes frames per launch, or as many as a launch of whole frames
  * takes (ocn_update_frames), reps launches each, on `stream`, which
  * it synchronises; it reserves nframes frames as ocn_reserve_frames does) and
