@@ -58,7 +58,6 @@ struct BatchMember {
     float2*       z1;
     float2*       z2;
     const float2* tw8;
-    const float2* tw16;
     float*        height;
     float*        dx;
     float*        dz;

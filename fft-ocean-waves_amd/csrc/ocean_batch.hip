@@ -85,7 +85,7 @@ __device__ __forceinline__ void batch_rows_item(const BatchMember& m, int first_
     // downwards: the upward walk of odd bands (ALT) made the 192-cascade frame
     // 0.7% slower in this kernel, which holds every N in one code object.
     rows_nrm_band<N, E, Sync, RENDER, !RENDER>(m.z1, m.z2, m.height, m.dx, m.dz, m.normals, m.jac,
-                                               E == 8 ? m.tw8 : m.tw16, lds + g * lds_len(N), j, band, R, m.lambda,
+                                               m.tw8, lds + g * lds_len(N), j, band, R, m.lambda,
                                                m.inv2d, m.disp, m.rnorm, m.dscale);
 }
 

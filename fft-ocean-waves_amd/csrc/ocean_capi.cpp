@@ -6,7 +6,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <array>
 #include <cmath>
 #include <cstdarg>
 #include <cstdint>
@@ -228,7 +227,7 @@ struct ocn_handle {
     float4*    uv = nullptr;        // uv_entries(N): the folded spectrum, read by the column pass
     float2*    z1 = nullptr;        // zcap*N*N: intermediate; frame 0 doubles as butterfly scratch
     float2*    z2 = nullptr;        // zcap*N*N/2
-    float2*    tw[3] = {nullptr, nullptr, nullptr};  // Stockham twiddles, radix 4 / 8 / 16
+    float2*    tw[2] = {nullptr, nullptr};  // Stockham twiddles, radix 8 / 16
     float2*    spec[3] = {nullptr, nullptr, nullptr};  // tilde_h0_t textures (lazy)
     uint8_t*   noise = nullptr;     // 4*256*256 (lazy)
     float*     height = nullptr;
@@ -242,7 +241,7 @@ namespace {
 
 void free_all(ocn_handle* h)
 {
-    // uv and the output textures lie behind h0, the other radices' twiddles behind tw[0]
+    // uv and the output textures lie behind h0, the radix-16 twiddles behind tw[0]
     void* ptrs[] = {h->h0, h->z1, h->z2, h->tw[0], h->spec[0], h->spec[1], h->spec[2], h->noise};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
@@ -271,23 +270,23 @@ int dalloc(T** p, size_t count, const char* what)
     return OCN_OK;
 }
 
-// The three radices' tables in one allocation and one copy (tw[0] owns it).
+// Both radices' tables in one allocation and one copy (tw[0] owns it).
 int upload_twiddles(ocn_handle* h)
 {
-    const int          radices[3] = {4, 8, 16};
+    const int          radices[2] = {8, 16};
     std::vector<float> all;
-    size_t             at[3];
-    for (int i = 0; i < 3; ++i) {
+    size_t             at[2];
+    for (int i = 0; i < 2; ++i) {
         at[i] = all.size() / 2;
         const std::vector<float> t = stockham_twiddles(h->p.N, radices[i]);
         all.insert(all.end(), t.begin(), t.end());
         all.resize((all.size() + 31) & ~size_t(31));  // 128-byte starts
     }
     if (h->tw[0]) (void)hipFree(h->tw[0]);
-    h->tw[0] = h->tw[1] = h->tw[2] = nullptr;
+    h->tw[0] = h->tw[1] = nullptr;
     int rc = dalloc(&h->tw[0], all.size() / 2, "twiddles");
     if (rc) return rc;
-    for (int i = 1; i < 3; ++i) h->tw[i] = h->tw[0] + at[i];
+    h->tw[1] = h->tw[0] + at[1];
     hipError_t e = hipMemcpy(h->tw[0], all.data(), all.size() * sizeof(float), hipMemcpyHostToDevice);
     return e == hipSuccess ? OCN_OK : hip_fail(e, "hipMemcpy(twiddles)");
 }
@@ -352,7 +351,7 @@ void frame_args(const ocn_handle* h, float2* z1, float2* z2, const double* t, in
     a->uv = h->uv;
     a->z1 = z1;
     a->z2 = z2;
-    for (int i = 0; i < 3; ++i) a->tw[i] = h->tw[i];
+    for (int i = 0; i < 2; ++i) a->tw[i] = h->tw[i];
     a->sc = spec_const(h->p);
     for (int f = 0; f < nframes; ++f) a->fb.t_rev[f] = t[f] / (2.0 * kPi);
     a->fb.z1_stride  = nn;
@@ -494,7 +493,7 @@ struct ocn_batch {
     char*                                  pool      = nullptr;  // every member's buffers
     char*                                  render_pool = nullptr;    // render exports (on request)
     bool                                   render      = false;
-    std::map<int, std::array<float2*, 2>>  tw;  // per N: radix-8 and radix-16 Stockham twiddles
+    std::map<int, float2*>                 tw;  // per N: radix-8 Stockham twiddles
     bool                                   h0_ready  = false;
     mutable std::vector<char>              h0_out;  // members whose h0 a caller has the address of
     hipGraph_t                             graph     = nullptr;
@@ -514,8 +513,7 @@ void batch_free(ocn_batch* b)
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     for (auto& kv : b->tw)
-        for (float2* q : kv.second)
-            if (q) (void)hipFree(q);
+        if (kv.second) (void)hipFree(kv.second);
 }
 
 int upload_table(float2** dst, const std::vector<float>& t)
@@ -671,7 +669,7 @@ struct ocn_fit {
     int2*                                 d_cols    = nullptr;
     int                                   n_cols    = 0;
     char*                                 pool      = nullptr;
-    std::map<int, std::array<float2*, 2>> tw;  // per N: radix-8 and radix-16 Stockham twiddles
+    std::map<int, float2*>                tw;  // per N: radix-8 Stockham twiddles
     // Members whose targets may have changed since their spectra T^ were
     // made: set by ocn_fit_targets (which hands out the writable buffer) and
     // ocn_fit_upload_targets, cleared when the next fit call remakes T^.
@@ -687,8 +685,7 @@ void fit_free(ocn_fit* f)
         if (q) (void)hipFree(q);
     if (f->reports) (void)hipHostFree(f->reports);
     for (auto& kv : f->tw)
-        for (float2* q : kv.second)
-            if (q) (void)hipFree(q);
+        if (kv.second) (void)hipFree(kv.second);
 }
 
 int check_fit(const ocn_fit* f, int member)
@@ -1289,9 +1286,7 @@ int ocn_batch_create(const ocn_params* params, int count, ocn_batch** out)
     if (!rc) rc = dalloc(&b->pool, total, "batch pool");
     for (const ocn_params& p : b->params) {
         if (rc || b->tw.count(p.N)) continue;
-        std::array<float2*, 2>& t = b->tw[p.N];
-        t = {nullptr, nullptr};
-        if (!(rc = upload_table(&t[0], stockham_twiddles(p.N, 8)))) rc = upload_table(&t[1], stockham_twiddles(p.N, 16));
+        rc = upload_table(&b->tw[p.N], stockham_twiddles(p.N, 8));
     }
     if (!rc) {
         char*     q     = b->pool;
@@ -1309,8 +1304,7 @@ int ocn_batch_create(const ocn_params* params, int count, ocn_batch** out)
             m.dz      = reinterpret_cast<float*>(q), q += al(nn * 4);
             m.jac     = reinterpret_cast<float*>(q), q += al(nn * 4);
             m.normals = reinterpret_cast<float4*>(q), q += al(nn * 16);
-            m.tw8     = b->tw[p.N][0];
-            m.tw16    = b->tw[p.N][1];
+            m.tw8     = b->tw[p.N];
             m.sc      = spec_const(p);
             m.lambda  = (float)p.choppiness;
             m.inv2d   = (float)((double)p.N / (2.0 * p.L));
@@ -1745,9 +1739,7 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
     if (!rc && (e = hipMemset(f->pool, 0, total)) != hipSuccess) rc = hip_fail(e, "hipMemset(fit pool)");
     for (const ocn_params& p : f->params) {
         if (rc || f->tw.count(p.N)) continue;
-        std::array<float2*, 2>& t = f->tw[p.N];
-        t = {nullptr, nullptr};
-        if (!(rc = upload_table(&t[0], stockham_twiddles(p.N, 8)))) rc = upload_table(&t[1], stockham_twiddles(p.N, 16));
+        rc = upload_table(&f->tw[p.N], stockham_twiddles(p.N, 8));
     }
     if (!rc) rc = dalloc(&f->d_vars, (size_t)count, "fit variables");
     if (!rc) {
@@ -1774,7 +1766,6 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
             m.inv_knn   = (float)(1.0 / ((double)K * (double)nn));
             m.k2_d      = (2.0 * kPi / p.L) * (2.0 * kPi / p.L);
             m.g2_d      = p.gravity * p.gravity;
-            m.g_d       = p.gravity;
             for (int k = 0; k < K; ++k) m.t_rev[k] = times[k] / (2.0 * kPi);
             m.uniform = uniform_times ? 1 : 0;
             m.dt_rev  = uniform_dt / (2.0 * kPi);
@@ -1786,8 +1777,7 @@ int ocn_fit_create(const ocn_params* params, int count, int K, const double* tim
             m.phase     = phase_table ? reinterpret_cast<const float4*>(q) : nullptr, q += phase_bytes(p.N);
             m.pq        = reinterpret_cast<const float4*>(q), q += al(sizeof(float4) * ocn::fit_phase_entries(p.N));
             m.edge      = reinterpret_cast<const float4*>(q), q += al(2 * sizeof(float4) * ocn::fit_edge_pairs(p.N));
-            m.tw8       = f->tw[p.N][0];
-            m.tw16      = f->tw[p.N][1];
+            m.tw8       = f->tw[p.N];
             m.key0      = (uint32_t)p.seed;
             m.key1      = (uint32_t)(p.seed >> 32);
             m.ocean_id  = p.ocean_id;

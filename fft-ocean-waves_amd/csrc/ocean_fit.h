@@ -94,7 +94,6 @@ struct FitMember {
     float   g;
     float   inv_knn;        // 1 / (K N^2)
     double  k2_d, g2_d;     // (2 pi / L)^2, g^2
-    double  g_d;            // g
     double  t_rev[kFitMaxK];  // t_k / (2 pi)
     double  dt_rev;         // (t_{k+1} - t_k) / (2 pi) when `uniform`
     int     uniform;        // 1: the times are equally spaced (phases by recurrence)
@@ -111,8 +110,7 @@ struct FitMember {
     // e^{i w dt} as (cos, sin, cos, sin), written once at creation (launch_fit_phase); entry
     // (strip * N + ty) * C + c.  Null otherwise.
     const float4* phase;
-    const float2* tw8;      // Stockham twiddles (N, 8) and (N, 16)
-    const float2* tw16;
+    const float2* tw8;      // Stockham twiddles (N, 8)
     const float* targets;   // K * N*N
     // Per target frame k, the sign-shifted 2-D DFT of the targets,
     // T^_k(n) = sum_x T_k(x) e^{-2 pi i n.x / N} over centred wave numbers n,

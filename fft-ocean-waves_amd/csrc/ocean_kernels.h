@@ -43,7 +43,7 @@ struct FrameArgs {
     const float4* uv;         // folded spectrum (uv_entries(N) values)
     float2*       z1;         // nframes x N x N
     float2*       z2;         // nframes x N/2 x N
-    const float2* tw[3];      // Stockham twiddles for radix 4, 8, 16
+    const float2* tw[2];      // Stockham twiddles for radix 8, 16
     SpecConst     sc;
     FrameBatch    fb;
     int           nframes;

@@ -738,7 +738,7 @@ constexpr bool rows_fits()
     }
 }
 
-constexpr int radix_slot(int E) { return E == 16 ? 2 : E == 8 ? 1 : 0; }
+constexpr int radix_slot(int E) { return E == 16 ? 1 : 0; }
 
 template <int N, int V>
 static hipError_t launch_cols_v(const FrameArgs& a, hipStream_t s)
