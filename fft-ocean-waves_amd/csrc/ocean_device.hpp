@@ -459,8 +459,10 @@ __device__ __forceinline__ void cols_lds_strip(const float4* __restrict__ uv, fl
 // real multiples of one another (-i n kinv A): it runs the three transforms one
 // after another in its one LDS buffer and keeps the results in registers until
 // they are staged, so the strip needs a third of the LDS of cols_lds_strip
-// (35 KB at N = 1024 and C = 4: four blocks of four waves per CU instead of one
-// of twelve) and one block's loads, arithmetic and stores overlap another's.
+// (35 KB at N = 1024 and C = 4).  Registers (127 a thread, four waves per SIMD) leave
+// two blocks of eight waves per CU there, instead of one of twelve, and one block's
+// loads, arithmetic and stores overlap the other's; at N = 4096 a block of 16 waves
+// is alone.
 // Dz goes first: its result leaves the registers before the height's and Dx's,
 // which meet in Z1, are made.  Stores go through the buffers so that C lanes
 // write C adjacent columns of a tile (16 bytes each).

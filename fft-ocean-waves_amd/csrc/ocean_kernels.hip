@@ -159,7 +159,8 @@ __device__ __forceinline__ void cols_block(const FrameBatch& fb, int& f, int& st
 // the strips it replaced, us per frame (column pass alone): N=1024, 16 frames per
 // launch 4.56 -> 3.6 (4 columns); N=2048, 4 frames 26.8 -> 17.6; N=4096, 4 frames
 // 179 -> 151; the 192-cascade batch 627 -> 430 us.  It writes 12 B/texel at 3.5 TB/s
-// (N=1024): bound by the chain of each block's phases, four blocks per CU deep.
+// (N=1024): bound by the chain of each block's phases, two blocks of eight waves per
+// CU deep.
 template <int N, int C>
 __global__ __launch_bounds__(C*(N / 8), 4) void k_cols(const float4* __restrict__ uv, float2* __restrict__ z1,
                                                        float2* __restrict__ z2, const float2* __restrict__ tw,

@@ -16,8 +16,8 @@ def _member(N, i):
     return pyocean.make_params(N=N, L=2.0 * N, wind_speed=12.0 + i % 7, wind_dir=(1.0, 0.3 * (i % 5)), seed=3, ocean_id=i)
 
 
-# 510, 515, 513, 597 and 600 strips: 3 each at N = 64, 9 at 128, 33 at 256, 257 at 512, 513 at 1024
-@pytest.mark.parametrize("sizes,even", [((64,) * 170, 1), ((64,) * 80 + (128,) * 2 + (512,), 1), ((1024,), 1),
+# 510, 513, 513, 513, 597 and 600 strips: 3 each at N = 64, 9 at 128, 33 at 256, 129 at 512, 513 at 1024
+@pytest.mark.parametrize("sizes,even", [((64,) * 170, 1), ((64,) * 3 + (128,) * 2 + (256,) * 3 + (512,) * 3, 1), ((1024,), 1),
                                         ((1024,), 0), ((256,) * 18 + (64,), 1), ((64,) * 200, 1)])
 def test_members_of_halved_strips_equal_single_fits(sizes, even):
     K = 3
